@@ -92,7 +92,11 @@ __global__ __launch_bounds__(256) void rope_kv_write_kernel(uint8_t* __restrict_
                                                             const int* __restrict__ dpos, int n_heads, int n_kv,
                                                             int hd, int bits) {
     constexpr int kMaxPairs = kMaxHd / 2 / 64;
-    const int pos = *dpos;
+    // blockIdx.y: slot of a batched pass (consecutive positions)
+    const int pos = *dpos + (int)blockIdx.y;
+    q += (size_t)blockIdx.y * n_heads * hd;
+    k += (size_t)blockIdx.y * n_kv * hd;
+    v += (size_t)blockIdx.y * n_kv * hd;
     const int lane = threadIdx.x & 63;
     int id = blockIdx.x * 4 + (threadIdx.x >> 6);
     if (id >= n_heads + 2 * n_kv) return;
@@ -199,7 +203,7 @@ __global__ __launch_bounds__(256) void attn_partial(float* __restrict__ part, co
                                                     int T, const int* __restrict__ dpos, int n_heads, int n_kv,
                                                     int hd, float scale, int nchunks) {
     constexpr int CT = kChunk;
-    if (dpos) T = *dpos + 1;           // position read on the device (graph replay)
+    if (dpos) T += *dpos;           // position read on the device (graph replay)
     if ((int)blockIdx.y * CT >= T) return;
     __shared__ float qs[GRP * kMaxHd];
     __shared__ float kv[CT * (kMaxHd + 1)];
@@ -326,7 +330,7 @@ __global__ __launch_bounds__(256) void attn_chunk(float* __restrict__ part, cons
     using G = ChunkGeo<BITS, HD>;
     constexpr int CT = G::CT, RB = G::RB;
     static_assert(G::NV >= 1 && CT * RB % (16 * 256) == 0, "V chunk split");
-    if (dpos) T = *dpos + 1;
+    if (dpos) T += *dpos;
     const int kh = blockIdx.x, c = blockIdx.y, t0 = c * CT;
     if (t0 >= T) return;
     const int tn = min(CT, T - t0);
@@ -442,7 +446,7 @@ __global__ __launch_bounds__(256) void attn_merge(float* __restrict__ out, const
     __shared__ float lw[kMaxChunks / 4];
     __shared__ float red[4];
     __shared__ float tot[2];
-    if (dpos) T = *dpos + 1;
+    if (dpos) T += *dpos;
     const int h = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int nch = (T + ct - 1) / ct;
     const float* ph = part + (size_t)h * nstride * (HD + 2);
@@ -486,7 +490,7 @@ __global__ __launch_bounds__(256) void attn_combine(float* __restrict__ out, con
                                                     int T, const int* __restrict__ dpos, int n_heads, int hd,
                                                     int nstride) {
     const int h = blockIdx.x;
-    if (dpos) T = *dpos + 1;
+    if (dpos) T += *dpos;
     const int nchunks = (T + kChunk - 1) / kChunk;
     const float* ph = part + (size_t)h * nstride * (hd + 2);
     __shared__ float w[kMaxChunks];
@@ -634,7 +638,14 @@ __global__ __launch_bounds__(kSplitThreads) void attn_split(float* __restrict__ 
     constexpr int MB = 64;                                // chunks one merge pass loads per thread
     static_assert(TR >= 1 && CT % TR == 0, "P.V split");
     AS_TT(0);
-    if (dpos) T = *dpos + 1;
+    // blockIdx.z: slot of a batched pass (consecutive positions, partials of
+    // their own); never with ROPE
+    if (dpos) T += *dpos;
+    if constexpr (!ROPE) {
+        T += (int)blockIdx.z;
+        q += (size_t)blockIdx.z * n_kv * GRP * HD;
+        part += (size_t)blockIdx.z * n_kv * GRP * nstride * (HD + 2);
+    }
     // ROPE: the chunks cover positions 0 .. T-2 and the last row of blocks
     // (blockIdx.y == gridDim.y - 1) takes position T-1 alone, with its rotary
     // embedding and cache write, as one more partial (slot nmain), so that
@@ -876,7 +887,7 @@ __global__ __launch_bounds__(1024) void attn_merge_wide(float* __restrict__ out,
     __shared__ float osum[NCQ][DS];
     __shared__ float tot;
     const int h = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const float* ph = part + (size_t)h * nstride * (HD + 2);
+    const float* ph = part + ((size_t)blockIdx.z * gridDim.x + h) * nstride * (HD + 2);   // blockIdx.z: slot
     const int cq = tid / DS, d = blockIdx.y * DS + tid % DS;
     // every slot of the head is loaded before the position is known (slots
     // past the last chunk hold stale values that are never used), so the
@@ -891,7 +902,8 @@ __global__ __launch_bounds__(1024) void attn_merge_wide(float* __restrict__ out,
         wmv = ph[(size_t)tid * (HD + 2)];
         wlv = ph[(size_t)tid * (HD + 2) + 1];
     }
-    if (dpos) T = *dpos + 1;
+    if (dpos) T += *dpos;
+    T += (int)blockIdx.z;
     const int nch = rope ? (T - 1 + ct - 1) / ct + 1 : (T + ct - 1) / ct;   // rope: one more partial, position T-1
     if (tid < nch) {
         wm[tid] = wmv;
@@ -922,7 +934,7 @@ __global__ __launch_bounds__(1024) void attn_merge_wide(float* __restrict__ out,
         float r = 0.f;
 #pragma unroll
         for (int k = 0; k < NCQ; k++) r += osum[k][tid];
-        out[(size_t)h * HD + blockIdx.y * DS + tid] = r / tot;
+        out[((size_t)blockIdx.z * gridDim.x + h) * HD + blockIdx.y * DS + tid] = r / tot;
     }
 }
 
@@ -934,10 +946,13 @@ namespace {
 
 // The one-launch split attention + merge where the shape allows it (1 if
 // launched).  rope: the position's rotary embedding and cache write done by
-// the same launch (dpos required).
+// the same launch (dpos required, one slot).  T counts from *dpos when dpos
+// is given; slots > 1: the positions T - 1 .. T + slots - 2 behind it, each
+// with its own partials.
 int launch_split(float* out, float* part, const float* q, const void* kdata, const void* vdata,
                  const float* kscales, const float* vscales, int T, const int* dpos, int max_pos, int n_heads,
-                 int n_kv, int head_dim, int kv_bits, float scale, const SplitRope* rope, hipStream_t st) {
+                 int n_kv, int head_dim, int kv_bits, float scale, const SplitRope* rope, hipStream_t st,
+                 int slots = 1) {
     const int grp = n_heads / n_kv;
     if (!(g_attn_split && (kv_bits == 32 || kv_bits == 8 || kv_bits == 4) && (head_dim == 64 || head_dim == 128) &&
           (grp == 1 || grp == 2 || grp == 4 || grp == 8) && n_kv <= kSplitMaxKv))
@@ -953,10 +968,10 @@ int launch_split(float* out, float* part, const float* q, const void* kdata, con
 #define IBH_AS(B_, G_, H_) do { \
         if (rope) attn_split<B_, G_, H_, true><<<dim3(n_kv, nchunk + 1), kSplitThreads, 0, st>>>( \
                       out, part, q, K, V, kscales, vscales, T, dpos, n_kv, scale, nstride, rp); \
-        else attn_split<B_, G_, H_, false><<<dim3(n_kv, nchunk), kSplitThreads, 0, st>>>( \
+        else attn_split<B_, G_, H_, false><<<dim3(n_kv, nchunk, slots), kSplitThreads, 0, st>>>( \
                  out, part, q, K, V, kscales, vscales, T, dpos, n_kv, scale, nstride, rp); \
         IBH_CHECK_LAUNCH("ibh_attn_decode (split)"); \
-        attn_merge_wide<H_><<<dim3(n_heads, H_ / 32), 1024, 0, st>>>(out, part, T, dpos, ct, nstride, rope ? 1 : 0); } while (0)
+        attn_merge_wide<H_><<<dim3(n_heads, H_ / 32, slots), 1024, 0, st>>>(out, part, T, dpos, ct, nstride, rope ? 1 : 0); } while (0)
 #define IBH_ASG(B_, H_) do { if (grp == 1) IBH_AS(B_, 1, H_); else if (grp == 2) IBH_AS(B_, 2, H_); \
                          else if (grp == 4) IBH_AS(B_, 4, H_); else IBH_AS(B_, 8, H_); } while (0)
 #define IBH_ASH(B_) do { if (head_dim == 64) IBH_ASG(B_, 64); else IBH_ASG(B_, 128); } while (0)
@@ -1064,6 +1079,37 @@ generic:
     return IBH_OK;
 }
 
+// Attention of `slots` consecutive positions *dpos, *dpos + 1, ... whose cache
+// rows are written, q / out [slot][n_heads * head_dim].  Where the split
+// kernels take the shape, one launch pair serves as many slots as ws has
+// partials for (ibh_attn_workspace_bytes each); else slot by slot.
+int ibh_launch_attn_batch(float* out, const float* q, const void* kdata, const void* vdata, const float* kscales,
+                          const float* vscales, const int* dpos, int slots, int max_pos, int n_heads, int n_kv,
+                          int head_dim, int kv_bits, void* ws, size_t ws_bytes, hipStream_t st) {
+    const size_t one = ibh_attn_workspace_bytes(n_heads, head_dim, max_pos + 1);
+    if (!dpos || slots < 1 || slots > max_pos + 1 || !ws || ws_bytes < one) {
+        ibh_set_error("batched attention: invalid arguments (%d slots)", slots);
+        return IBH_ERROR_PARAM;
+    }
+    const size_t per = ws_bytes / one, row = (size_t)n_heads * head_dim;
+    for (int b = 0; b < slots;) {
+        const int nb = per < (size_t)(slots - b) ? (int)per : slots - b;
+        const int f = launch_split(out + b * row, (float*)ws, q + b * row, kdata, vdata, kscales, vscales, 1 + b, dpos,
+                                   max_pos, n_heads, n_kv, head_dim, kv_bits, 1.0f / sqrtf((float)head_dim), nullptr,
+                                   st, nb);
+        if (f < 0) return f;
+        if (f) {
+            b += nb;
+            continue;
+        }
+        const int rc = ibh_launch_attn(out + b * row, q + b * row, kdata, vdata, kscales, vscales, b, dpos, max_pos,
+                                       n_heads, n_kv, head_dim, kv_bits, ws, ws_bytes, st);
+        if (rc) return rc;
+        b++;
+    }
+    return IBH_OK;
+}
+
 // Decode attention at position *dpos with that position's rotary embedding
 // and cache write (the non-exact rule of ibh_launch_rope_kv_write) done by
 // the split attention launch itself.  Returns 1 if launched, 0 if the shape
@@ -1082,22 +1128,23 @@ int ibh_launch_attn_rope(float* out, const float* q, const float* k, const float
 }
 
 // Rotary embedding of q and k at position *dpos plus the cache write of the
-// rotated k and of v, in one launch (head_dim even, <= 256).
+// rotated k and of v, in one launch (head_dim even, <= 256); with slots > 1
+// for the positions *dpos .. *dpos + slots - 1, q / k / v [slot][heads * hd].
 int ibh_launch_rope_kv_write(void* kdata, void* vdata, float* kscales, float* vscales, float* q, const float* k,
                              const float* v, const float* table, const int* dpos, int n_heads, int n_kv,
-                             int head_dim, int kv_bits, bool exact, hipStream_t st) {
-    if (head_dim % 2 || head_dim > kMaxHd || !dpos ||
+                             int head_dim, int kv_bits, bool exact, hipStream_t st, int slots) {
+    if (slots < 1 || head_dim % 2 || head_dim > kMaxHd || !dpos ||
         (kv_bits != 32 && kv_bits != 16 && kv_bits != 8 && kv_bits != 4)) {
         ibh_set_error("rope + kv write: unsupported geometry (head_dim %d, bits %d)", head_dim, kv_bits);
         return IBH_ERROR_PARAM;
     }
-    const int waves = n_heads + 2 * n_kv;
+    const dim3 grid((n_heads + 2 * n_kv + 3) / 4, slots);
     if (exact)
-        rope_kv_write_kernel<true><<<(waves + 3) / 4, 256, 0, st>>>((uint8_t*)kdata, (uint8_t*)vdata, kscales, vscales,
+        rope_kv_write_kernel<true><<<grid, 256, 0, st>>>((uint8_t*)kdata, (uint8_t*)vdata, kscales, vscales,
                                                                      q, k, v, table, dpos, n_heads, n_kv, head_dim,
                                                                      kv_bits);
     else
-        rope_kv_write_kernel<false><<<(waves + 3) / 4, 256, 0, st>>>((uint8_t*)kdata, (uint8_t*)vdata, kscales, vscales,
+        rope_kv_write_kernel<false><<<grid, 256, 0, st>>>((uint8_t*)kdata, (uint8_t*)vdata, kscales, vscales,
                                                                       q, k, v, table, dpos, n_heads, n_kv, head_dim,
                                                                       kv_bits);
     IBH_CHECK_LAUNCH("rope + kv write");

@@ -42,13 +42,13 @@ int ibh_launch_attn(float* out, const float* q, const void* kdata, const void* v
                     int head_dim, int kv_bits, void* ws, size_t ws_bytes, hipStream_t st);
 
 int ibh_launch_rmsnorm_exact(float* out, float* x, const float* delta, const uint16_t* w, float eps, int n,
-                             hipStream_t st);
+                             hipStream_t st, int slots = 1);
 int ibh_launch_matvec_exact(float* y, const void* w, const void* sc, int kind, const float* x, int M, int N, int bits,
                             const uint8_t* mask, hipStream_t st);
 int ibh_launch_silu_mul_exact(float* out, const float* g, const float* u, const uint8_t* mask, int n, hipStream_t st);
 int ibh_launch_rope_kv_write(void* kdata, void* vdata, float* kscales, float* vscales, float* q, const float* k,
                              const float* v, const float* table, const int* dpos, int n_heads, int n_kv,
-                             int head_dim, int kv_bits, bool exact, hipStream_t st);
+                             int head_dim, int kv_bits, bool exact, hipStream_t st, int slots = 1);
 int ibh_launch_silu_quant(float* out, const float* gate, const float* up, const uint8_t* mask, int8_t* q, float* s,
                           int N, bool exact, hipStream_t st);
 int ibh_launch_rows_w4a8_multi(const MatDesc* d, int n, int kind, const int8_t* qx, const float* sa, int N,
@@ -72,8 +72,14 @@ int ibh_launch_attn_exact_rope(float* out, const float* q, const float* k, const
                                void* kdata, void* vdata, float* ks, float* vs, const int* dpos, int max_pos,
                                int n_heads, int n_kv, int hd, int kv_bits, float* att, hipStream_t st);
 size_t ibh_exact_matvec_lds(int N, bool norm);
-int ibh_launch_int8_batch_exact(float* y, const void* w, const void* sc, int kind, const float* x, int M, int N,
-                                int B, int M_stride, hipStream_t st);
+int ibh_launch_int8_batch_exact(const MatDesc* d, int n, int kind, const float* x, int N, int B, bool avx,
+                                hipStream_t st, int M_stride = 0);
+int ibh_launch_attn_exact_batch(float* out, const float* q, const void* kdata, const void* vdata, const float* ks,
+                                const float* vs, const int* dpos, int slots, int max_pos, int n_heads, int n_kv,
+                                int hd, int kv_bits, float* att, size_t att_bytes, hipStream_t st);
+int ibh_launch_attn_batch(float* out, const float* q, const void* kdata, const void* vdata, const float* kscales,
+                          const float* vscales, const int* dpos, int slots, int max_pos, int n_heads, int n_kv,
+                          int head_dim, int kv_bits, void* ws, size_t ws_bytes, hipStream_t st);
 int ibh_launch_attn_exact(float* out, const float* q, const void* kdata, const void* vdata, const float* ks,
                           const float* vs, const int* dpos, int max_pos, int n_heads, int n_kv, int hd, int kv_bits,
                           float* att, hipStream_t st);
@@ -121,10 +127,12 @@ struct DLayer {
 constexpr int kNormThreads = 1024;
 constexpr int kNormMaxPer = 16;   // hidden <= 16384
 
-// embedding_lookup (forward.c:90-135) of tokens[*pos].
+// embedding_lookup (forward.c:90-135) of tokens[*pos]; blockIdx.y: slot of a
+// batched pass (tokens[*pos + slot] into x[slot]).
 __global__ void embed_kernel(float* __restrict__ x, const uint8_t* __restrict__ emb, const uint16_t* __restrict__ sc,
                              int bits, int hidden, const int* __restrict__ tokens, const int* __restrict__ pos) {
-    const int tok = tokens[*pos];
+    const int tok = tokens[*pos + (int)blockIdx.y];
+    x += (size_t)blockIdx.y * hidden;
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= hidden) return;
     if (bits == 8) {
@@ -141,12 +149,15 @@ __global__ void embed_kernel(float* __restrict__ x, const uint8_t* __restrict__ 
 
 // Residual add fused with rmsnorm_fp16 (forward.c:322-327, kernels rmsnorm):
 //   x += delta (when delta != null);  out = x * (1/sqrtf(mean(x^2) + eps)) * w.
-// One block; out may alias x.
+// One block per vector (slot blockIdx.x of a batched pass); out may alias x.
 __global__ __launch_bounds__(kNormThreads) void add_rmsnorm_kernel(float* __restrict__ out, float* x,
                                                                    const float* __restrict__ delta,
                                                                    const uint16_t* __restrict__ w, float eps,
                                                                    int n) {
     __shared__ float red[kNormThreads / 64];
+    out += (size_t)blockIdx.x * n;
+    x += (size_t)blockIdx.x * n;
+    if (delta) delta += (size_t)blockIdx.x * n;
     float v[kNormMaxPer];
     float ss = 0.f;
 #pragma unroll
@@ -242,6 +253,9 @@ __global__ __launch_bounds__(1024) void argmax_advance_kernel(const float* __res
     }
 }
 
+// Moves the device position past a batched pass of n slots.
+__global__ void advance_kernel(int* pos, int n) { *pos += n; }
+
 bool w4a8_enabled() {
     const char* e = getenv("IB_W4A8");   // forward.c:14-21
     return !(e && e[0] == '0');
@@ -273,11 +287,13 @@ struct ibh_model {
     size_t attn_ws_bytes = 0;
     int* dstate = nullptr;   // [0] pos, [1] prompt_end, [2..] tokens[capacity + 1]
     // batched positions (forward_positions), allocated on first use for
-    // kMaxBatch slots: activations [slot][dim], positions [slot]
+    // kMaxBatch slots: activations [slot][dim], the attention's score rows or
+    // partials per slot
     float *bx = nullptr, *bxb = nullptr, *bxb2 = nullptr, *bq = nullptr, *bk = nullptr, *bv = nullptr;
     float *bhb = nullptr, *bhb2 = nullptr, *blogits = nullptr, *bsa = nullptr;
     int8_t* bqx = nullptr;
-    int* bpos = nullptr;
+    void* battn = nullptr;
+    size_t battn_bytes = 0;
     int hpos = 0;
     hipGraphExec_t exec = nullptr;
     hipGraphExec_t bexec[2][33] = {};   // forward_batch graphs per (exact, B)
@@ -655,7 +671,7 @@ int step(ibh_model* m) {
 constexpr int kMaxBatch = 32;   // IB_BATCH_MAX (inferbit_internal.h:287)
 
 int alloc_batch(ibh_model* m) {
-    if (m->bx) return IBH_OK;
+    if (m->battn) return IBH_OK;   // the last one allocated
     const size_t B = kMaxBatch, H = m->hidden, KV = (size_t)m->n_kv * m->head_dim, I = m->inter, V = m->vocab;
     const size_t NM = H > I ? H : I;
     int rc;
@@ -664,87 +680,107 @@ int alloc_batch(ibh_model* m) {
         (rc = dalloc(m, (void**)&m->bk, B * KV * 4)) || (rc = dalloc(m, (void**)&m->bv, B * KV * 4)) ||
         (rc = dalloc(m, (void**)&m->bhb, B * I * 4)) || (rc = dalloc(m, (void**)&m->bhb2, B * I * 4)) ||
         (rc = dalloc(m, (void**)&m->blogits, B * V * 4)) || (rc = dalloc(m, (void**)&m->bqx, B * NM + 64)) ||
-        (rc = dalloc(m, (void**)&m->bsa, B * (NM / 128 + 2) * 4)) || (rc = dalloc(m, (void**)&m->bpos, B * 4)))
+        (rc = dalloc(m, (void**)&m->bsa, B * (NM / 128 + 2) * 4)))
         return rc;
+    // one buffer for both modes' attention: exact mode (up to 8192 positions)
+    // keeps every slot's score rows, fast mode as many slots' partials as
+    // fit 256 MB
+    const size_t ex = m->max_pos + 1 <= 8192 ? B * ibh_attn_exact_scratch(m->n_heads, m->max_pos) : 0;
+    const size_t one = m->attn_ws_bytes, fit = ((size_t)256 << 20) / one;
+    const size_t fast = one * (fit < 1 ? 1 : fit < B ? fit : B);
+    m->battn_bytes = ex > fast ? ex : fast;
+    return dalloc(m, &m->battn, m->battn_bytes);
+}
+
+// int8 activation codes and group scales of B vectors.  Rows of whole groups
+// are one run of groups, so one launch quantizes every slot.
+int quant_batch(ibh_model* m, const float* in, int N, int B) {
+    void* st = (void*)m->st;
+    if (N % 128 == 0) return ibh_quantize_act_g128(in, m->bqx, m->bsa, B * N, st);
+    const int G = (N + 127) / 128;
+    for (int b = 0; b < B; b++)
+        if (const int rc = ibh_quantize_act_g128(in + (size_t)b * N, m->bqx + (size_t)b * N, m->bsa + (size_t)b * G, N, st))
+            return rc;
     return IBH_OK;
 }
 
-// tensor_matmul_batch (forward.c:200-246): INT4 through the per-slot int8
-// activation quantizer + W4A8 batch kernel (unless IB_W4A8=0), INT8 through
-// matmul_int8_batch, everything else one slot at a time.
-int mm_batch(ibh_model* m, const DTensor& t, float* out, const float* in, int M, int N, int B, bool exact) {
+// tensor_matmul_batch (forward.c:200-246) of 1-3 tensors on the same input:
+// INT4 through the per-slot int8 activation quantizer (once for all of them)
+// + W4A8 batch kernel (unless IB_W4A8=0), INT8 through matmul_int8_batch,
+// everything else one slot at a time.  d[i].out is [slot][d[i].M].
+int mm_batch(ibh_model* m, const DTensor* const* t, const MatDesc* d, int n, const float* in, int N, int B,
+             bool exact) {
     void* st = (void*)m->st;
     int rc;
-    if (t.bits == 4 && m->w4a8) {
-        const int G = (N + 127) / 128;
-        for (int b = 0; b < B; b++)
-            if ((rc = ibh_quantize_act_g128(in + (size_t)b * N, m->bqx + (size_t)b * N, m->bsa + (size_t)b * G, N, st)))
-                return rc;
-        return ibh_matmul_w4a8_batch(out, t.w, t.s, t.skind, m->bqx, m->bsa, M, N, B, M, st);
-    }
-    if (t.bits == 8)
-        return exact ? ibh_launch_int8_batch_exact(out, t.w, t.s, t.skind, in, M, N, B, M, m->st)
-                     : ibh_matmul_int8_batch(out, t.w, t.s, t.skind, in, M, N, B, M, st);
-    for (int b = 0; b < B; b++) {
-        float* o = out + (size_t)b * M;
-        const float* x = in + (size_t)b * N;
-        if ((rc = exact ? mm_exact(m, t, o, x, M, N, nullptr, false) : mm(m, t, o, x, M, N))) return rc;
+    bool same = exact;
+    for (int i = 1; i < n; i++) same = same && t[i]->bits == t[0]->bits && t[i]->skind == t[0]->skind;
+    if (same && t[0]->bits == 8) return ibh_launch_int8_batch_exact(d, n, t[0]->skind, in, N, B, false, m->st);
+    bool coded = false;
+    for (int i = 0; i < n; i++) {
+        const int M = d[i].M;
+        float* out = d[i].out;
+        if (t[i]->bits == 4 && m->w4a8) {
+            if (!coded && (rc = quant_batch(m, in, N, B))) return rc;
+            coded = true;
+            rc = ibh_matmul_w4a8_batch(out, t[i]->w, t[i]->s, t[i]->skind, m->bqx, m->bsa, M, N, B, M, st);
+        } else if (t[i]->bits == 8) {
+            rc = exact ? ibh_launch_int8_batch_exact(d + i, 1, t[i]->skind, in, N, B, false, m->st)
+                       : ibh_matmul_int8_batch(out, t[i]->w, t[i]->s, t[i]->skind, in, M, N, B, M, st);
+        } else {
+            rc = IBH_OK;
+            for (int b = 0; b < B && !rc; b++) {
+                float* o = out + (size_t)b * M;
+                const float* x = in + (size_t)b * N;
+                rc = exact ? mm_exact(m, *t[i], o, x, M, N, nullptr, false) : mm(m, *t[i], o, x, M, N);
+            }
+            coded = false;   // the one-slot form may have used the code buffers
+        }
+        if (rc) return rc;
     }
     return IBH_OK;
+}
+
+int mm_batch1(ibh_model* m, const DTensor& t, float* out, const float* in, int M, int N, int B, bool exact) {
+    const DTensor* const tp[1] = {&t};
+    const MatDesc d{out, t.w, t.s, M};
+    return mm_batch(m, tp, &d, 1, in, N, B, exact);
 }
 
 // x[b] += delta[b] (when given); out[b] = rmsnorm_fp16(x[b]) for every slot.
 int norm_batch(ibh_model* m, float* out, float* x, const float* delta, const uint16_t* w, int B, bool exact) {
-    const int H = m->hidden;
-    int rc;
-    for (int b = 0; b < B; b++) {
-        float* o = out + (size_t)b * H;
-        float* xx = x + (size_t)b * H;
-        const float* d = delta ? delta + (size_t)b * H : nullptr;
-        if (exact) {
-            if ((rc = ibh_launch_rmsnorm_exact(o, xx, d, w, m->eps, H, m->st))) return rc;
-        } else {
-            add_rmsnorm_kernel<<<1, kNormThreads, 0, m->st>>>(o, xx, d, w, m->eps, H);
-            IBH_CHECK_LAUNCH("ibh_model: rmsnorm");
-        }
-    }
+    if (exact) return ibh_launch_rmsnorm_exact(out, x, delta, w, m->eps, m->hidden, m->st, B);
+    add_rmsnorm_kernel<<<B, kNormThreads, 0, m->st>>>(out, x, delta, w, m->eps, m->hidden);
+    IBH_CHECK_LAUNCH("ibh_model: rmsnorm");
     return IBH_OK;
 }
 
-// forward_batch over B slots whose tokens sit at dtokens[pos0 + b] and whose
-// positions are pos0 + b (in bpos): per-position embedding, norms, RoPE, KV
-// write and attention; batched projections; logits of every slot.
+// forward_batch over B slots at the positions *dpos + b, their tokens in
+// dtokens: every step of a layer is one launch for all slots (embedding,
+// norms, RoPE + KV write, attention, quantizers and projections); logits of
+// every slot.
 int forward_batch(ibh_model* m, int B) {
     const int H = m->hidden, KV = m->n_kv * m->head_dim, I = m->inter;
     const bool exact = m->exact;
     int rc;
     const uint16_t* esc = (const uint16_t*)(m->emb.skind == IBH_SCALE_F16 ? m->emb.s : nullptr);
-    for (int b = 0; b < B; b++) {
-        embed_kernel<<<(H + 255) / 256, 256, 0, m->st>>>(m->bx + (size_t)b * H, m->emb.w, esc, m->emb.bits, H,
-                                                         m->dtokens(), m->bpos + b);
-        IBH_CHECK_LAUNCH("ibh_model: embedding");
-    }
+    embed_kernel<<<dim3((H + 255) / 256, B), 256, 0, m->st>>>(m->bx, m->emb.w, esc, m->emb.bits, H, m->dtokens(),
+                                                              m->dpos());
+    IBH_CHECK_LAUNCH("ibh_model: embedding");
     for (int l = 0; l < m->n_layers; l++) {
         DLayer& L = m->layers[l];
+        const DTensor* const qkv_t[3] = {&L.q, &L.k, &L.v};
+        const MatDesc qkv_d[3] = {{m->bq, L.q.w, L.q.s, H}, {m->bk, L.k.w, L.k.s, KV}, {m->bv, L.v.w, L.v.s, KV}};
         if ((rc = norm_batch(m, m->bxb, m->bx, l ? m->bxb : nullptr, L.in_norm, B, exact)) ||
-            (rc = mm_batch(m, L.q, m->bq, m->bxb, H, H, B, exact)) ||
-            (rc = mm_batch(m, L.k, m->bk, m->bxb, KV, H, B, exact)) ||
-            (rc = mm_batch(m, L.v, m->bv, m->bxb, KV, H, B, exact)))
+            (rc = mm_batch(m, qkv_t, qkv_d, 3, m->bxb, H, B, exact)) ||
+            (rc = ibh_launch_rope_kv_write(L.kd, L.vd, L.ks, L.vs, m->bq, m->bk, m->bv, m->rope, m->dpos(), m->n_heads,
+                                           m->n_kv, m->head_dim, m->kv_bits, exact, m->st, B)))
             return rc;
-        for (int b = 0; b < B; b++) {
-            float* q = m->bq + (size_t)b * H;
-            float* o = m->bxb2 + (size_t)b * H;
-            if ((rc = ibh_launch_rope_kv_write(L.kd, L.vd, L.ks, L.vs, q, m->bk + (size_t)b * KV, m->bv + (size_t)b * KV,
-                                               m->rope, m->bpos + b, m->n_heads, m->n_kv, m->head_dim, m->kv_bits,
-                                               exact, m->st)))
-                return rc;
-            rc = exact ? ibh_launch_attn_exact(o, q, L.kd, L.vd, L.ks, L.vs, m->bpos + b, m->max_pos, m->n_heads,
-                                               m->n_kv, m->head_dim, m->kv_bits, m->att, m->st)
-                       : ibh_launch_attn(o, q, L.kd, L.vd, L.ks, L.vs, 0, m->bpos + b, m->max_pos, m->n_heads,
-                                         m->n_kv, m->head_dim, m->kv_bits, m->attn_ws, m->attn_ws_bytes, m->st);
-            if (rc) return rc;
-        }
-        if ((rc = mm_batch(m, L.o, m->bxb, m->bxb2, H, H, B, exact)) ||
+        rc = exact ? ibh_launch_attn_exact_batch(m->bxb2, m->bq, L.kd, L.vd, L.ks, L.vs, m->dpos(), B, m->max_pos,
+                                                 m->n_heads, m->n_kv, m->head_dim, m->kv_bits, (float*)m->battn,
+                                                 m->battn_bytes, m->st)
+                   : ibh_launch_attn_batch(m->bxb2, m->bq, L.kd, L.vd, L.ks, L.vs, m->dpos(), B, m->max_pos, m->n_heads,
+                                           m->n_kv, m->head_dim, m->kv_bits, m->battn, m->battn_bytes, m->st);
+        if (rc || (rc = mm_batch1(m, L.o, m->bxb, m->bxb2, H, H, B, exact)) ||
             (rc = norm_batch(m, m->bxb2, m->bx, m->bxb, L.post_norm, B, exact)))
             return rc;
         if (L.mask) {
@@ -768,36 +804,40 @@ int forward_batch(ibh_model* m, int B) {
                     if ((rc = mm(m, L.down, xo, hb, H, I))) return rc;
                 }
             }
-        } else {
-            if ((rc = mm_batch(m, L.gate, m->bhb, m->bxb2, I, H, B, exact)) ||
-                (rc = mm_batch(m, L.up, m->bhb2, m->bxb2, I, H, B, exact)))
-                return rc;
-            if (m->w4a8 && L.down.bits == 4) {
-                // silu_mul + the down projection's activation quantizer, fused
-                // per slot as on the single-position path
-                const int G = (I + 127) / 128;
-                for (int b = 0; b < B; b++) {
-                    float* hb = m->bhb + (size_t)b * I;
-                    if ((rc = ibh_launch_silu_quant(hb, hb, m->bhb2 + (size_t)b * I, nullptr, m->bqx + (size_t)b * I,
-                                                    m->bsa + (size_t)b * G, I, exact, m->st)))
-                        return rc;
-                }
-                if ((rc = ibh_matmul_w4a8_batch(m->bxb, L.down.w, L.down.s, L.down.skind, m->bqx, m->bsa, H, I, B, H,
-                                                (void*)m->st)))
-                    return rc;
-                continue;
-            }
-            if (exact) {
-                if ((rc = ibh_launch_silu_mul_exact(m->bhb, m->bhb, m->bhb2, nullptr, B * I, m->st))) return rc;
-            } else {
-                silu_mul_kernel<<<(B * I + 255) / 256, 256, 0, m->st>>>(m->bhb, m->bhb, m->bhb2, nullptr, B * I);
-                IBH_CHECK_LAUNCH("ibh_model: silu_mul");
-            }
-            if ((rc = mm_batch(m, L.down, m->bxb, m->bhb, H, I, B, exact))) return rc;
+            continue;
         }
+        const DTensor* const gu_t[2] = {&L.gate, &L.up};
+        const MatDesc gu_d[2] = {{m->bhb, L.gate.w, L.gate.s, I}, {m->bhb2, L.up.w, L.up.s, I}};
+        if ((rc = mm_batch(m, gu_t, gu_d, 2, m->bxb2, H, B, exact))) return rc;
+        if (m->w4a8 && L.down.bits == 4) {
+            // silu_mul + the down projection's activation quantizer in one
+            // launch (rows of whole groups: for every slot)
+            const int G = (I + 127) / 128, per = I % 128 ? 1 : B;
+            for (int b = 0; b < B; b += per) {
+                float* hb = m->bhb + (size_t)b * I;
+                if ((rc = ibh_launch_silu_quant(hb, hb, m->bhb2 + (size_t)b * I, nullptr, m->bqx + (size_t)b * I,
+                                                m->bsa + (size_t)b * G, per * I, exact, m->st)))
+                    return rc;
+            }
+            if ((rc = ibh_matmul_w4a8_batch(m->bxb, L.down.w, L.down.s, L.down.skind, m->bqx, m->bsa, H, I, B, H,
+                                            (void*)m->st)))
+                return rc;
+            continue;
+        }
+        if (exact) {
+            if ((rc = ibh_launch_silu_mul_exact(m->bhb, m->bhb, m->bhb2, nullptr, B * I, m->st))) return rc;
+        } else {
+            silu_mul_kernel<<<(B * I + 255) / 256, 256, 0, m->st>>>(m->bhb, m->bhb, m->bhb2, nullptr, B * I);
+            IBH_CHECK_LAUNCH("ibh_model: silu_mul");
+        }
+        if ((rc = mm_batch1(m, L.down, m->bxb, m->bhb, H, I, B, exact))) return rc;
     }
-    if ((rc = norm_batch(m, m->bx, m->bx, m->bxb, m->out_norm, B, exact))) return rc;
-    return mm_batch(m, m->head, m->blogits, m->bx, m->vocab, H, B, exact);
+    if ((rc = norm_batch(m, m->bx, m->bx, m->bxb, m->out_norm, B, exact)) ||
+        (rc = mm_batch1(m, m->head, m->blogits, m->bx, m->vocab, H, B, exact)))
+        return rc;
+    advance_kernel<<<1, 1, 0, m->st>>>(m->dpos(), B);
+    IBH_CHECK_LAUNCH("ibh_model: advance");
+    return IBH_OK;
 }
 
 bool eager_mode() {
@@ -1276,12 +1316,8 @@ extern "C" int ibh_model_forward_positions(ibh_model* m, const int32_t* tokens, 
     }
     int rc;
     if ((rc = check_tokens(m, tokens, n, "ibh_model_forward_positions")) || (rc = alloc_batch(m))) return rc;
-    int pos[kMaxBatch];
-    for (int b = 0; b < n; b++) pos[b] = m->hpos + b;
     IBH_HIP(hipMemcpyAsync(m->dtokens() + m->hpos, tokens, (size_t)n * 4, hipMemcpyHostToDevice, m->st),
             "ibh_model_forward_positions: tokens");
-    IBH_HIP(hipMemcpyAsync(m->bpos, pos, (size_t)n * 4, hipMemcpyHostToDevice, m->st),
-            "ibh_model_forward_positions: positions");
     // one captured graph per (mode, B): the positions and tokens are device
     // state, so the same graph serves every kv_length
     hipGraphExec_t& ge = m->bexec[m->exact ? 1 : 0][n];
@@ -1310,8 +1346,8 @@ extern "C" int ibh_model_forward_positions(ibh_model* m, const int32_t* tokens, 
     IBH_HIP(hipMemcpyAsync(logits, m->blogits, (size_t)n * vocab * 4, hipMemcpyDeviceToHost, m->st),
             "ibh_model_forward_positions: logits");
     IBH_HIP(hipStreamSynchronize(m->st), "ibh_model_forward_positions");
-    m->hpos += n;
-    return set_state(m, m->hpos, m->hpos);
+    m->hpos += n;   // the pass advanced the device position itself
+    return IBH_OK;
 }
 
 extern "C" int ibh_model_generate_greedy(ibh_model* m, const int32_t* in, int n_in, int32_t* out, int max_out) {

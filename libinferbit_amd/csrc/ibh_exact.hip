@@ -23,6 +23,8 @@
 //   silu_mul  (kernels/avx2.c:233-250): g / (1 + expf(-g)) * up.
 //
 // expf is ib_expf (ibh_common.h), bit-identical to the host glibc expf.
+#include <type_traits>
+
 #include "ibh_common.h"
 
 using namespace ibh;
@@ -31,7 +33,8 @@ namespace {
 
 constexpr int kExactNormMax = 12288;     // floats of x staged in LDS
 
-// Residual add + rmsnorm_fp16 in the x86 order.  One block; out may alias x.
+// Residual add + rmsnorm_fp16 in the x86 order.  One block per vector (slot
+// blockIdx.x of a batched pass, rows of n floats); out may alias x.
 // x is staged chain-major (xt[l][k] = x[8k + l]) so each chain thread reads
 // its elements as float4s.
 __global__ __launch_bounds__(256) void rmsnorm_exact(float* out, float* x, const float* __restrict__ delta,
@@ -39,6 +42,9 @@ __global__ __launch_bounds__(256) void rmsnorm_exact(float* out, float* x, const
     __shared__ __align__(16) float xt[kExactNormMax];
     __shared__ float part[8];
     __shared__ float scale_s;
+    out += (size_t)blockIdx.x * n;
+    x += (size_t)blockIdx.x * n;
+    if (delta) delta += (size_t)blockIdx.x * n;
     const int n8 = n >> 3;                                // elements per chain (n % 8 == 0)
     // all loads first (unconditional, clamped), then the stores
     constexpr int NQ = kExactNormMax / 4 / 256;
@@ -635,7 +641,10 @@ __global__ __launch_bounds__(64) void attn_scores_exact(float* __restrict__ att,
     __shared__ float qs[256];
     __shared__ float knew[ROPE ? 256 : 1];
     const int h = blockIdx.x;
-    const int T = *dpos + 1;
+    // blockIdx.z: slot of a batched pass (the slots sit at consecutive positions)
+    const int T = *dpos + 1 + (int)blockIdx.z;
+    q += (size_t)blockIdx.z * n_heads * hd;
+    att += (size_t)blockIdx.z * n_heads * tstride;
     const int t = blockIdx.y * 64 + threadIdx.x;
     if ((int)blockIdx.y * 64 >= T) return;
     const int grp = n_heads / n_kv;
@@ -772,7 +781,10 @@ __global__ __launch_bounds__(64 * GRP) void attn_scores_grp(float* __restrict__ 
     __shared__ __align__(16) float knew[ROPE ? HD : 4];
     const int kh = blockIdx.x;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;   // wave g scores query head kh * GRP + g
-    const int T = *dpos + 1;
+    // blockIdx.z: slot of a batched pass (the slots sit at consecutive positions)
+    const int T = *dpos + 1 + (int)blockIdx.z;
+    q += (size_t)blockIdx.z * n_kv * GRP * HD;
+    att += (size_t)blockIdx.z * n_kv * GRP * tstride;
     // position tiles in reverse launch order: the tile of the current
     // position (the block with the cache write) is dispatched first instead of
     // last, onto a CU not yet shared with two other tiles
@@ -1281,15 +1293,364 @@ __global__ __launch_bounds__(kAoThreads) void attn_out_exact(float* __restrict__
         attn_out_body<BITS, HD, NB, 224>(out, att, vd, vs, T, n_heads, n_kv, tstride, tcap, sm, red, &inv_s, etab);
 }
 
+// ── batched positions ─────────────────────────────────────────────────────────
+// Slots of a batched pass (consecutive positions) share every launch.
+
+// INT8 matrices x `slots` fp32 vectors with the chains of one of the two x86
+// orders, y[slot * ys + row]:
+//   AVX  = false  matmul_int8_batch (kernels/scalar.c:70-84): one chain per
+//                 (row, slot), the product rounded and then added;
+//   AVX  = true   matmul_int8 (kernels/avx2.c:17-68): 16 fused chains per
+//                 (row, slot), folded as matvec_exact folds them.
+// What bounds it is the VALU: a chain step is one add and one multiply (or
+// one fma) per (row, slot, column) plus the int8 conversion, and packed or
+// matrix instructions do not keep the order.  A lane is a row and a wavefront
+// has SP slots of its own, so x is wave-uniform: it comes through the scalar
+// cache as an SGPR operand and costs no vector or LDS read, and one
+// conversion serves SP slots.  The block's 4 wavefronts share a 64-row x
+// 128-column weight tile in LDS (rows padded to 36 dwords: 16 lanes' 16-byte
+// reads cover all 64 banks), double buffered, the next tile's loads in flight
+// during the chains.  Measured at 8 slots, 4096 columns: 32000 rows 677 ->
+// 94 us, q + k + v (6144 rows, one launch where there were three) 288 -> 43 us.
+constexpr int kBcRows = 64, kBcTile = 128, kBcStride = kBcTile + 16;
+
+struct BatchSet {
+    RowSet rs;
+    int ys[3];
+};
+
+// x of one batch of columns of a slot, wave-uniform: 16 (or 8) floats in
+// scalar registers by one load.
+template <int W> struct XVec;
+template <> struct XVec<16> { typedef float t __attribute__((ext_vector_type(16), aligned(4))); };
+template <> struct XVec<8> { typedef float t __attribute__((ext_vector_type(8), aligned(4))); };
+
+template <int KIND, bool AVX, int SP>
+__global__ __launch_bounds__(256) void int8_batch_chains(const BatchSet bs, const float* __restrict__ x, int N,
+                                                         int slots) {
+    // a batch: NV vectors of VW columns per slot, two batches in registers
+    // (64 scalar registers), 290-380 issue cycles of chains each
+    constexpr int VW = SP == 4 ? 8 : 16, NV = SP == 1 ? 2 : 1, BC = VW * NV;
+    typedef typename XVec<VW>::t xv_t;
+    __shared__ __align__(16) uint8_t wt[2][kBcRows * kBcStride];
+    const RowPick P = pick_rows(bs.rs);
+    const int ys = (int)blockIdx.x >= bs.rs.b2 ? bs.ys[2] : ((int)blockIdx.x >= bs.rs.b1 ? bs.ys[1] : bs.ys[0]);
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int row0 = P.bid * kBcRows, row = row0 + lane;
+    const int s0 = ((int)blockIdx.y * 4 + wave) * SP;     // wave-uniform
+    const bool act = s0 < slots;
+    const uint32_t scb = scale_bits<KIND>(P.sc, min(row, P.M - 1));
+    // staging: thread -> rows tid / 8 and tid / 8 + 32, 16 bytes at 16 * (tid % 8)
+    const int sr = tid >> 3, sc16 = 16 * (tid & 7);
+    const uint8_t* w0 = P.W + (size_t)min(row0 + sr, P.M - 1) * N;
+    const uint8_t* w1 = P.W + (size_t)min(row0 + sr + 32, P.M - 1) * N;
+    uint4 g0 = *(const uint4*)(w0 + min(sc16, N - 16)), g1 = *(const uint4*)(w1 + min(sc16, N - 16));
+    constexpr int NA = AVX ? 16 : 1;
+    float acc[SP][NA];
+#pragma unroll
+    for (int s = 0; s < SP; s++)
+#pragma unroll
+        for (int c = 0; c < NA; c++) acc[s][c] = 0.f;
+    const float* xp[SP];
+#pragma unroll
+    for (int s = 0; s < SP; s++) xp[s] = x + (size_t)min(s0 + s, slots - 1) * N;
+    // A batch in registers: x of its columns per slot (scalar) and the row's
+    // weights.  Scalar loads return out of order, so a wait for one waits for
+    // everything on their counter, LDS reads too: the batch in hand is waited
+    // for as a whole (use) before anything of the next one is asked for.
+    struct Batch {
+        xv_t x[SP][NV];
+        uint2 w[NV][VW / 8];
+    };
+    auto xload = [&](Batch& b, int j) {
+#pragma unroll
+        for (int s = 0; s < SP; s++)
+#pragma unroll
+            for (int u = 0; u < NV; u++) b.x[s][u] = *(const xv_t*)(xp[s] + min(j + VW * u, N - VW));
+    };
+    auto wload = [&](Batch& b, const uint8_t* wl) {
+#pragma unroll
+        for (int u = 0; u < NV; u++)
+#pragma unroll
+            for (int h = 0; h < VW / 8; h++) b.w[u][h] = *(const uint2*)(wl + VW * u + 8 * h);
+    };
+    auto use = [&](const Batch& b) {
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int u = 0; u < NV; u++) {
+#pragma unroll
+            for (int s = 0; s < SP; s++) asm volatile("" ::"s"(b.x[s][u]));
+#pragma unroll
+            for (int h = 0; h < VW / 8; h++) asm volatile("" ::"v"(b.w[u][h].x), "v"(b.w[u][h].y));
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    // PH: the batch's place in its 16 columns (VW = 8: xa the first half, xb the second)
+    auto chains = [&](const Batch& b, int n, auto ph) {
+        constexpr int PH = decltype(ph)::value;
+#pragma unroll
+        for (int u = 0; u < NV; u++) {
+            if (u && n <= VW * u) break;                  // wave-uniform
+            auto cvt = [&](int e) {
+                const uint2 q = b.w[u][e >> 3];
+                return (float)(int8_t)(((e & 7) < 4 ? q.x : q.y) >> (8 * (e & 3)));
+            };
+            if constexpr (AVX) {
+#pragma unroll
+                for (int e = 0; e < VW; e++) {
+                    const float wv = cvt(e);
+#pragma unroll
+                    for (int s = 0; s < SP; s++)
+                        acc[s][(VW * PH + e) & 15] = fmaf(wv, b.x[s][u][e], acc[s][(VW * PH + e) & 15]);
+                }
+            } else {
+                // conversion, product and add of a column two steps apart, so
+                // no instruction waits for the one in front of it
+                float wv[VW], p[SP][VW];
+#pragma unroll
+                for (int e = 0; e < VW + 4; e++) {
+                    if (e < VW) wv[e] = cvt(e);
+                    if (e >= 2 && e < VW + 2) {
+#pragma unroll
+                        for (int s = 0; s < SP; s++) p[s][e - 2] = wv[e - 2] * b.x[s][u][e - 2];
+                    }
+                    if (e >= 4) {
+#pragma unroll
+                        for (int s = 0; s < SP; s++) acc[s][0] = acc[s][0] + p[s][e - 4];
+                    }
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+            }
+        }
+    };
+    Batch xa, xb;
+    xload(xa, 0);
+    const int nt = (N + kBcTile - 1) / kBcTile;
+    for (int t = 0; t < nt; t++) {
+        uint8_t* buf = wt[t & 1];
+        *(uint4*)(buf + sr * kBcStride + sc16) = g0;
+        *(uint4*)(buf + (sr + 32) * kBcStride + sc16) = g1;
+        __syncthreads();                                  // tile t whole; nobody reads buffer (t + 1) & 1 any more
+        const int j0 = t * kBcTile;
+        if (t + 1 < nt) {
+            const int c = min(j0 + kBcTile + sc16, N - 16);
+            g0 = *(const uint4*)(w0 + c);
+            g1 = *(const uint4*)(w1 + c);
+        }
+        if (!act) continue;
+        const uint8_t* wl = buf + lane * kBcStride;
+        // a tile is an even number of batches: xa and xb in turn.  Past the
+        // end of a row the chains get no columns (n <= 0); the loads of x
+        // clamp, those of the tile stay inside it (its padding behind the
+        // last batch).
+        const int n = min(kBcTile, N - j0);               // N % 16 == 0
+        wload(xa, wl);
+        for (int c = 0; c < n; c += 2 * BC) {
+            use(xa);
+            xload(xb, j0 + c + BC);
+            wload(xb, wl + c + BC);
+            chains(xa, n - c, std::integral_constant<int, 0>{});
+            use(xb);
+            xload(xa, j0 + c + 2 * BC);
+            wload(xa, wl + min(c + 2 * BC, kBcTile - BC));
+            if (n - c > BC) chains(xb, n - c - BC, std::integral_constant<int, VW == 8>{});
+        }
+    }
+    if (!act || row >= P.M) return;
+    const float scale = scale_from_bits<KIND>(scb);
+#pragma unroll
+    for (int s = 0; s < SP; s++) {
+        if (s0 + s >= slots) break;
+        float r = acc[s][0];
+        if constexpr (AVX) {
+            float f[8];
+#pragma unroll
+            for (int c = 0; c < 8; c++) f[c] = acc[s][c] + acc[s][c + 8];
+            const float q0 = f[0] + f[4], q1 = f[1] + f[5], q2 = f[2] + f[6], q3 = f[3] + f[7];
+            r = (q0 + q1) + (q2 + q3);
+        }
+        P.y[(size_t)(s0 + s) * ys + row] = r * scale;
+    }
+}
+
+// Softmax of the score rows in place, att[slot][head][0 .. T): a_t =
+// expf(s_t - max) * (1 / sum), the sum serial over t (kernels/avx2.c:192-229).
+// Block (head, slot).  In a batched pass the rows are many, so the serial sum
+// (one lane, about 2.8 ns a term) runs once a row here and beside the other
+// rows' sums, instead of once per 16-column output slice as the one-position
+// kernel has it (attn_out_exact).
+__global__ __launch_bounds__(256) void attn_soft_batch(float* __restrict__ att, const int* __restrict__ dpos,
+                                                       int n_heads, int tstride) {
+    extern __shared__ __align__(16) float es[];           // [tstride]
+    __shared__ float red[4];
+    __shared__ float inv_s;
+    __shared__ uint64_t etab[32];
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int T = *dpos + 1 + (int)blockIdx.y, n4 = (T + 3) >> 2;
+    float4* a4 = (float4*)(att + ((size_t)blockIdx.y * n_heads + blockIdx.x) * tstride);
+    float4 v[8];                                          // T <= 8192
+#pragma unroll
+    for (int u = 0; u < 8; u++) v[u] = a4[min(u * 256 + tid, n4 - 1)];
+    if (tid < 32) {
+        uint64_t e = 0;
+#pragma unroll
+        for (int i = 0; i < 32; i++) e = tid == i ? kExp2fTab[i] : e;
+        etab[tid] = e;
+    }
+    float mx = -INFINITY;
+#pragma unroll
+    for (int u = 0; u < 8; u++) {
+        const int t0 = 4 * (u * 256 + tid);
+        if (t0 < T) mx = fmaxf(mx, v[u].x);
+        if (t0 + 1 < T) mx = fmaxf(mx, v[u].y);
+        if (t0 + 2 < T) mx = fmaxf(mx, v[u].z);
+        if (t0 + 3 < T) mx = fmaxf(mx, v[u].w);
+    }
+    mx = wave_max_dpp(mx);
+    if (lane == 0) red[tid >> 6] = mx;
+    __syncthreads();
+    const float m = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
+#pragma unroll
+    for (int u = 0; u < 8; u++) {
+        const int f = u * 256 + tid;
+        if (f < n4) {
+            v[u] = float4{ib_expf_sel(v[u].x - m, etab), ib_expf_sel(v[u].y - m, etab),
+                          ib_expf_sel(v[u].z - m, etab), ib_expf_sel(v[u].w - m, etab)};
+            ((float4*)es)[f] = v[u];
+        }
+    }
+    __syncthreads();
+    if (tid == 0) {
+        // two register buffers of 32 values in turn: one is read while the other is added
+        float sum = 0.f;
+        float4 A[8], B[8];
+        auto ld = [&](float4 (&r)[8], int t0) {
+#pragma unroll
+            for (int u = 0; u < 8; u++) r[u] = *(const float4*)(es + t0 + 4 * u);
+        };
+        auto add = [&](const float4 (&r)[8]) {
+#pragma unroll
+            for (int u = 0; u < 8; u++) {
+                sum = sum + r[u].x; sum = sum + r[u].y; sum = sum + r[u].z; sum = sum + r[u].w;
+            }
+        };
+        const int T2 = T / 64 * 64;
+        if (T2 > 0) ld(A, 0);
+        for (int t = 0; t < T2; t += 64) {
+            ld(B, t + 32);
+            __builtin_amdgcn_sched_barrier(0);
+            add(A);
+            __builtin_amdgcn_sched_barrier(0);
+            ld(A, min(t + 64, T2 - 32));
+            __builtin_amdgcn_sched_barrier(0);
+            add(B);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        for (int t = T2; t < T; t++) sum = sum + es[t];
+        inv_s = 1.0f / sum;
+    }
+    __syncthreads();
+    const float inv = inv_s;
+#pragma unroll
+    for (int u = 0; u < 8; u++) {
+        const int f = u * 256 + tid;
+        if (f < n4) a4[f] = float4{v[u].x * inv, v[u].y * inv, v[u].z * inv, v[u].w * inv};
+    }
+}
+
+// Output sums o[d] = serial over t of a_t * v_t[d] (forward.c:487-502), every
+// slot of a batched pass: lane = dimension d of a 64-column slice, a
+// wavefront one (slot, head) pair of a KV head, a block 4 such pairs sharing
+// the value rows (64 positions a tile, dequantised once into LDS, the next
+// tile's loads in flight).  One multiply and one add per (pair, d, t) plus a
+// share of the dequantisation: the VALU sets the pace, near the add chain's
+// own latency.  Pairs are ordered slot-major, so a block's slots are adjacent.
+template <int BITS, int HD>
+__global__ __launch_bounds__(256) void attn_pv_batch(float* __restrict__ out, const float* __restrict__ att,
+                                                     const uint8_t* __restrict__ vd, const float* __restrict__ vs,
+                                                     const int* __restrict__ dpos, int n_heads, int n_kv, int tstride,
+                                                     int slots) {
+    constexpr int TT = 64, VS = 64 + 4;
+    __shared__ __align__(16) float vt[2][TT * VS];
+    __shared__ __align__(16) float as[2][4][TT];
+    const int kh = blockIdx.x / (HD / 64), d0 = 64 * (blockIdx.x % (HD / 64));
+    const int grp = n_heads / n_kv;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int np = slots * grp;
+    const int p = min((int)blockIdx.y * 4 + wave, np - 1), slot = p / grp, h = kh * grp + p % grp;
+    const int base = *dpos + 1;
+    const int T = base + slot;
+    const int Tm = base + min((int)blockIdx.y * 4 + 3, np - 1) / grp;    // the block's last slot is its longest
+    const float* a = att + ((size_t)slot * n_heads + h) * tstride;
+    const int st = tid >> 2, sd = 16 * (tid & 3);         // staging: position, 16 columns
+    KvRaw<BITS> raw;
+    kv_raw16<BITS>(raw, vd, vs, min(st, Tm - 1), kh, d0 + sd, HD, n_kv);
+    float av = a[min(lane, T - 1)];
+    float o = 0.f;
+    const int nt = (Tm + TT - 1) / TT;
+    for (int k = 0; k < nt; k++) {
+        float* vb = vt[k & 1];
+        float (*ab)[TT] = as[k & 1];
+        float dq[16];
+        kv_deq16<BITS>(dq, raw);
+#pragma unroll
+        for (int u = 0; u < 4; u++)
+            *(float4*)(vb + st * VS + sd + 4 * u) = float4{dq[4 * u], dq[4 * u + 1], dq[4 * u + 2], dq[4 * u + 3]};
+        ab[wave][lane] = av;
+        __syncthreads();                                  // tile k whole; nobody reads buffer (k + 1) & 1 any more
+        if (k + 1 < nt) {
+            kv_raw16<BITS>(raw, vd, vs, min((k + 1) * TT + st, Tm - 1), kh, d0 + sd, HD, n_kv);
+            av = a[min((k + 1) * TT + lane, T - 1)];
+        }
+        const int n = T - k * TT;                         // wave-uniform
+        const float* vl = vb + lane;
+        if (n >= TT) {
+            // 16 positions read ahead of the 16 being added
+            float va[16], vn[16];
+            float4 wa[4], wn[4];
+            auto rd = [&](float (&v)[16], float4 (&w)[4], int t0) {
+#pragma unroll
+                for (int e = 0; e < 16; e++) v[e] = vl[(t0 + e) * VS];
+#pragma unroll
+                for (int e = 0; e < 4; e++) w[e] = *(const float4*)(&ab[wave][t0 + 4 * e]);
+                __builtin_amdgcn_sched_barrier(0);
+            };
+            auto add = [&](const float (&v)[16], const float4 (&w)[4]) {
+#pragma unroll
+                for (int e = 0; e < 4; e++) {
+                    o = o + w[e].x * v[4 * e];
+                    o = o + w[e].y * v[4 * e + 1];
+                    o = o + w[e].z * v[4 * e + 2];
+                    o = o + w[e].w * v[4 * e + 3];
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            };
+            rd(va, wa, 0);
+            rd(vn, wn, 16);
+            add(va, wa);
+            rd(va, wa, 32);
+            add(vn, wn);
+            rd(vn, wn, 48);
+            add(va, wa);
+            add(vn, wn);
+        } else {
+            for (int t = 0; t < n; t++) o = o + ab[wave][t] * vl[t * VS];
+        }
+    }
+    if ((int)blockIdx.y * 4 + wave < np) out[((size_t)slot * n_heads + h) * HD + d0 + lane] = o;
+}
+
 }  // namespace
 
 int ibh_launch_rmsnorm_exact(float* out, float* x, const float* delta, const uint16_t* w, float eps, int n,
-                             hipStream_t st) {
-    if (n <= 0 || n > kExactNormMax || n % 8) {
+                             hipStream_t st, int slots) {
+    if (slots <= 0 || n <= 0 || n > kExactNormMax || n % 8) {
         ibh_set_error("exact rmsnorm: size %d unsupported (multiple of 8, <= %d)", n, kExactNormMax);
         return IBH_ERROR_PARAM;
     }
-    rmsnorm_exact<<<1, 256, 0, st>>>(out, x, delta, w, eps, n);
+    rmsnorm_exact<<<slots, 256, 0, st>>>(out, x, delta, w, eps, n);
     IBH_CHECK_LAUNCH("exact rmsnorm");
     return IBH_OK;
 }
@@ -1356,20 +1717,63 @@ int ibh_launch_matvec_exact_multi(const MatDesc* d, int n, int kind, const float
     return IBH_OK;
 }
 
-// matmul_int8_batch of the x86 kernel table (kernels/scalar.c:70-84):
-// out[b*M_stride + i] = (serial sum_j (float)W[i][j] * x[b][j]) * scale[i].
-int ibh_launch_int8_batch_exact(float* y, const void* w, const void* sc, int kind, const float* x, int M, int N,
-                                int B, int M_stride, hipStream_t st) {
-    if (B <= 0 || B > 65535 || M <= 0 || N <= 0) {
+// 1-3 INT8 matrices x B vectors x[b][N], d[i].out[b * ys + row], ys = d[i].M or
+// (one matrix) M_stride: the order
+// of the x86 table's matmul_int8_batch (kernels/scalar.c:70-84), or with
+// `avx` of its matmul_int8 (each column as the one-position matvec gives it).
+int ibh_launch_int8_batch_exact(const MatDesc* d, int n, int kind, const float* x, int N, int B, bool avx,
+                                hipStream_t st, int M_stride) {
+    if (B <= 0 || B > 65535 || N <= 0 || n < 1 || n > 3 || (M_stride && n > 1)) {
         ibh_set_error("exact int8 batch: bad sizes");
         return IBH_ERROR_PARAM;
     }
-    const dim3 grid((M + 255) / 256, B);
-    if (kind == IBH_SCALE_F16)
-        matvec_serial_exact<8, IBH_SCALE_F16><<<grid, 256, 0, st>>>(y, (const uint8_t*)w, sc, x, nullptr, M, N, M_stride);
-    else
-        matvec_serial_exact<8, IBH_SCALE_F32><<<grid, 256, 0, st>>>(y, (const uint8_t*)w, sc, x, nullptr, M, N, M_stride);
-    IBH_CHECK_LAUNCH("exact int8 batch");
+    bool al = N % 16 == 0 && ((uintptr_t)x & 3) == 0;
+    int rows = 0;
+    for (int i = 0; i < n; i++) {
+        al = al && ((uintptr_t)d[i].w & 15) == 0;
+        rows += (d[i].M + kBcRows - 1) / kBcRows;
+    }
+    if (al) {
+        // slots per wavefront: more share a conversion, fewer spread over more
+        // blocks.  Issue cycles per column per SIMD are rounds of 256 blocks x
+        // (1 conversion + SP steps of 2 instructions, fused 1).
+        int sp = 1, best = 1 << 30;
+        for (int c = 1; c <= 4; c *= 2) {
+            const int blocks = rows * ((B + 4 * c - 1) / (4 * c));
+            const int cost = ((blocks + 255) / 256) * (1 + (avx ? 1 : 2) * c);
+            if (cost < best) { best = cost; sp = c; }
+        }
+        BatchSet bs{make_rowset(d, n, kBcRows), {M_stride ? M_stride : d[0].M, d[n > 1 ? 1 : 0].M, d[n > 2 ? 2 : 0].M}};
+        const dim3 grid(rows, (B + 4 * sp - 1) / (4 * sp));
+#define IBH_BC(K_, A_) do { \
+        if (sp == 1) int8_batch_chains<K_, A_, 1><<<grid, 256, 0, st>>>(bs, x, N, B); \
+        else if (sp == 2) int8_batch_chains<K_, A_, 2><<<grid, 256, 0, st>>>(bs, x, N, B); \
+        else int8_batch_chains<K_, A_, 4><<<grid, 256, 0, st>>>(bs, x, N, B); } while (0)
+#define IBH_BCK(K_) do { if (avx) IBH_BC(K_, true); else IBH_BC(K_, false); } while (0)
+        if (kind == IBH_SCALE_F16) IBH_BCK(IBH_SCALE_F16); else IBH_BCK(IBH_SCALE_F32);
+#undef IBH_BC
+#undef IBH_BCK
+        IBH_CHECK_LAUNCH("exact int8 batch");
+        return IBH_OK;
+    }
+    for (int i = 0; i < n; i++) {
+        const uint8_t* W = (const uint8_t*)d[i].w;
+        const int M = d[i].M, ys = M_stride ? M_stride : M;
+        if (avx) {
+            for (int b = 0; b < B; b++) {
+                const int rc = ibh_launch_matvec_exact(d[i].out + (size_t)b * ys, W, d[i].s, kind, x + (size_t)b * N, M,
+                                                       N, 8, nullptr, st);
+                if (rc) return rc;
+            }
+            continue;
+        }
+        const dim3 grid((M + 255) / 256, B);
+        if (kind == IBH_SCALE_F16)
+            matvec_serial_exact<8, IBH_SCALE_F16><<<grid, 256, 0, st>>>(d[i].out, W, d[i].s, x, nullptr, M, N, ys);
+        else
+            matvec_serial_exact<8, IBH_SCALE_F32><<<grid, 256, 0, st>>>(d[i].out, W, d[i].s, x, nullptr, M, N, ys);
+        IBH_CHECK_LAUNCH("exact int8 batch");
+    }
     return IBH_OK;
 }
 
@@ -1460,6 +1864,48 @@ static int launch_attn_exact(float* out, const float* q, const void* kdata, cons
 #undef IBH_AG
 #undef IBH_AGG
     IBH_CHECK_LAUNCH("exact attention");
+    return IBH_OK;
+}
+
+// Attention of `slots` consecutive positions *dpos, *dpos + 1, ... (q and out
+// [slot][n_heads * hd]; the positions' cache rows are written already), each as
+// ibh_launch_attn_exact gives it.  att holds every slot's score rows
+// (slots x ibh_attn_exact_scratch).
+int ibh_launch_attn_exact_batch(float* out, const float* q, const void* kdata, const void* vdata, const float* ks,
+                                const float* vs, const int* dpos, int slots, int max_pos, int n_heads, int n_kv,
+                                int hd, int kv_bits, float* att, size_t att_bytes, hipStream_t st) {
+    const size_t one = ibh_attn_exact_scratch(n_heads, max_pos);
+    if ((hd != 64 && hd != 128 && hd != 256) || n_heads % n_kv || max_pos + 1 > 8192 || slots < 1 ||
+        att_bytes < one * slots || (kv_bits != 32 && kv_bits != 16 && kv_bits != 8 && kv_bits != 4)) {
+        ibh_set_error("exact attention: unsupported geometry (head_dim %d, %d positions, %d slots)", hd, max_pos + 1,
+                      slots);
+        return IBH_ERROR_PARAM;
+    }
+    const float scale = 1.0f / sqrtf((float)hd);
+    const int tstride = (max_pos + 1 + 3) & ~3;
+    const uint8_t* K = (const uint8_t*)kdata;
+    const uint8_t* V = (const uint8_t*)vdata;
+    const int grp = n_heads / n_kv;
+    const bool grouped = g_scores_grp && (hd == 64 || hd == 128) && (grp == 1 || grp == 2 || grp == 4 || grp == 8);
+    const dim3 g1(n_heads, (max_pos + 1 + 63) / 64, slots), g2(n_kv, (max_pos + 1 + 63) / 64, slots);
+    const dim3 gp(n_kv * (hd / 64), (slots * grp + 3) / 4);
+    const ExRope rz{};
+#define IBH_AG(B_, G_, H_) attn_scores_grp<B_, G_, H_, false><<<g2, 64 * G_, 0, st>>>(att, q, K, ks, dpos, n_kv, scale, tstride, rz)
+#define IBH_AGG(B_, H_) do { if (grp == 1) IBH_AG(B_, 1, H_); else if (grp == 2) IBH_AG(B_, 2, H_); \
+                             else if (grp == 4) IBH_AG(B_, 4, H_); else IBH_AG(B_, 8, H_); } while (0)
+#define IBH_PV(B_, H_) attn_pv_batch<B_, H_><<<gp, 256, 0, st>>>(out, att, V, vs, dpos, n_heads, n_kv, tstride, slots)
+#define IBH_AE(B_) do { \
+        if (grouped) { if (hd == 64) IBH_AGG(B_, 64); else IBH_AGG(B_, 128); } \
+        else attn_scores_exact<B_, false><<<g1, 64, 0, st>>>(att, q, K, ks, dpos, n_heads, n_kv, hd, scale, tstride); \
+        attn_soft_batch<<<dim3(n_heads, slots), 256, (size_t)tstride * 4, st>>>(att, dpos, n_heads, tstride); \
+        if (hd == 64) IBH_PV(B_, 64); else if (hd == 128) IBH_PV(B_, 128); else IBH_PV(B_, 256); \
+    } while (0)
+    if (kv_bits >= 16) IBH_AE(32); else if (kv_bits == 8) IBH_AE(8); else IBH_AE(4);
+#undef IBH_AE
+#undef IBH_PV
+#undef IBH_AG
+#undef IBH_AGG
+    IBH_CHECK_LAUNCH("exact attention (batched)");
     return IBH_OK;
 }
 

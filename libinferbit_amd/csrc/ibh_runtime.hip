@@ -65,8 +65,8 @@ int current_device() {
 int ibh_noalloc_setup(int device);   // ibh_gemv.hip
 int ibh_launch_matvec_exact(float* y, const void* w, const void* sc, int kind, const float* x, int M, int N, int bits,
                             const uint8_t* mask, hipStream_t st);   // ibh_exact.hip
-int ibh_launch_int8_batch_exact(float* y, const void* w, const void* sc, int kind, const float* x, int M, int N,
-                                int B, int M_stride, hipStream_t st);
+int ibh_launch_int8_batch_exact(const ibh::MatDesc* d, int n, int kind, const float* x, int N, int B, bool avx,
+                                hipStream_t st, int M_stride = 0);
 
 extern "C" int ibh_init(int device) {
     std::lock_guard<std::mutex> lk(g_mu);
@@ -308,7 +308,8 @@ void hip_int8_batch(float* out, const void* w, const float* sw, const float* x, 
     float* dx = (float*)S.put(x, 4 * (size_t)B * N, st);
     float* dout = (float*)S.put(out, ob, st);
     // scalar.c:70-84 (the x86 table's batched INT8 entry): serial sums
-    int rc = ibh_launch_int8_batch_exact(dout, dw, dsw, IBH_SCALE_F32, dx, M, N, B, M_stride, st);
+    const ibh::MatDesc d{dout, dw, dsw, M};
+    int rc = ibh_launch_int8_batch_exact(&d, 1, IBH_SCALE_F32, dx, N, B, false, st, M_stride);
     if (rc == IBH_OK && hipMemcpyAsync(out, dout, ob, hipMemcpyDeviceToHost, st) == hipSuccess &&
         hipStreamSynchronize(st) == hipSuccess)
         return;
