@@ -74,6 +74,8 @@ int ibh_launch_attn_exact_rope(float* out, const float* q, const float* k, const
 size_t ibh_exact_matvec_lds(int N, bool norm);
 int ibh_launch_int8_batch_exact(const MatDesc* d, int n, int kind, const float* x, int N, int B, bool avx,
                                 hipStream_t st, int M_stride = 0);
+int ibh_launch_w4a8_mfma(float* out, const void* w, const void* sw, int kind, const int8_t* qx, const float* sa,
+                         int M, int N, int B, int M_stride, bool fused, hipStream_t st);
 int ibh_launch_attn_exact_batch(float* out, const float* q, const void* kdata, const void* vdata, const float* ks,
                                 const float* vs, const int* dpos, int slots, int max_pos, int n_heads, int n_kv,
                                 int hd, int kv_bits, float* att, size_t att_bytes, hipStream_t st);
@@ -543,6 +545,25 @@ int norm_fused_exact(ibh_model* m, const DLayer& L, bool qkv, float*& xc, float*
     return 1;
 }
 
+// The end of a step from the residual stream x (dl: the delta not yet added,
+// or null): final norm, head, greedy pick, position advanced.
+int finish_step(ibh_model* m, float* x, const float* dl) {
+    const int H = m->hidden;
+    int rc;
+    if (m->exact) {
+        if ((rc = ibh_launch_rmsnorm_exact(m->x, x, dl, m->out_norm, m->eps, H, m->st)) ||
+            (rc = mm_exact(m, m->head, m->logits, m->x, m->vocab, H, nullptr, false)))
+            return rc;
+    } else {
+        add_rmsnorm_kernel<<<1, kNormThreads, 0, m->st>>>(m->x, x, dl, m->out_norm, m->eps, H);
+        IBH_CHECK_LAUNCH("ibh_model: final rmsnorm");
+        if ((rc = mm(m, m->head, m->logits, m->x, m->vocab, H))) return rc;
+    }
+    argmax_advance_kernel<<<1, 1024, 0, m->st>>>(m->logits, m->vocab, m->dtokens(), m->dpos(), m->dprompt_end());
+    IBH_CHECK_LAUNCH("ibh_model: argmax");
+    return IBH_OK;
+}
+
 // forward_single_ex(compute_logits=1) + greedy pick, bit-identical to the CPU.
 // The residual adds run inside the launches that produce or consume the
 // delta where the kernels allow (same operands, same single fp32 add).
@@ -597,12 +618,7 @@ int step_exact(ibh_model* m) {
             dl = acc ? nullptr : m->xb;
         }
     }
-    if ((rc = ibh_launch_rmsnorm_exact(m->x, xc, dl, m->out_norm, m->eps, H, m->st)) ||
-        (rc = mm_exact(m, m->head, m->logits, m->x, m->vocab, H, nullptr, false)))
-        return rc;
-    argmax_advance_kernel<<<1, 1024, 0, m->st>>>(m->logits, m->vocab, m->dtokens(), m->dpos(), m->dprompt_end());
-    IBH_CHECK_LAUNCH("ibh_model: argmax");
-    return IBH_OK;
+    return finish_step(m, xc, dl);
 }
 
 // One decode position with the fastest kernels (results within fp32
@@ -658,38 +674,50 @@ int step(ibh_model* m) {
             dl = acc ? nullptr : m->xb;
         }
     }
-    add_rmsnorm_kernel<<<1, kNormThreads, 0, m->st>>>(m->x, xc, dl, m->out_norm, m->eps, H);
-    IBH_CHECK_LAUNCH("ibh_model: final rmsnorm");
-    if ((rc = mm(m, m->head, m->logits, m->x, m->vocab, H))) return rc;
-    argmax_advance_kernel<<<1, 1024, 0, m->st>>>(m->logits, m->vocab, m->dtokens(), m->dpos(), m->dprompt_end());
-    IBH_CHECK_LAUNCH("ibh_model: argmax");
-    return IBH_OK;
+    return finish_step(m, xc, dl);
 }
 
 
 // ── batched positions: ib_forward_positions -> forward_batch (forward.c:682-939) ──
 constexpr int kMaxBatch = 32;   // IB_BATCH_MAX (inferbit_internal.h:287)
+constexpr int kPromptMin = 3;   // fewer prompt positions run as single steps
 
+// The batched passes' buffers, one allocation on first use.
 int alloc_batch(ibh_model* m) {
-    if (m->battn) return IBH_OK;   // the last one allocated
+    if (m->bx) return IBH_OK;
     const size_t B = kMaxBatch, H = m->hidden, KV = (size_t)m->n_kv * m->head_dim, I = m->inter, V = m->vocab;
     const size_t NM = H > I ? H : I;
-    int rc;
-    if ((rc = dalloc(m, (void**)&m->bx, B * H * 4)) || (rc = dalloc(m, (void**)&m->bxb, B * H * 4)) ||
-        (rc = dalloc(m, (void**)&m->bxb2, B * H * 4)) || (rc = dalloc(m, (void**)&m->bq, B * H * 4)) ||
-        (rc = dalloc(m, (void**)&m->bk, B * KV * 4)) || (rc = dalloc(m, (void**)&m->bv, B * KV * 4)) ||
-        (rc = dalloc(m, (void**)&m->bhb, B * I * 4)) || (rc = dalloc(m, (void**)&m->bhb2, B * I * 4)) ||
-        (rc = dalloc(m, (void**)&m->blogits, B * V * 4)) || (rc = dalloc(m, (void**)&m->bqx, B * NM + 64)) ||
-        (rc = dalloc(m, (void**)&m->bsa, B * (NM / 128 + 2) * 4)))
-        return rc;
-    // one buffer for both modes' attention: exact mode (up to 8192 positions)
-    // keeps every slot's score rows, fast mode as many slots' partials as
-    // fit 256 MB
+    // attention: exact mode (up to 8192 positions) keeps every slot's score
+    // rows, fast mode as many slots' partials as fit 256 MB
     const size_t ex = m->max_pos + 1 <= 8192 ? B * ibh_attn_exact_scratch(m->n_heads, m->max_pos) : 0;
     const size_t one = m->attn_ws_bytes, fit = ((size_t)256 << 20) / one;
     const size_t fast = one * (fit < 1 ? 1 : fit < B ? fit : B);
     m->battn_bytes = ex > fast ? ex : fast;
-    return dalloc(m, &m->battn, m->battn_bytes);
+    size_t off = 0;
+    auto take = [&](size_t bytes) {
+        const size_t at = off;
+        off += (bytes + 255) & ~(size_t)255;
+        return at;
+    };
+    const size_t ox = take(B * H * 4), oxb = take(B * H * 4), oxb2 = take(B * H * 4), oq = take(B * H * 4);
+    const size_t ok = take(B * KV * 4), ov = take(B * KV * 4), ohb = take(B * I * 4), ohb2 = take(B * I * 4);
+    const size_t olg = take(B * V * 4), oqx = take(B * NM + 64), osa = take(B * (NM / 128 + 2) * 4);
+    const size_t oat = take(m->battn_bytes);
+    uint8_t* p = nullptr;
+    if (const int rc = dalloc(m, (void**)&p, off)) return rc;
+    m->bxb = (float*)(p + oxb);
+    m->bxb2 = (float*)(p + oxb2);
+    m->bq = (float*)(p + oq);
+    m->bk = (float*)(p + ok);
+    m->bv = (float*)(p + ov);
+    m->bhb = (float*)(p + ohb);
+    m->bhb2 = (float*)(p + ohb2);
+    m->blogits = (float*)(p + olg);
+    m->bqx = (int8_t*)(p + oqx);
+    m->bsa = (float*)(p + osa);
+    m->battn = p + oat;
+    m->bx = (float*)(p + ox);
+    return IBH_OK;
 }
 
 // int8 activation codes and group scales of B vectors.  Rows of whole groups
@@ -704,17 +732,43 @@ int quant_batch(ibh_model* m, const float* in, int N, int B) {
     return IBH_OK;
 }
 
+// What a batched pass computes.  kVerify: forward_batch (the batch kernels of
+// the table), logits of every slot.  kPrompt / kPromptLast: positions of a
+// prompt as forward_single_ex runs them one by one (exact mode: the one-vector
+// kernels' operation order, so the cache and the logits are those of single
+// steps bit for bit); the last pass of a prompt ends as a step does, with the
+// logits of its last slot and the greedy pick.
+enum class Pass { kVerify, kPrompt, kPromptLast };
+
+// The W4A8 product of B coded vectors (m->bqx / bsa) with one tensor.
+int w4a8_batch(ibh_model* m, const DTensor& t, float* out, int M, int N, int B, bool single_order) {
+    void* st = (void*)m->st;
+    if (!single_order) return ibh_matmul_w4a8_batch(out, t.w, t.s, t.skind, m->bqx, m->bsa, M, N, B, M, st);
+    if (ibh_launch_w4a8_mfma(out, t.w, t.s, t.skind, m->bqx, m->bsa, M, N, B, M, true, m->st)) {
+        IBH_CHECK_LAUNCH("ibh_model: w4a8 (prompt)");
+        return IBH_OK;
+    }
+    const int G = (N + 127) / 128;
+    for (int b = 0; b < B; b++)
+        if (const int rc = ibh_matmul_w4a8(out + (size_t)b * M, t.w, t.s, t.skind, m->bqx + (size_t)b * N,
+                                           m->bsa + (size_t)b * G, M, N, st))
+            return rc;
+    return IBH_OK;
+}
+
 // tensor_matmul_batch (forward.c:200-246) of 1-3 tensors on the same input:
 // INT4 through the per-slot int8 activation quantizer (once for all of them)
 // + W4A8 batch kernel (unless IB_W4A8=0), INT8 through matmul_int8_batch,
-// everything else one slot at a time.  d[i].out is [slot][d[i].M].
+// everything else one slot at a time; in a prompt, tensor_matmul's one-vector
+// kernels.  d[i].out is [slot][d[i].M].
 int mm_batch(ibh_model* m, const DTensor* const* t, const MatDesc* d, int n, const float* in, int N, int B,
-             bool exact) {
+             bool exact, Pass pass) {
     void* st = (void*)m->st;
+    const bool single = exact && pass != Pass::kVerify;
     int rc;
     bool same = exact;
     for (int i = 1; i < n; i++) same = same && t[i]->bits == t[0]->bits && t[i]->skind == t[0]->skind;
-    if (same && t[0]->bits == 8) return ibh_launch_int8_batch_exact(d, n, t[0]->skind, in, N, B, false, m->st);
+    if (same && t[0]->bits == 8) return ibh_launch_int8_batch_exact(d, n, t[0]->skind, in, N, B, single, m->st);
     bool coded = false;
     for (int i = 0; i < n; i++) {
         const int M = d[i].M;
@@ -722,9 +776,9 @@ int mm_batch(ibh_model* m, const DTensor* const* t, const MatDesc* d, int n, con
         if (t[i]->bits == 4 && m->w4a8) {
             if (!coded && (rc = quant_batch(m, in, N, B))) return rc;
             coded = true;
-            rc = ibh_matmul_w4a8_batch(out, t[i]->w, t[i]->s, t[i]->skind, m->bqx, m->bsa, M, N, B, M, st);
+            rc = w4a8_batch(m, *t[i], out, M, N, B, single);
         } else if (t[i]->bits == 8) {
-            rc = exact ? ibh_launch_int8_batch_exact(d + i, 1, t[i]->skind, in, N, B, false, m->st)
+            rc = exact ? ibh_launch_int8_batch_exact(d + i, 1, t[i]->skind, in, N, B, single, m->st)
                        : ibh_matmul_int8_batch(out, t[i]->w, t[i]->s, t[i]->skind, in, M, N, B, M, st);
         } else {
             rc = IBH_OK;
@@ -733,17 +787,17 @@ int mm_batch(ibh_model* m, const DTensor* const* t, const MatDesc* d, int n, con
                 const float* x = in + (size_t)b * N;
                 rc = exact ? mm_exact(m, *t[i], o, x, M, N, nullptr, false) : mm(m, *t[i], o, x, M, N);
             }
-            coded = false;   // the one-slot form may have used the code buffers
         }
         if (rc) return rc;
     }
     return IBH_OK;
 }
 
-int mm_batch1(ibh_model* m, const DTensor& t, float* out, const float* in, int M, int N, int B, bool exact) {
+int mm_batch1(ibh_model* m, const DTensor& t, float* out, const float* in, int M, int N, int B, bool exact,
+              Pass pass) {
     const DTensor* const tp[1] = {&t};
     const MatDesc d{out, t.w, t.s, M};
-    return mm_batch(m, tp, &d, 1, in, N, B, exact);
+    return mm_batch(m, tp, &d, 1, in, N, B, exact, pass);
 }
 
 // x[b] += delta[b] (when given); out[b] = rmsnorm_fp16(x[b]) for every slot.
@@ -756,9 +810,8 @@ int norm_batch(ibh_model* m, float* out, float* x, const float* delta, const uin
 
 // forward_batch over B slots at the positions *dpos + b, their tokens in
 // dtokens: every step of a layer is one launch for all slots (embedding,
-// norms, RoPE + KV write, attention, quantizers and projections); logits of
-// every slot.
-int forward_batch(ibh_model* m, int B) {
+// norms, RoPE + KV write, attention, quantizers and projections).
+int forward_batch(ibh_model* m, int B, Pass pass) {
     const int H = m->hidden, KV = m->n_kv * m->head_dim, I = m->inter;
     const bool exact = m->exact;
     int rc;
@@ -771,7 +824,7 @@ int forward_batch(ibh_model* m, int B) {
         const DTensor* const qkv_t[3] = {&L.q, &L.k, &L.v};
         const MatDesc qkv_d[3] = {{m->bq, L.q.w, L.q.s, H}, {m->bk, L.k.w, L.k.s, KV}, {m->bv, L.v.w, L.v.s, KV}};
         if ((rc = norm_batch(m, m->bxb, m->bx, l ? m->bxb : nullptr, L.in_norm, B, exact)) ||
-            (rc = mm_batch(m, qkv_t, qkv_d, 3, m->bxb, H, B, exact)) ||
+            (rc = mm_batch(m, qkv_t, qkv_d, 3, m->bxb, H, B, exact, pass)) ||
             (rc = ibh_launch_rope_kv_write(L.kd, L.vd, L.ks, L.vs, m->bq, m->bk, m->bv, m->rope, m->dpos(), m->n_heads,
                                            m->n_kv, m->head_dim, m->kv_bits, exact, m->st, B)))
             return rc;
@@ -780,7 +833,7 @@ int forward_batch(ibh_model* m, int B) {
                                                  m->battn_bytes, m->st)
                    : ibh_launch_attn_batch(m->bxb2, m->bq, L.kd, L.vd, L.ks, L.vs, m->dpos(), B, m->max_pos, m->n_heads,
                                            m->n_kv, m->head_dim, m->kv_bits, m->battn, m->battn_bytes, m->st);
-        if (rc || (rc = mm_batch1(m, L.o, m->bxb, m->bxb2, H, H, B, exact)) ||
+        if (rc || (rc = mm_batch1(m, L.o, m->bxb, m->bxb2, H, H, B, exact, pass)) ||
             (rc = norm_batch(m, m->bxb2, m->bx, m->bxb, L.post_norm, B, exact)))
             return rc;
         if (L.mask) {
@@ -808,7 +861,7 @@ int forward_batch(ibh_model* m, int B) {
         }
         const DTensor* const gu_t[2] = {&L.gate, &L.up};
         const MatDesc gu_d[2] = {{m->bhb, L.gate.w, L.gate.s, I}, {m->bhb2, L.up.w, L.up.s, I}};
-        if ((rc = mm_batch(m, gu_t, gu_d, 2, m->bxb2, H, B, exact))) return rc;
+        if ((rc = mm_batch(m, gu_t, gu_d, 2, m->bxb2, H, B, exact, pass))) return rc;
         if (m->w4a8 && L.down.bits == 4) {
             // silu_mul + the down projection's activation quantizer in one
             // launch (rows of whole groups: for every slot)
@@ -819,9 +872,7 @@ int forward_batch(ibh_model* m, int B) {
                                                 m->bsa + (size_t)b * G, per * I, exact, m->st)))
                     return rc;
             }
-            if ((rc = ibh_matmul_w4a8_batch(m->bxb, L.down.w, L.down.s, L.down.skind, m->bqx, m->bsa, H, I, B, H,
-                                            (void*)m->st)))
-                return rc;
+            if ((rc = w4a8_batch(m, L.down, m->bxb, H, I, B, exact && pass != Pass::kVerify))) return rc;
             continue;
         }
         if (exact) {
@@ -830,14 +881,19 @@ int forward_batch(ibh_model* m, int B) {
             silu_mul_kernel<<<(B * I + 255) / 256, 256, 0, m->st>>>(m->bhb, m->bhb, m->bhb2, nullptr, B * I);
             IBH_CHECK_LAUNCH("ibh_model: silu_mul");
         }
-        if ((rc = mm_batch1(m, L.down, m->bxb, m->bhb, H, I, B, exact))) return rc;
+        if ((rc = mm_batch1(m, L.down, m->bxb, m->bhb, H, I, B, exact, pass))) return rc;
     }
-    if ((rc = norm_batch(m, m->bx, m->bx, m->bxb, m->out_norm, B, exact)) ||
-        (rc = mm_batch1(m, m->head, m->blogits, m->bx, m->vocab, H, B, exact)))
+    if (pass == Pass::kVerify &&
+        ((rc = norm_batch(m, m->bx, m->bx, m->bxb, m->out_norm, B, exact)) ||
+         (rc = mm_batch1(m, m->head, m->blogits, m->bx, m->vocab, H, B, exact, pass))))
         return rc;
-    advance_kernel<<<1, 1, 0, m->st>>>(m->dpos(), B);
-    IBH_CHECK_LAUNCH("ibh_model: advance");
-    return IBH_OK;
+    const int moved = pass == Pass::kPromptLast ? B - 1 : B;
+    if (moved) {
+        advance_kernel<<<1, 1, 0, m->st>>>(m->dpos(), moved);
+        IBH_CHECK_LAUNCH("ibh_model: advance");
+    }
+    if (pass != Pass::kPromptLast) return IBH_OK;
+    return finish_step(m, m->bx + (size_t)(B - 1) * H, m->bxb + (size_t)(B - 1) * H);
 }
 
 bool eager_mode() {
@@ -881,6 +937,23 @@ int run_steps(ibh_model* m, int n) {
     }
     m->hpos += n;
     return IBH_OK;
+}
+
+// A prompt of n tokens (in dtokens from the current position on) in passes
+// of up to kMaxBatch positions; ends as n single steps would.  A pass reads
+// every weight once for all its positions and its serial fp32 chains run side
+// by side, where n steps read and run them n times: 32 tokens through four
+// TinyLlama-width layers take 0.60 ms, as 32 steps 5.35 ms.
+int run_prompt(ibh_model* m, int n) {
+    int rc, done = 0;
+    if (n >= kPromptMin && (rc = alloc_batch(m))) return rc;
+    while (n - done >= kPromptMin) {
+        const int B = n - done < kMaxBatch ? n - done : kMaxBatch;
+        if ((rc = forward_batch(m, B, done + B == n ? Pass::kPromptLast : Pass::kPrompt))) return rc;
+        done += B;
+        m->hpos += B;
+    }
+    return done < n ? run_steps(m, n - done) : IBH_OK;
 }
 
 int set_state(ibh_model* m, int pos, int prompt_end) {
@@ -1286,7 +1359,7 @@ extern "C" int ibh_model_forward(ibh_model* m, const int32_t* tokens, int n, flo
     }
     int rc;
     if ((rc = check_tokens(m, tokens, n, "ibh_model_forward")) || (rc = put_tokens(m, tokens, n)) ||
-        (rc = run_steps(m, n)))
+        (rc = run_prompt(m, n)))
         return rc;
     IBH_HIP(hipMemcpyAsync(logits, m->logits, (size_t)vocab * 4, hipMemcpyDeviceToHost, m->st),
             "ibh_model_forward: logits");
@@ -1324,7 +1397,7 @@ extern "C" int ibh_model_forward_positions(ibh_model* m, const int32_t* tokens, 
     if (!ge && !eager_mode()) {
         hipGraph_t g = nullptr;
         IBH_HIP(hipStreamBeginCapture(m->st, hipStreamCaptureModeThreadLocal), "ibh_model_forward_positions: capture");
-        rc = forward_batch(m, n);
+        rc = forward_batch(m, n, Pass::kVerify);
         const hipError_t e = hipStreamEndCapture(m->st, &g);
         if (rc) {
             if (g) hipGraphDestroy(g);
@@ -1340,7 +1413,7 @@ extern "C" int ibh_model_forward_positions(ibh_model* m, const int32_t* tokens, 
     }
     if (ge) {
         IBH_HIP(hipGraphLaunch(ge, m->st), "ibh_model_forward_positions: graph launch");
-    } else if ((rc = forward_batch(m, n))) {
+    } else if ((rc = forward_batch(m, n, Pass::kVerify))) {
         return rc;
     }
     IBH_HIP(hipMemcpyAsync(logits, m->blogits, (size_t)n * vocab * 4, hipMemcpyDeviceToHost, m->st),
@@ -1364,7 +1437,7 @@ extern "C" int ibh_model_generate_greedy(ibh_model* m, const int32_t* in, int n_
     const int start = m->hpos;
     int rc;
     if ((rc = check_tokens(m, in, n_in, "ibh_model_generate_greedy")) || (rc = put_tokens(m, in, n_in)) ||
-        (rc = run_steps(m, steps)))
+        (rc = run_prompt(m, n_in)) || (max_out > 1 && (rc = run_steps(m, max_out - 1))))
         return rc;
     IBH_HIP(hipMemcpyAsync(out, m->dtokens() + start + n_in, (size_t)max_out * 4, hipMemcpyDeviceToHost, m->st),
             "ibh_model_generate_greedy: tokens");

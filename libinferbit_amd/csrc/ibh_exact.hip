@@ -23,8 +23,6 @@
 //   silu_mul  (kernels/avx2.c:233-250): g / (1 + expf(-g)) * up.
 //
 // expf is ib_expf (ibh_common.h), bit-identical to the host glibc expf.
-#include <type_traits>
-
 #include "ibh_common.h"
 
 using namespace ibh;
@@ -1296,22 +1294,19 @@ __global__ __launch_bounds__(kAoThreads) void attn_out_exact(float* __restrict__
 // ── batched positions ─────────────────────────────────────────────────────────
 // Slots of a batched pass (consecutive positions) share every launch.
 
-// INT8 matrices x `slots` fp32 vectors with the chains of one of the two x86
-// orders, y[slot * ys + row]:
-//   AVX  = false  matmul_int8_batch (kernels/scalar.c:70-84): one chain per
-//                 (row, slot), the product rounded and then added;
-//   AVX  = true   matmul_int8 (kernels/avx2.c:17-68): 16 fused chains per
-//                 (row, slot), folded as matvec_exact folds them.
-// What bounds it is the VALU: a chain step is one add and one multiply (or
-// one fma) per (row, slot, column) plus the int8 conversion, and packed or
-// matrix instructions do not keep the order.  A lane is a row and a wavefront
-// has SP slots of its own, so x is wave-uniform: it comes through the scalar
-// cache as an SGPR operand and costs no vector or LDS read, and one
-// conversion serves SP slots.  The block's 4 wavefronts share a 64-row x
-// 128-column weight tile in LDS (rows padded to 36 dwords: 16 lanes' 16-byte
-// reads cover all 64 banks), double buffered, the next tile's loads in flight
-// during the chains.  Measured at 8 slots, 4096 columns: 32000 rows 677 ->
-// 94 us, q + k + v (6144 rows, one launch where there were three) 288 -> 43 us.
+// INT8 matrices x `slots` fp32 vectors, y[slot * ys + row], in the order of the
+// x86 table's matmul_int8_batch (kernels/scalar.c:70-84): one chain per
+// (row, slot), the product rounded and then added.  What bounds it is the
+// VALU: a chain step is a multiply and an add per (row, slot, column) plus the
+// int8 conversion, and packed or matrix instructions do not keep the order.
+// A lane is a row and a wavefront has SP slots of its own, so x is
+// wave-uniform: it comes through the scalar cache as an SGPR operand and costs
+// no vector or LDS read, and one conversion serves SP slots.  The block's 4
+// wavefronts share a 64-row x 128-column weight tile in LDS (rows padded to 36
+// dwords: 16 lanes' 16-byte reads cover all 64 banks), double buffered, the
+// next tile's loads in flight during the chains.  Measured at 8 slots, 4096
+// columns: 32000 rows 677 -> 94 us, q + k + v (6144 rows, one launch where
+// there were three) 288 -> 43 us.
 constexpr int kBcRows = 64, kBcTile = 128, kBcStride = kBcTile + 16;
 
 struct BatchSet {
@@ -1325,7 +1320,7 @@ template <int W> struct XVec;
 template <> struct XVec<16> { typedef float t __attribute__((ext_vector_type(16), aligned(4))); };
 template <> struct XVec<8> { typedef float t __attribute__((ext_vector_type(8), aligned(4))); };
 
-template <int KIND, bool AVX, int SP>
+template <int KIND, int SP>
 __global__ __launch_bounds__(256) void int8_batch_chains(const BatchSet bs, const float* __restrict__ x, int N,
                                                          int slots) {
     // a batch: NV vectors of VW columns per slot, two batches in registers
@@ -1346,12 +1341,9 @@ __global__ __launch_bounds__(256) void int8_batch_chains(const BatchSet bs, cons
     const uint8_t* w0 = P.W + (size_t)min(row0 + sr, P.M - 1) * N;
     const uint8_t* w1 = P.W + (size_t)min(row0 + sr + 32, P.M - 1) * N;
     uint4 g0 = *(const uint4*)(w0 + min(sc16, N - 16)), g1 = *(const uint4*)(w1 + min(sc16, N - 16));
-    constexpr int NA = AVX ? 16 : 1;
-    float acc[SP][NA];
+    float acc[SP];
 #pragma unroll
-    for (int s = 0; s < SP; s++)
-#pragma unroll
-        for (int c = 0; c < NA; c++) acc[s][c] = 0.f;
+    for (int s = 0; s < SP; s++) acc[s] = 0.f;
     const float* xp[SP];
 #pragma unroll
     for (int s = 0; s < SP; s++) xp[s] = x + (size_t)min(s0 + s, slots - 1) * N;
@@ -1386,41 +1378,28 @@ __global__ __launch_bounds__(256) void int8_batch_chains(const BatchSet bs, cons
         }
         __builtin_amdgcn_sched_barrier(0);
     };
-    // PH: the batch's place in its 16 columns (VW = 8: xa the first half, xb the second)
-    auto chains = [&](const Batch& b, int n, auto ph) {
-        constexpr int PH = decltype(ph)::value;
+    auto chains = [&](const Batch& b, int n) {
 #pragma unroll
         for (int u = 0; u < NV; u++) {
             if (u && n <= VW * u) break;                  // wave-uniform
-            auto cvt = [&](int e) {
-                const uint2 q = b.w[u][e >> 3];
-                return (float)(int8_t)(((e & 7) < 4 ? q.x : q.y) >> (8 * (e & 3)));
-            };
-            if constexpr (AVX) {
+            // conversion, product and add of a column two steps apart, so no
+            // instruction waits for the one in front of it
+            float wv[VW], p[SP][VW];
 #pragma unroll
-                for (int e = 0; e < VW; e++) {
-                    const float wv = cvt(e);
-#pragma unroll
-                    for (int s = 0; s < SP; s++)
-                        acc[s][(VW * PH + e) & 15] = fmaf(wv, b.x[s][u][e], acc[s][(VW * PH + e) & 15]);
+            for (int e = 0; e < VW + 4; e++) {
+                if (e < VW) {
+                    const uint2 q = b.w[u][e >> 3];
+                    wv[e] = (float)(int8_t)(((e & 7) < 4 ? q.x : q.y) >> (8 * (e & 3)));
                 }
-            } else {
-                // conversion, product and add of a column two steps apart, so
-                // no instruction waits for the one in front of it
-                float wv[VW], p[SP][VW];
+                if (e >= 2 && e < VW + 2) {
 #pragma unroll
-                for (int e = 0; e < VW + 4; e++) {
-                    if (e < VW) wv[e] = cvt(e);
-                    if (e >= 2 && e < VW + 2) {
-#pragma unroll
-                        for (int s = 0; s < SP; s++) p[s][e - 2] = wv[e - 2] * b.x[s][u][e - 2];
-                    }
-                    if (e >= 4) {
-#pragma unroll
-                        for (int s = 0; s < SP; s++) acc[s][0] = acc[s][0] + p[s][e - 4];
-                    }
-                    __builtin_amdgcn_sched_barrier(0);
+                    for (int s = 0; s < SP; s++) p[s][e - 2] = wv[e - 2] * b.x[s][u][e - 2];
                 }
+                if (e >= 4) {
+#pragma unroll
+                    for (int s = 0; s < SP; s++) acc[s] = acc[s] + p[s][e - 4];
+                }
+                __builtin_amdgcn_sched_barrier(0);
             }
         }
     };
@@ -1450,27 +1429,126 @@ __global__ __launch_bounds__(256) void int8_batch_chains(const BatchSet bs, cons
             use(xa);
             xload(xb, j0 + c + BC);
             wload(xb, wl + c + BC);
-            chains(xa, n - c, std::integral_constant<int, 0>{});
+            chains(xa, n - c);
             use(xb);
             xload(xa, j0 + c + 2 * BC);
             wload(xa, wl + min(c + 2 * BC, kBcTile - BC));
-            if (n - c > BC) chains(xb, n - c - BC, std::integral_constant<int, VW == 8>{});
+            if (n - c > BC) chains(xb, n - c - BC);
         }
     }
     if (!act || row >= P.M) return;
     const float scale = scale_from_bits<KIND>(scb);
 #pragma unroll
-    for (int s = 0; s < SP; s++) {
-        if (s0 + s >= slots) break;
-        float r = acc[s][0];
-        if constexpr (AVX) {
-            float f[8];
+    for (int s = 0; s < SP; s++)
+        if (s0 + s < slots) P.y[(size_t)(s0 + s) * ys + row] = acc[s] * scale;
+}
+
+// The same product in the order of the x86 table's matmul_int8
+// (kernels/avx2.c:17-68): 16 fused chains per (row, slot), element j in chain
+// j mod 16, folded as matvec_exact folds them (the projections of a prompt's
+// positions, each as its single step computes it).  A chain step is one fused
+// multiply-add, which v_mfma_f32_4x4x1 performs with fmaf's rounding (checked
+// bit for bit, subnormals and cancellation included): with the weights of 64
+// rows as B (lane = row) and four slots' x of one column as A, broadcast to
+// all 16 of its blocks (cbsz 4, abid = the block that holds the column), one
+// instruction steps 64 rows x 4 slots, at twice the VALU's rate, and x of 16
+// columns x 4 slots is one register.  The 16 chains are split over the block's
+// 4 wavefronts (4 each), so even 40 row blocks fill the chip, and folded
+// through LDS at the end.  Measured at 32 slots, 2048 columns, q + k + v (2560
+// rows): the chains on the VALU 53 us, here 16 us.
+constexpr int kBaStride = 33;                             // dwords per tile row: 64 lanes' reads in 64 banks
+
+template <int KIND, int NS>                               // NS groups of 4 slots per block
+__global__ __launch_bounds__(256) void int8_batch_fused(const BatchSet bs, const float* __restrict__ x, int N,
+                                                        int slots) {
+    constexpr int kTile = kBcRows * kBaStride, kFold = 16 * 4 * NS * 64;
+    __shared__ uint32_t sm[2 * kTile > kFold ? 2 * kTile : kFold];
+    const RowPick P = pick_rows(bs.rs);
+    const int ys = (int)blockIdx.x >= bs.rs.b2 ? bs.ys[2] : ((int)blockIdx.x >= bs.rs.b1 ? bs.ys[1] : bs.ys[0]);
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int row0 = P.bid * kBcRows, row = row0 + lane;
+    const int s0 = (int)blockIdx.y * 4 * NS;
+    const uint32_t scb = scale_bits<KIND>(P.sc, min(row, P.M - 1));
+    // staging: thread -> rows tid / 8 and tid / 8 + 32, 16 bytes at 16 * (tid % 8)
+    const int sr = tid >> 3, sq = tid & 7;
+    const uint8_t* w0 = P.W + (size_t)min(row0 + sr, P.M - 1) * N;
+    const uint8_t* w1 = P.W + (size_t)min(row0 + sr + 32, P.M - 1) * N;
+    uint4 g0 = *(const uint4*)(w0 + min(16 * sq, N - 16)), g1 = *(const uint4*)(w1 + min(16 * sq, N - 16));
+    // x: lane (block 4t + c, slot i) holds x[slot][64 h + 16 t + 4 wave + c] of the tile
+    const float* xp[NS];
 #pragma unroll
-            for (int c = 0; c < 8; c++) f[c] = acc[s][c] + acc[s][c + 8];
-            const float q0 = f[0] + f[4], q1 = f[1] + f[5], q2 = f[2] + f[6], q3 = f[3] + f[7];
-            r = (q0 + q1) + (q2 + q3);
+    for (int g = 0; g < NS; g++) xp[g] = x + (size_t)min(s0 + 4 * g + (lane & 3), slots - 1) * N;
+    const int xo = 16 * (lane >> 4) + 4 * wave + ((lane >> 2) & 3);
+    float xn[NS][2];
+#pragma unroll
+    for (int g = 0; g < NS; g++)
+#pragma unroll
+        for (int h = 0; h < 2; h++) xn[g][h] = xp[g][min(64 * h + xo, N - 1)];
+    typedef float v4f __attribute__((ext_vector_type(4)));
+    v4f acc[NS][4];
+#pragma unroll
+    for (int g = 0; g < NS; g++)
+#pragma unroll
+        for (int c = 0; c < 4; c++) acc[g][c] = v4f{0.f, 0.f, 0.f, 0.f};
+    const int nt = (N + kBcTile - 1) / kBcTile;
+    for (int t = 0; t < nt; t++) {
+        uint32_t* buf = sm + (t & 1) * kTile;
+        {
+            uint32_t* d0 = buf + sr * kBaStride + 4 * sq;
+            uint32_t* d1 = buf + (sr + 32) * kBaStride + 4 * sq;
+            d0[0] = g0.x; d0[1] = g0.y; d0[2] = g0.z; d0[3] = g0.w;
+            d1[0] = g1.x; d1[1] = g1.y; d1[2] = g1.z; d1[3] = g1.w;
         }
-        P.y[(size_t)(s0 + s) * ys + row] = r * scale;
+        __syncthreads();                                  // tile t whole; nobody reads buffer (t + 1) & 1 any more
+        float xc[NS][2];
+#pragma unroll
+        for (int g = 0; g < NS; g++)
+#pragma unroll
+            for (int h = 0; h < 2; h++) xc[g][h] = xn[g][h];
+        const int j0 = t * kBcTile;
+        if (t + 1 < nt) {
+            const int c = min(j0 + kBcTile + 16 * sq, N - 16);
+            g0 = *(const uint4*)(w0 + c);
+            g1 = *(const uint4*)(w1 + c);
+#pragma unroll
+            for (int g = 0; g < NS; g++)
+#pragma unroll
+                for (int h = 0; h < 2; h++) xn[g][h] = xp[g][min(j0 + kBcTile + 64 * h + xo, N - 1)];
+        }
+        const int nb = min(kBcTile, N - j0) >> 4;         // N % 16 == 0
+        uint32_t wd[8];
+#pragma unroll
+        for (int b = 0; b < 8; b++) wd[b] = buf[lane * kBaStride + 4 * b + wave];
+#define IBH_STEP(B_, C_) do { \
+        const float wv = (float)(int8_t)(wd[B_] >> (8 * C_)); \
+        _Pragma("unroll") for (int g = 0; g < NS; g++) \
+            acc[g][C_] = __builtin_amdgcn_mfma_f32_4x4x1f32(xc[g][B_ / 4], wv, acc[g][C_], 4, 4 * (B_ & 3) + C_, 0); } while (0)
+#define IBH_BLK(B_) do { if (B_ < nb) { IBH_STEP(B_, 0); IBH_STEP(B_, 1); IBH_STEP(B_, 2); IBH_STEP(B_, 3); } } while (0)
+        IBH_BLK(0); IBH_BLK(1); IBH_BLK(2); IBH_BLK(3); IBH_BLK(4); IBH_BLK(5); IBH_BLK(6); IBH_BLK(7);
+#undef IBH_BLK
+#undef IBH_STEP
+    }
+    // fold: chains to LDS as [chain][slot][row], then a thread per (slot, row)
+    __syncthreads();
+    float* f = (float*)sm;
+#pragma unroll
+    for (int g = 0; g < NS; g++)
+#pragma unroll
+        for (int c = 0; c < 4; c++)
+#pragma unroll
+            for (int i = 0; i < 4; i++) f[((4 * wave + c) * 4 * NS + 4 * g + i) * 64 + lane] = acc[g][c][i];
+    __syncthreads();
+    const float scale = scale_from_bits<KIND>(scb);
+#pragma unroll
+    for (int k = 0; k < NS; k++) {
+        const int s = NS * wave + k;
+        float v[16], h[8];
+#pragma unroll
+        for (int c = 0; c < 16; c++) v[c] = f[(c * 4 * NS + s) * 64 + lane];
+#pragma unroll
+        for (int c = 0; c < 8; c++) h[c] = v[c] + v[c + 8];
+        const float q0 = h[0] + h[4], q1 = h[1] + h[5], q2 = h[2] + h[6], q3 = h[3] + h[7];
+        if (s0 + s < slots && row < P.M) P.y[(size_t)(s0 + s) * ys + row] = ((q0 + q1) + (q2 + q3)) * scale;
     }
 }
 
@@ -1734,25 +1812,35 @@ int ibh_launch_int8_batch_exact(const MatDesc* d, int n, int kind, const float* 
         rows += (d[i].M + kBcRows - 1) / kBcRows;
     }
     if (al) {
-        // slots per wavefront: more share a conversion, fewer spread over more
-        // blocks.  Issue cycles per column per SIMD are rounds of 256 blocks x
-        // (1 conversion + SP steps of 2 instructions, fused 1).
-        int sp = 1, best = 1 << 30;
-        for (int c = 1; c <= 4; c *= 2) {
-            const int blocks = rows * ((B + 4 * c - 1) / (4 * c));
-            const int cost = ((blocks + 255) / 256) * (1 + (avx ? 1 : 2) * c);
-            if (cost < best) { best = cost; sp = c; }
-        }
         BatchSet bs{make_rowset(d, n, kBcRows), {M_stride ? M_stride : d[0].M, d[n > 1 ? 1 : 0].M, d[n > 2 ? 2 : 0].M}};
-        const dim3 grid(rows, (B + 4 * sp - 1) / (4 * sp));
-#define IBH_BC(K_, A_) do { \
-        if (sp == 1) int8_batch_chains<K_, A_, 1><<<grid, 256, 0, st>>>(bs, x, N, B); \
-        else if (sp == 2) int8_batch_chains<K_, A_, 2><<<grid, 256, 0, st>>>(bs, x, N, B); \
-        else int8_batch_chains<K_, A_, 4><<<grid, 256, 0, st>>>(bs, x, N, B); } while (0)
-#define IBH_BCK(K_) do { if (avx) IBH_BC(K_, true); else IBH_BC(K_, false); } while (0)
-        if (kind == IBH_SCALE_F16) IBH_BCK(IBH_SCALE_F16); else IBH_BCK(IBH_SCALE_F32);
+        if (avx) {
+            // 8 slots per block share the conversions of 4; 4 make twice the
+            // blocks: fewer issue cycles per SIMD in rounds of 256 blocks
+            const int b4 = rows * ((B + 3) / 4), b8 = rows * ((B + 7) / 8);
+            const bool two = B > 4 && ((b8 + 255) / 256) * 3 <= ((b4 + 255) / 256) * 2;
+            const dim3 grid(rows, two ? (B + 7) / 8 : (B + 3) / 4);
+#define IBH_BF(K_) do { if (two) int8_batch_fused<K_, 2><<<grid, 256, 0, st>>>(bs, x, N, B); \
+                        else int8_batch_fused<K_, 1><<<grid, 256, 0, st>>>(bs, x, N, B); } while (0)
+            if (kind == IBH_SCALE_F16) IBH_BF(IBH_SCALE_F16); else IBH_BF(IBH_SCALE_F32);
+#undef IBH_BF
+        } else {
+            // slots per wavefront: more share a conversion, fewer spread over
+            // more blocks.  Issue cycles per column per SIMD are rounds of 256
+            // blocks x (1 conversion + SP products and adds).
+            int sp = 1, best = 1 << 30;
+            for (int c = 1; c <= 4; c *= 2) {
+                const int blocks = rows * ((B + 4 * c - 1) / (4 * c));
+                const int cost = ((blocks + 255) / 256) * (1 + 2 * c);
+                if (cost < best) { best = cost; sp = c; }
+            }
+            const dim3 grid(rows, (B + 4 * sp - 1) / (4 * sp));
+#define IBH_BC(K_) do { \
+        if (sp == 1) int8_batch_chains<K_, 1><<<grid, 256, 0, st>>>(bs, x, N, B); \
+        else if (sp == 2) int8_batch_chains<K_, 2><<<grid, 256, 0, st>>>(bs, x, N, B); \
+        else int8_batch_chains<K_, 4><<<grid, 256, 0, st>>>(bs, x, N, B); } while (0)
+            if (kind == IBH_SCALE_F16) IBH_BC(IBH_SCALE_F16); else IBH_BC(IBH_SCALE_F32);
 #undef IBH_BC
-#undef IBH_BCK
+        }
         IBH_CHECK_LAUNCH("exact int8 batch");
         return IBH_OK;
     }

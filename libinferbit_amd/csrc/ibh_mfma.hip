@@ -481,9 +481,11 @@ int ibh_launch_w4a8_mfma(float* out, const void* w, const void* sw, int kind, co
     // batch columns per pass: as many of B as one launch's LDS holds (a
     // pass reads every weight once)
     // (the fold takes 16 * NC threads)
+    // (the wider forms clamp the loads of both operands, so they need rows of
+    // whole 128-column groups)
     int NC = 4;
-    if (B > 8 && 16 * 16 <= 64 * KW && lds_of(16) <= 160 * 1024) NC = 16;
-    else if (B > 4 && 16 * 8 <= 64 * KW && lds_of(8) <= 160 * 1024) NC = 8;
+    if (N % 128 == 0 && B > 8 && 16 * 16 <= 64 * KW && lds_of(16) <= 160 * 1024) NC = 16;
+    else if (N % 128 == 0 && B > 4 && 16 * 8 <= 64 * KW && lds_of(8) <= 160 * 1024) NC = 8;
     const size_t lds = NC == 4 ? lds_st(NC) : lds_of(NC);
     const int blocks = (M + kRows - 1) / kRows;
     const uint8_t* W = (const uint8_t*)w;

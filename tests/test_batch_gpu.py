@@ -44,3 +44,73 @@ def test_int8_batch_chains_bit_exact(table, oracle_lib, M, N, B, ms):
     for b in range(B):
         np.testing.assert_array_equal(out[b * ms:b * ms + M].view(np.uint32), want[b * ms:b * ms + M].view(np.uint32))
         assert (out[b * ms + M:(b + 1) * ms] == 7.0).all()
+
+
+# rows that end inside a 128-column group, at every columns-per-pass form
+@pytest.mark.parametrize("M,N,B", [(48, 192, 5), (33, 160, 16), (100, 1056, 9), (17, 96, 32), (64, 416, 4), (20, 32, 6)])
+def test_w4a8_batch_ragged_groups_bit_exact(oracle_lib, M, N, B):
+    import torch
+
+    import libinferbit_amd as L
+    L.ops.init(0)
+    print(f"case w4a8 batch ragged M={M} N={N} B={B}", flush=True)
+    r = np.random.default_rng(M + N + B)
+    w = r.integers(0, 256, (M, N // 2), dtype=np.uint8)
+    s = (r.random(M) * 0.01 + 1e-3).astype(np.float16)
+    qx = r.integers(-127, 128, (B, N), dtype=np.int8)
+    sa = (r.random((B, (N + 127) // 128)) * 0.02 + 1e-3).astype(np.float32)
+    out = torch.empty(B * M, device="cuda")
+    L.ops.matmul_w4a8_batch(out, torch.from_numpy(w).cuda(), torch.from_numpy(s.view(np.int16)).cuda(),
+                            torch.from_numpy(qx).cuda(), torch.from_numpy(sa).cuda(), M, N, B, M)
+    want = oracle_lib.matmul_w4a8_batch(w, s.astype(np.float32), qx, sa).reshape(-1)
+    np.testing.assert_array_equal(out.cpu().numpy().view(np.uint32), want.view(np.uint32))
+
+
+PROMPT_MODELS = {
+    "int8kv": dict(kv_bits=8),
+    "fp32kv": dict(kv_bits=32),
+    "int4kv": dict(kv_bits=4, num_kv_heads=4),
+    "mlp_int2": dict(kv_bits=8, bits=dict(gate_proj=2, up_proj=2, down_proj=2)),
+    "all_int8": dict(kv_bits=8, bits=dict(o_proj=8, gate_proj=8, up_proj=8, down_proj=8)),
+    "all_int4": dict(kv_bits=32, bits=dict(q_proj=4, k_proj=4, v_proj=4, token_embedding=4, head=4)),
+    "mixed_qkv": dict(kv_bits=8, bits=dict(q_proj=8, k_proj=4, v_proj=8)),
+    "hd128": dict(kv_bits=8, hidden_size=512, num_heads=4, num_kv_heads=1, head_dim=128),
+    "ragged": dict(kv_bits=8, hidden_size=192, num_heads=3, num_kv_heads=1, intermediate_size=320),
+}
+
+
+@pytest.mark.parametrize("name", list(PROMPT_MODELS))
+def test_prompt_equals_single_steps(tmp_path, name):
+    """A prompt in batched passes leaves the logits, the cache and the greedy
+    stream of single steps, bit for bit (exact mode): prompts of one pass, of
+    several, with a short last one, and behind cached positions."""
+    from libinferbit_amd import ibf
+    from libinferbit_amd.model import Model
+    spec = dict(PROMPT_MODELS[name])
+    bits = spec.pop("bits", None)
+    cfg = dict(ibf.TINYLLAMA, num_layers=2, hidden_size=256, num_heads=4, num_kv_heads=2, head_dim=64,
+               intermediate_size=512, vocab_size=1000, max_context_length=200)
+    cfg.update(spec)
+    path = str(tmp_path / "m.ibf")
+    ibf.write_synthetic(path, cfg, seed=31, bits=bits)
+    toks = np.random.default_rng(7).integers(0, 1000, 130).astype(np.int32)
+    one, many = Model(path), Model(path)
+    at = 0
+    for n in (3, 33, 1, 70, 2, 16):
+        print(f"case prompt {name} {at}+{n}", flush=True)
+        for t in toks[at:at + n]:
+            a = one.forward([t])
+        b = many.forward(toks[at:at + n])
+        np.testing.assert_array_equal(a.view(np.uint32), b.view(np.uint32))
+        at += n
+    assert one.kv_length() == many.kv_length() == at
+    # the caches are the same: so is what follows from them
+    np.testing.assert_array_equal(one.forward_positions(toks[:5]).view(np.uint32),
+                                  many.forward_positions(toks[:5]).view(np.uint32))
+    one.kv_clear()
+    many.kv_clear()
+    for t in toks[:39]:
+        one.forward([t])
+    np.testing.assert_array_equal(one.generate(toks[39:40], 9), many.generate(toks[:40], 9))
+    one.close()
+    many.close()
