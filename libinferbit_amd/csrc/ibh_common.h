@@ -329,6 +329,11 @@ __device__ __forceinline__ RowPick pick_rows(const RowSet& s) {
     if (b >= s.b1) return {s.W[1], s.sc[1], s.y[1], s.M[1], b - s.b1};
     return {s.W[0], s.sc[0], s.y[0], s.M[0], b};
 }
+// The same for batched vectors: row r of matrix i, slot b at y[b * ys[i] + r].
+struct BatchSet {
+    RowSet rs;
+    int ys[3];
+};
 // One group-scaled INT4 matrix of a multi-matrix launch (ibh_rows.hip).
 struct IbhGrpMat {
     const uint8_t* q;

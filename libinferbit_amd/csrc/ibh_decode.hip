@@ -76,6 +76,8 @@ int ibh_launch_int8_batch_exact(const MatDesc* d, int n, int kind, const float* 
                                 hipStream_t st, int M_stride = 0);
 int ibh_launch_w4a8_mfma(float* out, const void* w, const void* sw, int kind, const int8_t* qx, const float* sa,
                          int M, int N, int B, int M_stride, bool fused, hipStream_t st);
+int ibh_launch_w4a8_batch(const MatDesc* d, int n, int kind, const int8_t* qx, const float* sa, int N, int B,
+                          bool fused, hipStream_t st, int M_stride);
 int ibh_launch_attn_exact_batch(float* out, const float* q, const void* kdata, const void* vdata, const float* ks,
                                 const float* vs, const int* dpos, int slots, int max_pos, int n_heads, int n_kv,
                                 int hd, int kv_bits, float* att, size_t att_bytes, hipStream_t st);
@@ -744,6 +746,9 @@ enum class Pass { kVerify, kPrompt, kPromptLast };
 int w4a8_batch(ibh_model* m, const DTensor& t, float* out, int M, int N, int B, bool single_order) {
     void* st = (void*)m->st;
     if (!single_order) return ibh_matmul_w4a8_batch(out, t.w, t.s, t.skind, m->bqx, m->bsa, M, N, B, M, st);
+    const MatDesc d{out, t.w, t.s, M};
+    const int f = ibh_launch_w4a8_batch(&d, 1, t.skind, m->bqx, m->bsa, N, B, true, m->st, 0);
+    if (f) return f < 0 ? f : IBH_OK;
     if (ibh_launch_w4a8_mfma(out, t.w, t.s, t.skind, m->bqx, m->bsa, M, N, B, M, true, m->st)) {
         IBH_CHECK_LAUNCH("ibh_model: w4a8 (prompt)");
         return IBH_OK;
@@ -766,10 +771,16 @@ int mm_batch(ibh_model* m, const DTensor* const* t, const MatDesc* d, int n, con
     void* st = (void*)m->st;
     const bool single = exact && pass != Pass::kVerify;
     int rc;
-    bool same = exact;
+    bool same = true;
     for (int i = 1; i < n; i++) same = same && t[i]->bits == t[0]->bits && t[i]->skind == t[0]->skind;
-    if (same && t[0]->bits == 8) return ibh_launch_int8_batch_exact(d, n, t[0]->skind, in, N, B, single, m->st);
+    if (same && exact && t[0]->bits == 8) return ibh_launch_int8_batch_exact(d, n, t[0]->skind, in, N, B, single, m->st);
     bool coded = false;
+    if (same && n > 1 && t[0]->bits == 4 && m->w4a8) {
+        if ((rc = quant_batch(m, in, N, B))) return rc;
+        coded = true;
+        const int f = ibh_launch_w4a8_batch(d, n, t[0]->skind, m->bqx, m->bsa, N, B, single, m->st, 0);
+        if (f) return f < 0 ? f : IBH_OK;
+    }
     for (int i = 0; i < n; i++) {
         const int M = d[i].M;
         float* out = d[i].out;

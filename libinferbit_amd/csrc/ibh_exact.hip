@@ -1309,11 +1309,6 @@ __global__ __launch_bounds__(kAoThreads) void attn_out_exact(float* __restrict__
 // there were three) 288 -> 43 us.
 constexpr int kBcRows = 64, kBcTile = 128, kBcStride = kBcTile + 16;
 
-struct BatchSet {
-    RowSet rs;
-    int ys[3];
-};
-
 // x of one batch of columns of a slot, wave-uniform: 16 (or 8) floats in
 // scalar registers by one load.
 template <int W> struct XVec;

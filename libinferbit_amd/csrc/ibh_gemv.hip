@@ -393,6 +393,8 @@ int ibh_launch_gemv_mfma(float* out, const void* w, const void* scales, int kind
                          int N, int bits, hipStream_t st);
 int ibh_launch_w4a8_mfma(float* out, const void* w, const void* sw, int kind, const int8_t* qx, const float* sa,
                          int M, int N, int B, int M_stride, bool fused, hipStream_t st);
+int ibh_launch_w4a8_batch(const MatDesc* d, int n, int kind, const int8_t* qx, const float* sa, int N, int B,
+                          bool fused, hipStream_t st, int M_stride);
 
 namespace {
 
@@ -430,6 +432,12 @@ int launch_w4a8(float* out, const void* w, const void* sw, const int8_t* qx, con
                 int N, int B, int M_stride, hipStream_t st) {
     const uint8_t* W = (const uint8_t*)w;
     const bool fast = N % 32 == 0 && aligned16(w) && aligned16(qx);
+    if (B > 1) {
+        const MatDesc d{out, w, sw, M};
+        const int f = ibh_launch_w4a8_batch(&d, 1, KIND, qx, sa, N, B, FUSED, st, M_stride);
+        if (f < 0) return f;
+        if (f) return IBH_OK;
+    }
     if (FUSED && B == 1 && M_stride == M && ibh_launch_rows_w4a8(out, w, sw, KIND, qx, sa, M, N, st)) {
     } else if (ibh_launch_w4a8_mfma(out, w, sw, KIND, qx, sa, M, N, B, M_stride, FUSED, st)) {
     } else if (fast && B == 1) {

@@ -114,3 +114,32 @@ def test_prompt_equals_single_steps(tmp_path, name):
     np.testing.assert_array_equal(one.generate(toks[39:40], 9), many.generate(toks[:40], 9))
     one.close()
     many.close()
+
+
+# both folds (tall matrices hand the sum on, others gather), 1 and 2 column
+# tiles, codes in LDS and (2048 x 5632 at 17 columns and more) from L2; a last
+# row tile and a last group that are not whole
+@pytest.mark.parametrize("M,N,B", [(6001, 2048, 5), (6001, 2048, 32), (8200, 4096, 16), (8200, 4096, 17), (4099, 2080, 9),
+                                   (2048, 2048, 9), (1003, 2048, 16), (1024, 4096, 17), (2048, 5632, 31),
+                                   (500, 6176, 20), (14336, 4096, 8), (5632, 6144, 12), (40, 64, 17)])
+def test_w4a8_batch_columns_bit_exact(oracle_lib, M, N, B):
+    import torch
+
+    import libinferbit_amd as L
+    L.ops.init(0)
+    print(f"case w4a8 columns M={M} N={N} B={B}", flush=True)
+    r = np.random.default_rng(M + N + B)
+    w = r.integers(0, 256, (M, N // 2), dtype=np.uint8)
+    s = (r.random(M) * 0.01 + 1e-3).astype(np.float16)
+    qx = r.integers(-127, 128, (B, N), dtype=np.int8)
+    sa = (r.random((B, (N + 127) // 128)) * 0.02 + 1e-3).astype(np.float32)
+    ms = M + 3
+    out = torch.full(((B - 1) * ms + M,), 7.0, device="cuda")
+    L.ops.matmul_w4a8_batch(out, torch.from_numpy(w).cuda(), torch.from_numpy(s.view(np.int16)).cuda(),
+                            torch.from_numpy(qx).cuda(), torch.from_numpy(sa).cuda(), M, N, B, ms)
+    got = out.cpu().numpy()
+    rows = np.unique(np.concatenate([np.arange(min(M, 40)), np.arange(max(0, M - 40), M), r.integers(0, M, 200)]))
+    want = oracle_lib.matmul_w4a8_batch(np.ascontiguousarray(w[rows]), s[rows].astype(np.float32), qx, sa).reshape(B, -1)
+    for b in range(B):
+        np.testing.assert_array_equal(got[b * ms + rows].view(np.uint32), want[b].view(np.uint32))
+        assert (got[b * ms + M:(b + 1) * ms] == 7.0).all()
