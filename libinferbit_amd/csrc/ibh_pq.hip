@@ -349,7 +349,7 @@ __global__ __launch_bounds__(kThreads) void pq_reduce(PqDev t, const float* __re
 }
 
 
-// ── one-launch PQ matvec (level 1, G <= 16, K <= 256) ──────────────────────
+// ── one-launch PQ matvec (G <= 16, up to 256 codes a level) ────────────────
 // Block = (tile of 512 rows, slab of 32 chunks), 1024 threads: two per row,
 // thread q of a row owns chunks 16q..16q+15 of the slab on both sides.  The
 // two slabs that share the 64-byte index segments of a row run on one XCD,
@@ -362,9 +362,11 @@ __global__ __launch_bounds__(kThreads) void pq_reduce(PqDev t, const float* __re
 //     v_mfma_f32_32x32x16_f16 with A = [cb | cb] (the fp16 codewords, exact)
 //     and B = [x_hi ; x_lo], x scaled per (chunk, side) by a power of two
 //     (exact) and split into two fp16 parts; products are exact and sums
-//     fp32.  x is scaled by one power of two per slab (2^-e, e the exponent
-//     of the slab's max|x|), so an entry carries ~2^-22 of the SLAB's max|x|
-//     (the CPU's fp32 table sum carries ~2^-24 per term).
+//     fp32.  x is scaled by one power of two per slab that takes its max|x|
+//     to the top of fp16: an element's two parts then keep 2^-23 of the
+//     element itself down to 2^-17 of the slab's max (scaled to 1 instead,
+//     small elements lost their low parts: error against 64 bits 3.0e-7 ->
+//     1.5e-7, 3489 rows of 201 chunks).
 //  3. Max|x| over the inner columns (the skipping rule of
 //     pq_decode.c:1569-1616), the slab's chunk maxima, max|codeword|.
 //  4. Gather: 32 LDS lookups per thread, the row's two partials summed.
@@ -384,7 +386,12 @@ __global__ __launch_bounds__(kThreads) void pq_reduce(PqDev t, const float* __re
 //     library workspace (ws == NULL) use a library array of words.
 //     A non-finite x (or a bound that overflows) would make the fixed-point
 //     terms meaningless: every slab then writes NaN to its rows (the CPU
-//     gives +-Inf or NaN there).
+//     gives +-Inf or NaN there); two-level calls, which had the three-kernel
+//     path's fp32 sums there, take them from plain_row.
+//  Two levels double the tables, the lookups and the index bytes and keep the
+//  rest: 4096 x 14336, 256 + 256 codes, streaming: 75.3 us in three launches
+//  (68 of them the gather, 16 chunks' tables re-read by every block of 512
+//  rows and two byte loads per lookup) -> 13.1 us, error 2.1e-7 -> 1.2e-7.
 constexpr int kFThreads = 1024;
 constexpr int kFRows = 512;
 constexpr int kFCS = 32;
@@ -414,10 +421,9 @@ typedef float f16x_t __attribute__((ext_vector_type(16)));
 // slab's x, scaled by 2^-e (e: exponent of max|x|, one per call, so the
 // entries are T * 2^-e and the row sums are rescaled once).  Tiles with
 // kt == 0 also record each (chunk, side)'s max|x|.
-template <bool KA, int CS>
-__device__ __forceinline__ void table_tile(const PqDev& t, const h8_t* cbs, const float* xsl, int it, int KT, int CT,
-                                           int cn, int lane, int TS, float xscale, float* T, float (*cmax_s)[CS]) {
-    const int K = t.K;
+template <bool KA, int CS, bool CMAX>
+__device__ __forceinline__ void table_tile(int K, const h8_t* cbs, const float* xsl, int it, int KT, int CT, int cn,
+                                           int lane, int TS, float xscale, float* T, float (*cmax_s)[CS]) {
     const int sd = it / (KT * CT), rest = it - sd * KT * CT, kt = rest / CT, ct = rest - kt * CT;
     const int k = min(kt * 32 + (lane & 31), K - 1);
     const int cc = ct * 32 + (lane & 31);
@@ -426,7 +432,7 @@ __device__ __forceinline__ void table_tile(const PqDev& t, const h8_t* cbs, cons
     const float4* xp = (const float4*)(xsl + ccl * kXS + sd * 8);
     const float4 x0 = xp[0], x1 = xp[1];
     const float xv[8] = {x0.x, x0.y, x0.z, x0.w, x1.x, x1.y, x1.z, x1.w};
-    if (kt == 0) {
+    if (CMAX && kt == 0) {
         float m = 0.f;
 #pragma unroll
         for (int i = 0; i < 8; i++) m = fmaxf(m, fabsf(xv[i]));
@@ -458,20 +464,55 @@ __device__ __forceinline__ void table_tile(const PqDev& t, const h8_t* cbs, cons
     }
 }
 
-template <bool KA>   // K % 32 == 0: every table row of a tile is stored
+// A row's sum from the codebooks and x directly, no tables (two-level calls
+// with a non-finite x, or sums past the fixed-point range): the entries in the
+// order of the three-kernel path, so +-Inf and NaN come out where they do there.
+__device__ float plain_row(const PqDev& t, const float* __restrict__ x, int r, float gmax) {
+    const int hf = t.G / 2;
+    const size_t l2s = l2_stride(t);
+    float acc = 0.f;
+    for (int c = 0; c < t.C; c++) {
+        float xv[16], cm = 0.f;
+        for (int i = 0; i < t.G; i++) {
+            xv[i] = x[inner_col(t, c * t.G + i)];
+            cm = fmaxf(cm, fabsf(xv[i]));
+        }
+        const bool keep = t.skip_mode == 1 ? (gmax > 0.f ? cm >= gmax * t.skip_val : true)
+                        : t.skip_mode == 2 ? (t.skip_val > 0.f ? cm > t.skip_val : true) : true;
+        if (!keep) continue;
+        const size_t io = (size_t)r * t.C + c;
+        acc = acc + (table_entry(t.cb1l + (size_t)t.i1l[io] * hf, xv, hf) +
+                     table_entry(t.cb1r + (size_t)t.i1r[io] * hf, xv + hf, hf));
+        acc = acc + (table_entry(t.cb2l + (size_t)l2_at(t, t.i2l + (size_t)r * l2s, c) * hf, xv, hf) +
+                     table_entry(t.cb2r + (size_t)l2_at(t, t.i2r + (size_t)r * l2s, c) * hf, xv + hf, hf));
+    }
+    return acc;
+}
+
+// KA: every codebook a multiple of 32 codes (every table row of a tile is
+// stored).  LV: 1 one level; 2 both, the second's tables beside the first's in
+// LDS (132 KB at 256 codes each) and its index bytes behind the first's; 3 the
+// second's indices packed 4-bit (16 codes).  NR: row
+// tiles per block, the tables shared by both (used where one tile each would
+// need a second round of blocks: 32000 x 4096, level 1, 504 blocks of one 17.7
+// us, 256 of two 13.5 us).
+template <bool KA, int LV, int NR>
 __global__ __launch_bounds__(kFThreads) void pq_fused(PqDev t, const float* __restrict__ x, float* __restrict__ out,
                                                       int S, unsigned long long* __restrict__ racc,
                                                       const unsigned long long* __restrict__ hdr) {
     constexpr int CS = kFCS;
+    constexpr bool TWO = LV > 1, P4 = LV == 3;
     extern __shared__ __align__(16) float T[];            // [CS][TS]
-    __shared__ float red[kFThreads / 64], redc[kFThreads / 64];
+    __shared__ float red[kFThreads / 64], redc[kFThreads / 64], redc2[TWO ? kFThreads / 64 : 1];
     __shared__ float cmax_s[2][CS];
     __shared__ int8_t qq_s[1024];
     __shared__ float meta_s;
-    __shared__ h8_t cbs[2 * 256];                          // both codebooks, fp16 rows padded to 8
+    __shared__ h8_t cbs[(TWO ? 4 : 2) * 256];              // the codebooks, fp16 rows padded to 8
     __shared__ __align__(16) float xsl[CS * kXS];          // the slab's x: [chunk][side][8], zero padded
     const int K = t.K, C = t.C, G = t.G, M = t.M, hf = G / 2;
     const int TS = 2 * K + 4;                              // padded chunk stride (bank spread)
+    const int K2 = TWO ? t.K2 : 0, TS2 = 2 * K2 + 4;
+    float* T2 = T + (size_t)CS * TS;                       // TWO: [CS][TS2]
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     // XCD-aware order: dispatch puts block b on XCD b % 8, so logical block
@@ -481,12 +522,13 @@ __global__ __launch_bounds__(kFThreads) void pq_fused(PqDev t, const float* __re
     const int rt = lb / S, sl = lb - rt * S;
     const int c0 = sl * CS, cn = min(CS, C - c0);
     const int q = tid & 1;
-    const int r = rt * kFRows + (tid >> 1);
-    const int row = min(r, M - 1);
+    const int r0 = rt * (kFRows * NR) + (tid >> 1);        // row of tile h: r0 + h * kFRows
     // the workspace stamp (caller workspaces): its address, and the magic
     const bool wsok = !hdr || (hdr[0] == kPqStamp && hdr[1] == (unsigned long long)(uintptr_t)hdr);
     if (S > 1 && !wsok) {
-        if (q == 0 && r < M) out[r] = __builtin_nanf("");
+#pragma unroll
+        for (int h = 0; h < NR; h++)
+            if (q == 0 && r0 + h * kFRows < M) out[r0 + h * kFRows] = __builtin_nanf("");
         if (tid == 0) __hip_atomic_fetch_or(&ibh_pq_err, (unsigned)IBH_DEVERR_PQ_WS, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         return;
     }
@@ -505,6 +547,11 @@ __global__ __launch_bounds__(kFThreads) void pq_fused(PqDev t, const float* __re
         const int ci = min(tid, 2 * K - 1);
         cbv = *(const uint4*)((ci < K ? t.cb1l : t.cb1r) + (size_t)(ci < K ? ci : ci - K) * 8);
     }
+    uint4 cbv2 = make_uint4(0, 0, 0, 0);
+    if (TWO && cb16) {
+        const int ci = min(tid, 2 * K2 - 1);
+        cbv2 = *(const uint4*)((ci < K2 ? t.cb2l : t.cb2r) + (size_t)(ci < K2 ? ci : ci - K2) * 8);
+    }
     __builtin_amdgcn_sched_barrier(0);
     float4 xs4[4];
     if (x4ok) {
@@ -517,13 +564,27 @@ __global__ __launch_bounds__(kFThreads) void pq_fused(PqDev t, const float* __re
     // slab is ragged; a load under a branch is waited for where it joins)
     __builtin_amdgcn_sched_barrier(0);
     const bool vec = cn == CS && (C & 15) == 0;
-    const size_t io = vec ? (size_t)row * C + c0 + 16 * q : 0;
-    const uint4 ivl = *(const uint4*)(t.i1l + io);
-    const uint4 ivr = *(const uint4*)(t.i1r + io);
+    // level 2: 16 bytes a side, or 8 of packed 4-bit indices (C % 16 == 0: whole bytes)
+    uint4 ivl[NR], ivr[NR], jvl[NR], jvr[NR];
+#pragma unroll
+    for (int h = 0; h < NR; h++) {
+        const size_t io = vec ? (size_t)min(r0 + h * kFRows, M - 1) * C + c0 + 16 * q : 0;
+        ivl[h] = *(const uint4*)(t.i1l + io);
+        ivr[h] = *(const uint4*)(t.i1r + io);
+        jvl[h] = jvr[h] = make_uint4(0, 0, 0, 0);
+        if constexpr (P4) {
+            const uint2 a = *(const uint2*)((vec ? t.i2l : t.i1l) + io / 2), b = *(const uint2*)((vec ? t.i2r : t.i1r) + io / 2);
+            jvl[h] = make_uint4(a.x, a.y, 0, 0);
+            jvr[h] = make_uint4(b.x, b.y, 0, 0);
+        } else if constexpr (TWO) {
+            jvl[h] = *(const uint4*)((vec ? t.i2l : t.i1l) + io);
+            jvr[h] = *(const uint4*)((vec ? t.i2r : t.i1r) + io);
+        }
+    }
     PQ_TT(0);
 
     // codebooks and the slab's x into LDS; the slab's max|x| and max|codeword|
-    float mc = 0.f, ms = 0.f;
+    float mc = 0.f, ms = 0.f, mc2 = 0.f;
     if (tid < 2 * K) {
         h8_t h;
         if (cb16) h = __builtin_bit_cast(h8_t, cbv);
@@ -535,6 +596,20 @@ __global__ __launch_bounds__(kFThreads) void pq_fused(PqDev t, const float* __re
         cbs[tid] = h;
 #pragma unroll
         for (int i = 0; i < 8; i++) mc = fmaxf(mc, fabsf((float)h[i]));
+    }
+    if (TWO && tid < 2 * K2) {
+        h8_t h;
+        if (cb16) h = __builtin_bit_cast(h8_t, cbv2);
+        else {
+            const uint16_t* cr = (tid < K2 ? t.cb2l : t.cb2r) + (size_t)(tid < K2 ? tid : tid - K2) * hf;
+#pragma unroll
+            for (int i = 0; i < 8; i++) h[i] = i < hf ? __builtin_bit_cast(_Float16, cr[min(i, hf - 1)]) : (_Float16)0.f;
+        }
+        cbs[2 * K + tid] = h;
+        float m2 = 0.f;
+#pragma unroll
+        for (int i = 0; i < 8; i++) m2 = fmaxf(m2, fabsf((float)h[i]));
+        mc2 = m2;
     }
     if (slab4) {
         if (tid < cn * 4) {
@@ -551,26 +626,38 @@ __global__ __launch_bounds__(kFThreads) void pq_fused(PqDev t, const float* __re
     }
     ms = wave_max_dpp(ms);
     mc = wave_max_dpp(mc);
+    if (TWO) mc2 = wave_max_dpp(mc2);
     if (lane == 0) {
         red[wave] = ms;
         redc[wave] = mc;
+        if (TWO) redc2[wave] = mc2;
     }
     __syncthreads();
-    float smax = 0.f, cbmax = 0.f;
+    float smax = 0.f, cbmax = 0.f, cbmax2 = 0.f;
 #pragma unroll
     for (int w = 0; w < kFThreads / 64; w++) {
         smax = fmaxf(smax, red[w]);
         cbmax = fmaxf(cbmax, redc[w]);
+        if (TWO) cbmax2 = fmaxf(cbmax2, redc2[w]);
     }
-    // the tables carry 2^-ex, ex the exponent of the slab's max|x|
+    if (TWO) cbmax += cbmax2;
+    // the tables carry 2^-ex: x scaled so that the slab's max|x| sits just
+    // below 2^15, the top of fp16, and the low halves of its elements stay
+    // normal numbers down to 2^-17 of it
     int ex = 0;
     if (smax > 0.f) frexpf(smax, &ex);                     // smax < 2^ex
+    ex = max(ex, -100) - 15;
     const float xscale = ldexpf(1.0f, -ex);
 
     // 2. tables: items (side, 32-code tile, 32-chunk tile), <= 32
     const int KT = (K + 31) / 32, CT = (cn + 31) / 32, items = 2 * KT * CT;
     for (int it = wave; it < items; it += kFThreads / 64)
-        table_tile<KA, CS>(t, cbs, xsl, it, KT, CT, cn, lane, TS, xscale, T, cmax_s);
+        table_tile<KA, CS, true>(K, cbs, xsl, it, KT, CT, cn, lane, TS, xscale, T, cmax_s);
+    if constexpr (TWO) {
+        const int KT2 = (K2 + 31) / 32;
+        for (int it = wave; it < 2 * KT2 * CT; it += kFThreads / 64)
+            table_tile<KA, CS, false>(K2, cbs + 2 * K, xsl, it, KT2, CT, cn, lane, TS2, xscale, T2, cmax_s);
+    }
     PQ_TT(1);
     // max|x| over the inner columns (the skipping rule's reference)
     // (fmaxf drops NaN, so non-finite inputs are flagged on their own)
@@ -614,69 +701,90 @@ __global__ __launch_bounds__(kFThreads) void pq_fused(PqDev t, const float* __re
     const unsigned long long full = cn == 64 ? ~0ull : ((1ull << cn) - 1);
     PQ_TT(2);
 
-    // 4. gather: the thread's 16 chunks, L then R per chunk (entries carry 2^-ex)
-    float acc = 0.f;
-    if (vec) {
-        const uint32_t wl[4] = {ivl.x, ivl.y, ivl.z, ivl.w}, wr[4] = {ivr.x, ivr.y, ivr.z, ivr.w};
-        const float* Tq = T + (size_t)(16 * q) * TS;
-        if (keepm == full) {
+    // 2^qe maps 2 * N_inner * max|cb| * max|x| (a bound on |row sum|) to
+    // <= 2^50; the same on every slab (cbmax, gmax and the flag are over the
+    // whole tensor), so either every slab adds or none does
+    const float bound = 2.0f * (float)ninner * cbmax * gmax;
+    const bool off = x_nonfinite || !(bound <= 3.4e38f);
+    bool fin[NR];
+    float sum[NR];
+    uint16_t rs_bits[NR];
 #pragma unroll
-            for (int j = 0; j < 16; j++) {
+    for (int h = 0; h < NR; h++) {
+        const int r = r0 + h * kFRows;
+        // 4. gather: the thread's 16 chunks, L then R per chunk (entries carry 2^-ex)
+        float acc = 0.f;
+        if (vec) {
+            const uint32_t wl[4] = {ivl[h].x, ivl[h].y, ivl[h].z, ivl[h].w}, wr[4] = {ivr[h].x, ivr[h].y, ivr[h].z, ivr[h].w};
+            const uint32_t vl[4] = {jvl[h].x, jvl[h].y, jvl[h].z, jvl[h].w}, vr[4] = {jvr[h].x, jvr[h].y, jvr[h].z, jvr[h].w};
+            const float* Tq = T + (size_t)(16 * q) * TS;
+            const float* Tq2 = T2 + (size_t)(16 * q) * TS2;
+            auto term = [&](int j) {
                 const int il = (wl[j >> 2] >> (8 * (j & 3))) & 0xff, ir = (wr[j >> 2] >> (8 * (j & 3))) & 0xff;
-                acc = acc + (Tq[j * TS + il] + Tq[j * TS + K + ir]);
+                float v = Tq[j * TS + il] + Tq[j * TS + K + ir];
+                if constexpr (TWO) {
+                    const int jl = P4 ? (vl[j >> 3] >> (4 * (j & 7))) & 0xf : (vl[j >> 2] >> (8 * (j & 3))) & 0xff;
+                    const int jr = P4 ? (vr[j >> 3] >> (4 * (j & 7))) & 0xf : (vr[j >> 2] >> (8 * (j & 3))) & 0xff;
+                    v = v + (Tq2[j * TS2 + jl] + Tq2[j * TS2 + K2 + jr]);
+                }
+                return v;
+            };
+            if (keepm == full) {
+#pragma unroll
+                for (int j = 0; j < 16; j++) acc = acc + term(j);
+            } else {
+#pragma unroll
+                for (int j = 0; j < 16; j++) {
+                    const float val = term(j);
+                    acc = acc + (((keepm >> (16 * q + j)) & 1) ? val : 0.f);
+                }
             }
-        } else {
-#pragma unroll
-            for (int j = 0; j < 16; j++) {
-                const int c = 16 * q + j;
-                const int il = (wl[j >> 2] >> (8 * (j & 3))) & 0xff, ir = (wr[j >> 2] >> (8 * (j & 3))) & 0xff;
-                const float val = Tq[j * TS + il] + Tq[j * TS + K + ir];
+        } else if (r < M) {
+            const uint8_t* pl = t.i1l + (size_t)r * C + c0;
+            const uint8_t* pr = t.i1r + (size_t)r * C + c0;
+            const size_t l2s = TWO ? l2_stride(t) : 0;
+            for (int c = 16 * q; c < min(16 * q + 16, cn); c++) {
+                const float* Tc = T + (size_t)c * TS;
+                float val = Tc[pl[c]] + Tc[K + pr[c]];
+                if constexpr (TWO) {
+                    const float* Tc2 = T2 + (size_t)c * TS2;
+                    val = val + (Tc2[l2_at(t, t.i2l + (size_t)r * l2s, c0 + c)] +
+                                 Tc2[K2 + l2_at(t, t.i2r + (size_t)r * l2s, c0 + c)]);
+                }
                 acc = acc + (((keepm >> c) & 1) ? val : 0.f);
             }
         }
-    } else if (r < M) {
-        const uint8_t* pl = t.i1l + (size_t)r * C + c0;
-        const uint8_t* pr = t.i1r + (size_t)r * C + c0;
-        for (int c = 16 * q; c < min(16 * q + 16, cn); c++) {
-            const float* Tc = T + (size_t)c * TS;
-            const float val = Tc[pl[c]] + Tc[K + pr[c]];
-            acc = acc + (((keepm >> c) & 1) ? val : 0.f);
-        }
-    }
-    // the row's two partials, lanes 2i, 2i+1
-    acc += __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, acc), 0xB1, 0xF, 0xF, false));
-    PQ_TT(3);
+        // the row's two partials, lanes 2i, 2i+1
+        acc += __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, acc), 0xB1, 0xF, 0xF, false));
+        PQ_TT(3);
 
-    // 5. the rows' words
-    const bool own = q == 0 && r < M;
-    bool fin = own;
-    float sum = ldexpf(acc, ex);
-    const uint16_t rs_bits = t.row_scale[row];   // in flight with the atomic below
-    if (S > 1) {
-        // 2^qe maps 2 * N_inner * max|cb| * max|x| (a bound on |row sum|) to
-        // <= 2^50; the same on every slab (cbmax, gmax and the flag are over
-        // the whole tensor), so either every slab adds or none does
-        const float bound = 2.0f * (float)ninner * cbmax * gmax;
-        if (x_nonfinite || !(bound <= 3.4e38f)) {
+        // 5. the rows' words
+        const bool own = q == 0 && r < M;
+        fin[h] = own;
+        sum[h] = ldexpf(acc, ex);
+        rs_bits[h] = t.row_scale[min(r, M - 1)];   // in flight with the atomic below
+        if (TWO && off) {
+            fin[h] = own && sl == 0;
+            if (fin[h]) sum[h] = plain_row(t, x, r, gmax);
+        } else if (S > 1 && off) {
             if (own) out[r] = __builtin_nanf("");
-            return;
+            fin[h] = false;
         }
-    }
-    if (S > 1 && own) {
-        const float bound = 2.0f * (float)ninner * cbmax * gmax;
-        int eb = 0;
-        if (bound > 0.f) frexpf(bound, &eb);               // bound < 2^eb
-        const int qe = 50 - eb;
-        const long long v = llrint((double)acc * ldexp(1.0, qe + ex));
-        const unsigned long long add = (1ull << 58) + (unsigned long long)(v + (1ll << 50));
-        const unsigned long long old =
-            __hip_atomic_fetch_add(&words[r], add, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        const unsigned long long tot = old + add;
-        fin = (tot >> 58) == (unsigned long long)S;
-        if (fin) {
-            const long long val = (long long)(tot & ((1ull << 58) - 1)) - (long long)S * (1ll << 50);
-            sum = (float)((double)val * ldexp(1.0, -qe));
-            __hip_atomic_store(&words[r], 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (S > 1 && own && !off) {
+            int eb = 0;
+            if (bound > 0.f) frexpf(bound, &eb);               // bound < 2^eb
+            const int qe = 50 - eb;
+            const long long v = llrint((double)acc * ldexp(1.0, qe + ex));
+            const unsigned long long add = (1ull << 58) + (unsigned long long)(v + (1ll << 50));
+            const unsigned long long old =
+                __hip_atomic_fetch_add(&words[r], add, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            const unsigned long long tot = old + add;
+            fin[h] = (tot >> 58) == (unsigned long long)S;
+            if (fin[h]) {
+                const long long val = (long long)(tot & ((1ull << 58) - 1)) - (long long)S * (1ll << 50);
+                sum[h] = (float)((double)val * ldexp(1.0, -qe));
+                __hip_atomic_store(&words[r], 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            }
         }
     }
     PQ_TT(4);
@@ -685,7 +793,10 @@ __global__ __launch_bounds__(kFThreads) void pq_fused(PqDev t, const float* __re
     const int no = t.n_outlier;
     const bool quant = no >= 32;
     if (no > 0) {
-        if (__syncthreads_or(fin) == 0) return;
+        bool any = false;
+#pragma unroll
+        for (int h = 0; h < NR; h++) any |= fin[h];
+        if (__syncthreads_or(any) == 0) return;
         if (quant) {
             if (tid == 0) {
                 float m = 0.f;
@@ -706,19 +817,23 @@ __global__ __launch_bounds__(kFThreads) void pq_fused(PqDev t, const float* __re
             __syncthreads();
         }
     }
-    if (!fin) return;
-    float y = sum * f16_to_f32(rs_bits);
-    if (no > 0) {
-        const int8_t* sdc = t.oside + (size_t)r * no;
-        if (quant) {
-            int32_t isum = 0;
-            for (int j = 0; j < no; j++) isum += (int32_t)sdc[j] * (int32_t)qq_s[j];
-            y = fmaf((float)isum, meta_s, y);
-        } else {
-            for (int j = 0; j < no; j++) y = fmaf((float)sdc[j] * f16_to_f32(t.oscale[j]), x[t.ocols[j]], y);
+#pragma unroll
+    for (int h = 0; h < NR; h++) {
+        if (!fin[h]) continue;
+        const int r = r0 + h * kFRows;
+        float y = sum[h] * f16_to_f32(rs_bits[h]);
+        if (no > 0) {
+            const int8_t* sdc = t.oside + (size_t)r * no;
+            if (quant) {
+                int32_t isum = 0;
+                for (int j = 0; j < no; j++) isum += (int32_t)sdc[j] * (int32_t)qq_s[j];
+                y = fmaf((float)isum, meta_s, y);
+            } else {
+                for (int j = 0; j < no; j++) y = fmaf((float)sdc[j] * f16_to_f32(t.oscale[j]), x[t.ocols[j]], y);
+            }
         }
+        out[r] = y;
     }
-    out[r] = y;
     PQ_TT(5);
 }
 
@@ -736,8 +851,7 @@ constexpr int kSelThreads = 1024;
 // per-wavefront histograms, the bin search one wavefront-wide scan), then
 // every element above it plus the first ties of the K-th key in index order;
 // the selection ends sorted by row index.  One block.
-__global__ __launch_bounds__(kSelThreads) void pq_topk_select(const float* __restrict__ v, int M, int K,
-                                                              int32_t* __restrict__ sel) {
+__device__ void topk_radix(const float* __restrict__ v, int M, int K, int32_t* __restrict__ sel) {
     constexpr int NW = kSelThreads / 64;
     __shared__ int hist[NW][256];
     __shared__ int tot[256];
@@ -836,109 +950,172 @@ __global__ __launch_bounds__(kSelThreads) void pq_topk_select(const float* __res
     for (int i = tid; i < K; i += kSelThreads) sel[i] = tmp[i];
 }
 
-// Two-pass selection for small K on long vectors: every block of
-// kLocalSpan values keeps its K largest (ties: lowest index) in descending
-// order, then the one-block select runs over the B*K candidates.  The global
-// K largest are among the candidates, and the candidates' order (block,
-// rank) agrees with row order among equal values, so the result equals the
-// one-pass select.
-constexpr int kLocalSpan = 1024, kLocalMaxK = 16;
-
-__global__ __launch_bounds__(256) void pq_topk_local(const float* __restrict__ v, int M, int K,
-                                                     float* __restrict__ cval, int32_t* __restrict__ cidx) {
-    constexpr int PER = kLocalSpan / 256;
-    __shared__ uint32_t wk[4];
-    __shared__ int wi[4];
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int base = blockIdx.x * kLocalSpan;
-    uint32_t key[PER];   // descending key: smaller = larger value; taken = 0xFFFFFFFF
-#pragma unroll
-    for (int j = 0; j < PER; j++) {
-        const int i = base + threadIdx.x + 256 * j;
-        key[j] = i < M ? desc_key(v[i]) : 0xFFFFFFFFu;
-    }
-    for (int r = 0; r < K; r++) {
-        uint32_t bk = 0xFFFFFFFFu;
-        int bi = 0x7fffffff;
-#pragma unroll
-        for (int j = 0; j < PER; j++) {
-            const int i = base + threadIdx.x + 256 * j;
-            if (key[j] < bk || (key[j] == bk && i < bi)) { bk = key[j]; bi = i; }
-        }
-#pragma unroll
-        for (int o = 32; o > 0; o >>= 1) {
-            const uint32_t ok = __shfl_xor(bk, o, 64);
-            const int oi = __shfl_xor(bi, o, 64);
-            if (ok < bk || (ok == bk && oi < bi)) { bk = ok; bi = oi; }
-        }
-        if (lane == 0) { wk[wave] = bk; wi[wave] = bi; }
-        __syncthreads();
-        uint32_t k2 = wk[0];
-        int i2 = wi[0];
-        for (int w = 1; w < 4; w++)
-            if (wk[w] < k2 || (wk[w] == k2 && wi[w] < i2)) { k2 = wk[w]; i2 = wi[w]; }
-        if (threadIdx.x == 0) {
-            const bool ok = k2 != 0xFFFFFFFFu;
-            cval[blockIdx.x * K + r] = ok ? v[i2] : -INFINITY;
-            cidx[blockIdx.x * K + r] = ok ? i2 : 0x7fffffff;
-        }
-#pragma unroll
-        for (int j = 0; j < PER; j++)
-            if (base + (int)threadIdx.x + 256 * j == i2) key[j] = 0xFFFFFFFFu;
-        __syncthreads();
-    }
+__global__ __launch_bounds__(kSelThreads) void pq_topk_select(const float* __restrict__ v, int M, int K,
+                                                              int32_t* __restrict__ sel) {
+    topk_radix(v, M, K, sel);
 }
 
-// Candidate positions -> rows, in row order (K <= kLocalMaxK).
-__global__ void pq_topk_rows(const int32_t* __restrict__ selc, const int32_t* __restrict__ cidx, int K,
-                             int32_t* __restrict__ sel) {
-    __shared__ int rows[kLocalMaxK];
-    if (threadIdx.x < K) rows[threadIdx.x] = cidx[selc[threadIdx.x]];
+// The same selection for K <= kPickK without histograms (logits crowd a few
+// exponents, so the radix passes' LDS atomics pile up on a few bins: 44.8 us
+// for 50 of 32000).  Each thread keeps the best of its share; the K-th best of
+// those 1024 is a bound that at least K values reach and few others do, found
+// bit by bit with ballots; the values within it (more than kSelThreads of
+// them, as with many ties, take the radix passes) are ranked by (key, index)
+// against each other.  One block, one read of v up to 32768 values: 13.4 us.
+constexpr int kPickK = 256, kPickPer = 32;
+
+__global__ __launch_bounds__(kSelThreads) void pq_topk_pick(const float* __restrict__ v, int M, int K,
+                                                            int32_t* __restrict__ sel) {
+    constexpr int NW = kSelThreads / 64;
+    __shared__ __align__(16) int cnt[2][NW];
+    __shared__ unsigned long long ck[kSelThreads];        // key, row
+    __shared__ int pick[kPickK];
+    __shared__ int nc_s;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    if (tid == 0) nc_s = 0;
+    // v is a workspace array of whole 256-byte lines, so the last float4 may
+    // hold values past M that no key is made of
+    uint32_t key[kPickPer], best = 0xFFFFFFFFu;
+    const int span = kPickPer * kSelThreads, n4 = (M + 3) >> 2;
+    auto at = [&](int base, int u) { return base + 4 * ((u >> 2) * kSelThreads + tid) + (u & 3); };
+    auto load = [&](int base) {
+        float4 f[kPickPer / 4];
+#pragma unroll
+        for (int u = 0; u < kPickPer / 4; u++) f[u] = ((const float4*)v)[min(base / 4 + u * kSelThreads + tid, n4 - 1)];
+#pragma unroll
+        for (int u = 0; u < kPickPer; u++) {
+            const float4 q = f[u >> 2];
+            const float e = (u & 3) == 0 ? q.x : (u & 3) == 1 ? q.y : (u & 3) == 2 ? q.z : q.w;
+            key[u] = at(base, u) < M ? desc_key(e) : 0xFFFFFFFFu;
+        }
+    };
+    for (int base = 0; base < M; base += span) {
+        load(base);
+#pragma unroll
+        for (int u = 0; u < kPickPer; u++) best = min(best, key[u]);
+    }
+    // smallest bound with at least K of the threads' best keys at or below it
+    uint32_t p = 0;
+    for (int bit = 31; bit >= 0; bit--) {
+        const uint32_t trial = p + ((1u << bit) - 1u);
+        const int c = __popcll(__ballot(best <= trial));
+        if (lane == 0) cnt[bit & 1][wave] = c;
+        __syncthreads();
+        int n = 0;
+#pragma unroll
+        for (int w = 0; w < NW; w += 4) {
+            const int4 q = *(const int4*)&cnt[bit & 1][w];
+            n += q.x + q.y + q.z + q.w;
+        }
+        if (n < K) p += 1u << bit;
+    }
+    for (int base = 0; base < M; base += span) {
+        if (M > span) load(base);
+#pragma unroll
+        for (int u = 0; u < kPickPer; u++) {
+            const int i = at(base, u);
+            if (i < M && key[u] <= p) {
+                const int n = atomicAdd(&nc_s, 1);
+                if (n < kSelThreads) ck[n] = ((unsigned long long)key[u] << 32) | (uint32_t)i;
+            }
+        }
+    }
     __syncthreads();
-    if (threadIdx.x < K) {
-        const int r = rows[threadIdx.x];
+    const int nc = nc_s;
+    if (nc > kSelThreads) {
+        topk_radix(v, M, K, sel);
+        return;
+    }
+    // ranks, 8 lanes a candidate (their shares of the comparisons independent)
+    const int sub = tid & 7;
+    for (int b = 0; b < nc; b += kSelThreads / 8) {
+        const int c = b + (tid >> 3);
+        const unsigned long long k = ck[min(c, nc - 1)];
         int rank = 0;
-        for (int j = 0; j < K; j++) rank += rows[j] < r;
-        sel[rank] = r;
+#pragma unroll 4
+        for (int j = sub; j < nc; j += 8) rank += ck[j] < k;
+        rank = (int)group_sum_dpp<8>((float)rank);
+        if (c < nc && rank < K && sub == 0) pick[rank] = (int)(uint32_t)k;
+    }
+    __syncthreads();
+    for (int b = 0; b < K; b += kSelThreads / 8) {
+        const int c = b + (tid >> 3), i = pick[min(c, K - 1)];
+        int rank = 0;
+#pragma unroll 4
+        for (int j = sub; j < K; j += 8) rank += pick[j] < i;
+        rank = (int)group_sum_dpp<8>((float)rank);
+        if (c < K && sub == 0) sel[rank] = i;
     }
 }
 
 // Full-pyramid logits of the selected rows (ib_pq_matmul_fp32_subset,
-// pq_decode.c:2145-2250): one wavefront per row, lanes over chunks; the
-// outlier sidecar in fp32.
+// pq_decode.c:2145-2250): one block per row, a chunk per thread, the outlier
+// sidecar in fp32.  Two dependent reads (indices, codewords) set its time, so
+// a codeword of 8 halves is one 16-byte load and no thread has a second chunk
+// up to 256 (one wavefront per row with 2-byte loads, 4 chunks a lane: 18.5 us
+// for 50 rows of 256 chunks; 5.2 us).
 __global__ __launch_bounds__(256) void pq_subset_rows(PqDev t, const float* __restrict__ x,
                                                       const int32_t* __restrict__ rows, int n,
                                                       float* __restrict__ out) {
-    const int lane = threadIdx.x & 63;
-    const int i = blockIdx.x * 4 + (threadIdx.x >> 6);
-    if (i >= n) return;
+    __shared__ float red[2][4];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int i = blockIdx.x;
     const int r = rows[i], C = t.C, G = t.G, hf = G / 2;
-    const size_t l2s = t.n_levels == 2 ? l2_stride(t) : 0;
+    const bool two = t.n_levels == 2;
+    const size_t l2s = two ? l2_stride(t) : 0;
+    const bool wide = hf == 8 && (((uintptr_t)t.cb1l | (uintptr_t)t.cb1r | (two ? (uintptr_t)t.cb2l | (uintptr_t)t.cb2r : 0)) & 15) == 0;
     float acc = 0.f;
-    for (int c = lane; c < C; c += 64) {
-        const uint16_t* el = t.cb1l + (size_t)t.i1l[(size_t)r * C + c] * hf;
-        const uint16_t* er = t.cb1r + (size_t)t.i1r[(size_t)r * C + c] * hf;
-        const uint16_t *e2l = nullptr, *e2r = nullptr;
-        if (t.n_levels == 2) {
-            e2l = t.cb2l + (size_t)l2_at(t, t.i2l + (size_t)r * l2s, c) * hf;
-            e2r = t.cb2r + (size_t)l2_at(t, t.i2r + (size_t)r * l2s, c) * hf;
+    for (int c = tid; c < C; c += 256) {
+        const uint16_t* e[4];
+        e[0] = t.cb1l + (size_t)t.i1l[(size_t)r * C + c] * hf;
+        e[1] = t.cb1r + (size_t)t.i1r[(size_t)r * C + c] * hf;
+        e[2] = two ? t.cb2l + (size_t)l2_at(t, t.i2l + (size_t)r * l2s, c) * hf : e[0];
+        e[3] = two ? t.cb2r + (size_t)l2_at(t, t.i2r + (size_t)r * l2s, c) * hf : e[1];
+        if (wide) {
+            uint4 w[4];
+#pragma unroll
+            for (int k = 0; k < 4; k++) w[k] = *(const uint4*)e[k];
+            float xv[16];
+#pragma unroll
+            for (int j = 0; j < 16; j++) xv[j] = x[inner_col(t, c * 16 + j)];
+#pragma unroll
+            for (int j = 0; j < 8; j++) {
+                auto half = [&](int k) {
+                    const uint32_t d[4] = {w[k].x, w[k].y, w[k].z, w[k].w};
+                    return f16_to_f32((uint16_t)(d[j >> 1] >> (16 * (j & 1))));
+                };
+                acc = fmaf(half(0), xv[j], acc);
+                acc = fmaf(half(1), xv[8 + j], acc);
+                if (two) {
+                    acc = fmaf(half(2), xv[j], acc);
+                    acc = fmaf(half(3), xv[8 + j], acc);
+                }
+            }
+            continue;
         }
         for (int j = 0; j < hf; j++) {
             const float xl = x[inner_col(t, c * G + j)], xr = x[inner_col(t, c * G + hf + j)];
-            acc = fmaf(f16_to_f32(el[j]), xl, acc);
-            acc = fmaf(f16_to_f32(er[j]), xr, acc);
-            if (e2l) {
-                acc = fmaf(f16_to_f32(e2l[j]), xl, acc);
-                acc = fmaf(f16_to_f32(e2r[j]), xr, acc);
+            acc = fmaf(f16_to_f32(e[0][j]), xl, acc);
+            acc = fmaf(f16_to_f32(e[1][j]), xr, acc);
+            if (two) {
+                acc = fmaf(f16_to_f32(e[2][j]), xl, acc);
+                acc = fmaf(f16_to_f32(e[3][j]), xr, acc);
             }
         }
     }
-    acc = wave_sum(acc) * f16_to_f32(t.row_scale[r]);
     float o = 0.f;
-    for (int j = lane; j < t.n_outlier; j += 64)
+    for (int j = tid; j < t.n_outlier; j += 256)
         o = fmaf((float)t.oside[(size_t)r * t.n_outlier + j] * f16_to_f32(t.oscale[j]), x[t.ocols[j]], o);
+    acc = wave_sum(acc);
     o = wave_sum(o);
-    if (lane == 0) out[i] = acc + o;
+    if (lane == 0) {
+        red[0][wave] = acc;
+        red[1][wave] = o;
+    }
+    __syncthreads();
+    if (tid == 0)
+        out[i] = ((red[0][0] + red[0][1]) + (red[0][2] + red[0][3])) * f16_to_f32(t.row_scale[r]) +
+                 ((red[1][0] + red[1][1]) + (red[1][2] + red[1][3]));
 }
 
 // Descending order of the refined logits (the reference's insertion sort:
@@ -1216,17 +1393,32 @@ static int pq_run(const ibh_pq_tensor_abi* t, const float* x, float* out, void* 
     float* c2max = (float*)(base + w.c2max);
     d.cnorm = cnorm;
     d.c2max = c2max;
-    // one launch for level-1 work with half-chunks of <= 8 columns and <= 256
-    // codes (the scope of pq_fused); other tensors and policies take the
-    // three-kernel path below
-    const int tiles = (t->M + kFRows - 1) / kFRows;
+    // one launch for half-chunks of <= 8 columns and <= 256 codes a level with
+    // byte or 4-bit level-2 indices (the scope of pq_fused); 2-byte indices,
+    // the level-2 skip and the int8 tables take the three-kernel path below
+    int tiles = (t->M + kFRows - 1) / kFRows;
     const int S = (t->C + kFCS - 1) / kFCS;
-    if (!two && !md.q8 && !md.tq8 && t->G <= 16 && t->K <= 256 && S <= kFMaxS && t->M <= kFMaxRows && g_pq_fused) {
-        const size_t flds = (size_t)kFCS * (2 * t->K + 4) * sizeof(float);
+    const bool l2ok = !two || (!d.l2skip && d.l2_idx_bytes == 1 && d.K2 <= 256);
+    if (l2ok && !md.q8 && !md.tq8 && t->G <= 16 && t->K <= 256 && S <= kFMaxS && t->M <= kFMaxRows && g_pq_fused) {
+        const size_t flds = (size_t)kFCS * (2 * t->K + 4 + (two ? 2 * d.K2 + 4 : 0)) * sizeof(float);
         unsigned long long* hdr = own_ws ? (unsigned long long*)ws : nullptr;
         unsigned long long* racc = own_ws ? hdr + 32 : nullptr;
-        if (t->K % 32 == 0) pq_fused<true><<<tiles * S, kFThreads, flds, st>>>(d, x, out, S, racc, hdr);
-        else pq_fused<false><<<tiles * S, kFThreads, flds, st>>>(d, x, out, S, racc, hdr);
+        const bool ka = t->K % 32 == 0 && (!two || d.K2 % 32 == 0);
+        const bool nr2 = tiles * S > 256;                  // more than one round of blocks
+        if (nr2) tiles = (tiles + 1) / 2;
+#define IBH_PF1(A_, L_, R_) do { \
+        if (L_ > 1 && flds > 65536 && hipFuncSetAttribute((const void*)pq_fused<A_, L_, R_>, hipFuncAttributeMaxDynamicSharedMemorySize, \
+                                                          (int)flds) != hipSuccess) { \
+            ibh_set_error("%s: %zu bytes of LDS not available", who, flds); \
+            return IBH_ERROR_INTERNAL; } \
+        pq_fused<A_, L_, R_><<<tiles * S, kFThreads, flds, st>>>(d, x, out, S, racc, hdr); } while (0)
+#define IBH_PF(A_, L_) do { if (nr2) IBH_PF1(A_, L_, 2); else IBH_PF1(A_, L_, 1); } while (0)
+        if (two && d.K2 == 16) IBH_PF(false, 3);
+        else if (two) { if (ka) IBH_PF(true, 2); else IBH_PF(false, 2); }
+        else if (ka) IBH_PF(true, 1);
+        else IBH_PF(false, 1);
+#undef IBH_PF
+#undef IBH_PF1
         IBH_CHECK_LAUNCH("ibh_pq_matmul (one launch)");
         return IBH_OK;
     }
@@ -1258,8 +1450,7 @@ static size_t pq_topk_need(const ibh_pq_tensor_abi* t, int k_top, bool front) {
     const size_t base = pq_ws_need(t, front);
     if (!base || k_top <= 0) return 0;
     auto al = [](size_t v) { return (v + 255) / 256 * 256; };
-    const size_t nb = ((size_t)t->M + kLocalSpan - 1) / kLocalSpan;   // two-pass select candidates
-    return base + al((size_t)t->M * 4) + 3 * al((size_t)k_top * 4) + 2 * al(nb * kLocalMaxK * 4);
+    return base + al((size_t)t->M * 4) + 2 * al((size_t)k_top * 4);
 }
 
 extern "C" size_t ibh_pq_topk_workspace_bytes(const ibh_pq_tensor_abi* t, int k_top) {
@@ -1299,21 +1490,9 @@ extern "C" int ibh_pq_lm_head_topk(const ibh_pq_tensor_abi* t, const float* x, i
     int rc = pq_run(t, x, coarse, ws, base, stream, md, "ibh_pq_lm_head_topk", lib_ws);
     if (rc) return rc;
     // 2. the K largest, 3. their full-pyramid logits, 4. sorted
-    const int nb = (t->M + kLocalSpan - 1) / kLocalSpan;
-    if (k_top <= kLocalMaxK && nb >= 4) {
-        int32_t* selc = (int32_t*)((char*)refined + al((size_t)k_top * 4));
-        float* cval = (float*)((char*)selc + al((size_t)k_top * 4));
-        int32_t* cidx = (int32_t*)((char*)cval + al((size_t)nb * kLocalMaxK * 4));
-        pq_topk_local<<<nb, 256, 0, st>>>(coarse, t->M, k_top, cval, cidx);
-        IBH_CHECK_LAUNCH("ibh_pq_lm_head_topk (local select)");
-        pq_topk_select<<<1, kSelThreads, 0, st>>>(cval, nb * k_top, k_top, selc);
-        IBH_CHECK_LAUNCH("ibh_pq_lm_head_topk (select)");
-        pq_topk_rows<<<1, 64, 0, st>>>(selc, cidx, k_top, sel);
-        IBH_CHECK_LAUNCH("ibh_pq_lm_head_topk (rows)");
-    } else {
-        pq_topk_select<<<1, kSelThreads, 0, st>>>(coarse, t->M, k_top, sel);
-        IBH_CHECK_LAUNCH("ibh_pq_lm_head_topk (select)");
-    }
+    if (k_top <= kPickK) pq_topk_pick<<<1, kSelThreads, 0, st>>>(coarse, t->M, k_top, sel);
+    else pq_topk_select<<<1, kSelThreads, 0, st>>>(coarse, t->M, k_top, sel);
+    IBH_CHECK_LAUNCH("ibh_pq_lm_head_topk (select)");
     PqDev d{};
     d.M = t->M; d.N = t->N; d.G = t->G; d.K = t->K; d.K2 = t->K_l2 > 0 ? t->K_l2 : t->K;
     d.n_levels = t->n_levels; d.n_outlier = t->n_outlier; d.C = t->C;
@@ -1322,7 +1501,7 @@ extern "C" int ibh_pq_lm_head_topk(const ibh_pq_tensor_abi* t, const float* x, i
     d.i1l = t->indices_l1_l; d.i1r = t->indices_l1_r; d.i2l = t->indices_l2_l; d.i2r = t->indices_l2_r;
     d.row_scale = t->row_scale; d.ocols = t->outlier_cols; d.oside = t->outlier_sidecar;
     d.oscale = t->outlier_scale; d.inner = t->n_outlier > 0 ? t->inner_cols : nullptr;
-    pq_subset_rows<<<(k_top + 3) / 4, 256, 0, st>>>(d, x, sel, k_top, refined);
+    pq_subset_rows<<<k_top, 256, 0, st>>>(d, x, sel, k_top, refined);
     IBH_CHECK_LAUNCH("ibh_pq_lm_head_topk (refine)");
     pq_topk_sort<<<1, 1024, 0, st>>>(refined, sel, k_top, out_logits, out_ids);
     IBH_CHECK_LAUNCH("ibh_pq_lm_head_topk (sort)");

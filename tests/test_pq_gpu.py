@@ -295,3 +295,79 @@ def test_pq_workspace_needs_stamp(ops, oracle_lib):
     torch.cuda.synchronize()
     assert relerr(out.cpu().numpy(), oracle_lib.pq_matmul(t, x)) <= 1e-4
     assert lib.ibh_device_errors(0) == 0
+
+
+def _fused(ops, on):
+    import libinferbit_amd as L
+    L.lib().ibh_pq_set_fused(int(on))
+
+
+# M, C, G, K, K2, outliers: whole and partial row tiles and slabs, odd chunk
+# counts (byte-wise indices), packed 4-bit and byte level-2 indices, codebooks
+# that are not whole 32-code tiles, short half-chunks, both outlier rules
+TWO_LEVEL = [(512, 32, 16, 256, 256, 0), (700, 33, 16, 256, 256, 8), (1, 1, 16, 256, 16, 0), (513, 95, 16, 256, 16, 40),
+             (300, 64, 16, 256, 64, 0), (1025, 160, 16, 100, 100, 0), (257, 48, 8, 64, 16, 4), (100, 31, 6, 16, 16, 0),
+             (64, 896, 16, 256, 256, 128), (600, 64, 4, 33, 256, 0), (4700, 864, 4, 16, 16, 4)]
+
+
+@pytest.mark.parametrize("M,C,G,K,K2,no", TWO_LEVEL)
+def test_two_level_one_launch_matches_three(ops, M, C, G, K, K2, no):
+    """The one-launch kernel on two-level tensors against the three-kernel
+    path: every chunk rule, and non-finite x value for value."""
+    from gen_golden import make_pq
+    t = make_pq(np.random.default_rng(M + C), M, C, G, K, 2, K2, no)
+    d = ops.PqDeviceTensor(t)
+    x = torch.randn(t["N"], generator=torch.Generator().manual_seed(C)) * 0.7
+    x[torch.rand(t["N"], generator=torch.Generator().manual_seed(M)) < 0.3] *= 1e-4
+    big = x.clone()
+    big[: t["N"] // 2] *= 1e30
+    inf, nan = x.clone(), x.clone()
+    inf[t["N"] // 3] = float("inf")
+    nan[t["N"] // 3] = float("nan")
+    out = torch.empty(M, device="cuda")
+    try:
+        for name, v in (("plain", x), ("tiny", x * 1e-36), ("big", big), ("inf", inf), ("nan", nan)):
+            for pol in (None, (0, 0.0, 0.0), (3, 0.0, 1e-2)):
+                print(f"case two-level {M}x{C} G={G} K={K}/{K2} no={no} {name} {pol}", flush=True)
+                got = []
+                for on in (1, 0):
+                    _fused(ops, on)
+                    for _ in range(2):
+                        if pol is None:
+                            d.matmul(v.cuda(), out)
+                        else:
+                            d.matmul_policy(v.cuda(), out, *pol)
+                    got.append(out.cpu().numpy().astype(np.float64))
+                fin = np.isfinite(got[1])
+                assert np.array_equal(fin, np.isfinite(got[0])) and np.array_equal(np.isnan(got[1]), np.isnan(got[0]))
+                assert np.array_equal(got[0][~fin & ~np.isnan(got[1])], got[1][~fin & ~np.isnan(got[1])])
+                if fin.any():
+                    # fp32 sums of up to 2 * 2 * 896 terms in two orders
+                    assert np.abs(got[0] - got[1])[fin].max() <= 2e-6 * max(np.abs(got[1][fin]).max(), 1e-37)
+    finally:
+        _fused(ops, 1)
+
+
+@pytest.mark.parametrize("M,k", [(256, 256), (300, 50), (1025, 256), (1024, 1), (33000, 8), (33000, 256), (2000, 257)])
+def test_pq_lm_head_topk_pick(ops, oracle_lib, M, k):
+    """The candidate selection at the edges of a thread's share, of the
+    one-read span (32768) and of its K limit; all logits equal (lowest rows)."""
+    from gen_golden import make_pq
+    print(f"case topk pick M={M} k={k}", flush=True)
+    t = make_pq(np.random.default_rng(M + k), M, 24, 16, 256, 2, 64, 0)
+    x = np.random.default_rng(k).standard_normal(t["N"]).astype(np.float32)
+    d = ops.PqDeviceTensor(t)
+    lg, ids = d.lm_head_topk(torch.from_numpy(x).cuda(), k)
+    want_lg, want_ids = oracle_lib.pq_lm_head_topk(t, x, k)
+    got = ids.cpu().numpy()
+    # the rows selected are the same; two may change places only where their
+    # logits are closer than the rounding of two fp32 sums of 24 * 32 terms
+    # (2 * sqrt(768) * 2^-24 of the largest)
+    np.testing.assert_array_equal(np.sort(got), np.sort(want_ids))
+    by_row = dict(zip(want_ids.tolist(), want_lg.tolist()))
+    moved = got != want_ids
+    assert np.abs(np.array([by_row[i] for i in got[moved].tolist()]) - want_lg[moved]).max(initial=0) \
+        <= 2 * 768 ** 0.5 * 2.0 ** -24 * np.abs(want_lg).max()
+    assert relerr(lg.cpu().numpy(), want_lg) <= 1e-5
+    lg, ids = d.lm_head_topk(torch.zeros(t["N"], device="cuda"), k)
+    np.testing.assert_array_equal(ids.cpu().numpy(), np.arange(k))
