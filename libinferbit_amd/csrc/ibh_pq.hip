@@ -464,9 +464,10 @@ __device__ __forceinline__ void table_tile(int K, const h8_t* cbs, const float* 
     }
 }
 
-// A row's sum from the codebooks and x directly, no tables (two-level calls
-// with a non-finite x, or sums past the fixed-point range): the entries in the
-// order of the three-kernel path, so +-Inf and NaN come out where they do there.
+// A row's sum from the codebooks and x directly, no tables and no row words
+// (two-level calls with a non-finite x, sums past the fixed-point range, or a
+// workspace without the stamp, all of which the three-kernel path served): the
+// entries in that path's order, so +-Inf and NaN come out where they do there.
 __device__ float plain_row(const PqDev& t, const float* __restrict__ x, int r, float gmax) {
     const int hf = t.G / 2;
     const size_t l2s = l2_stride(t);
@@ -525,7 +526,7 @@ __global__ __launch_bounds__(kFThreads) void pq_fused(PqDev t, const float* __re
     const int r0 = rt * (kFRows * NR) + (tid >> 1);        // row of tile h: r0 + h * kFRows
     // the workspace stamp (caller workspaces): its address, and the magic
     const bool wsok = !hdr || (hdr[0] == kPqStamp && hdr[1] == (unsigned long long)(uintptr_t)hdr);
-    if (S > 1 && !wsok) {
+    if (!TWO && S > 1 && !wsok) {
 #pragma unroll
         for (int h = 0; h < NR; h++)
             if (q == 0 && r0 + h * kFRows < M) out[r0 + h * kFRows] = __builtin_nanf("");
@@ -705,7 +706,7 @@ __global__ __launch_bounds__(kFThreads) void pq_fused(PqDev t, const float* __re
     // <= 2^50; the same on every slab (cbmax, gmax and the flag are over the
     // whole tensor), so either every slab adds or none does
     const float bound = 2.0f * (float)ninner * cbmax * gmax;
-    const bool off = x_nonfinite || !(bound <= 3.4e38f);
+    const bool off = x_nonfinite || !(bound <= 3.4e38f) || (TWO && S > 1 && !wsok);
     bool fin[NR];
     float sum[NR];
     uint16_t rs_bits[NR];

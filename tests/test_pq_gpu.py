@@ -371,3 +371,21 @@ def test_pq_lm_head_topk_pick(ops, oracle_lib, M, k):
     assert relerr(lg.cpu().numpy(), want_lg) <= 1e-5
     lg, ids = d.lm_head_topk(torch.zeros(t["N"], device="cuda"), k)
     np.testing.assert_array_equal(ids.cpu().numpy(), np.arange(k))
+
+
+def test_two_level_unprepared_workspace(ops):
+    """Two-level calls on a workspace that ibh_pq_workspace_init did not
+    prepare keep giving the product (they never needed the row words)."""
+    import ctypes
+
+    import libinferbit_amd as L
+    from gen_golden import make_pq
+    t = make_pq(np.random.default_rng(77), 300, 70, 16, 256, 2, 64, 8)
+    d = ops.PqDeviceTensor(t)
+    x = torch.randn(t["N"], generator=torch.Generator().manual_seed(3)).cuda()
+    want, out = torch.empty(300, device="cuda"), torch.empty(300, device="cuda")
+    d.matmul(x, want)
+    ws = torch.full((d.ws.numel(),), 0x5A, dtype=torch.uint8, device="cuda")
+    L._lib.check(L.lib().ibh_pq_matmul(ctypes.byref(d.s), x.data_ptr(), out.data_ptr(), ws.data_ptr(), ws.numel(),
+                                       torch.cuda.current_stream().cuda_stream), "ibh_pq_matmul")
+    assert relerr(out.cpu().numpy(), want.cpu().numpy()) <= 2e-6   # two orders of the same fp32 terms
