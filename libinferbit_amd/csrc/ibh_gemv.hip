@@ -321,66 +321,6 @@ __global__ __launch_bounds__(kBlock) void silu_quant_g128(float* __restrict__ ou
     quant_group(h[0], h[1], j0, j1, end, g, q, s);
 }
 
-// ── int8 weights x fp32 activations, batched (scalar.c:70-84) ─────────────
-template <int KIND, int BMAX>
-__global__ __launch_bounds__(kBlock) void int8_batch_fast(float* __restrict__ y,
-                                                          const uint8_t* __restrict__ W,
-                                                          const void* __restrict__ sc,
-                                                          const float* __restrict__ x,
-                                                          int M, int N, int B, int M_stride) {
-    const int lane = threadIdx.x & (kWave - 1);
-    const int row = blockIdx.x * kWavesPerBlock + (threadIdx.x >> 6);
-    if (row >= M) return;
-    const uint8_t* wr = W + (size_t)row * N;
-    const int U = N / 16;
-    float acc[BMAX], sx[BMAX];
-#pragma unroll
-    for (int b = 0; b < BMAX; b++) { acc[b] = 0.f; sx[b] = 0.f; }
-    for (int u = lane; u < U; u += kWave) {
-        const uint4 wv = ld_stream16(wr + (size_t)u * 16);
-#pragma unroll
-        for (int b = 0; b < BMAX; b++) {
-            if (b < B) {
-                const float4* xp = (const float4*)(x + (size_t)b * N + (size_t)u * 16);
-                float xv[16];
-#pragma unroll
-                for (int t = 0; t < 4; t++) {
-                    const float4 v = xp[t];
-                    xv[4 * t] = v.x; xv[4 * t + 1] = v.y; xv[4 * t + 2] = v.z; xv[4 * t + 3] = v.w;
-                }
-                float s = 0.f;
-#pragma unroll
-                for (int c = 0; c < 16; c++) s += xv[c];
-                sx[b] += s;
-                acc[b] = unit_dot<8>(wv, xv, acc[b]);
-            }
-        }
-    }
-    const float scale = load_scale<KIND>(sc, row);
-#pragma unroll
-    for (int b = 0; b < BMAX; b++) {
-        if (b < B) {
-            const float v = wave_sum(fmaf(-128.f, sx[b], acc[b]));
-            if (lane == 0) y[(size_t)b * M_stride + row] = v * scale;
-        }
-    }
-}
-
-template <int KIND>
-void launch_int8_batch(float* out, const void* w, const void* sc, const float* x, int M, int N, int B,
-                       int M_stride, hipStream_t st) {
-    const int blocks = (M + kWavesPerBlock - 1) / kWavesPerBlock;
-    const uint8_t* W = (const uint8_t*)w;
-#define IBH_I8B(BM) int8_batch_fast<KIND, BM><<<blocks, kBlock, 0, st>>>(out, W, sc, x, M, N, B, M_stride)
-    if (B <= 1) IBH_I8B(1);
-    else if (B <= 2) IBH_I8B(2);
-    else if (B <= 4) IBH_I8B(4);
-    else if (B <= 8) IBH_I8B(8);
-    else if (B <= 16) IBH_I8B(16);
-    else IBH_I8B(32);
-#undef IBH_I8B
-}
-
 inline bool aligned16(const void* p) { return ((uintptr_t)p & 15) == 0; }
 
 }  // namespace
@@ -393,6 +333,8 @@ int ibh_launch_gemv_mfma(float* out, const void* w, const void* scales, int kind
                          int N, int bits, hipStream_t st);
 int ibh_launch_w4a8_mfma(float* out, const void* w, const void* sw, int kind, const int8_t* qx, const float* sa,
                          int M, int N, int B, int M_stride, bool fused, hipStream_t st);
+int ibh_launch_int8_skinny(float* out, const void* w, const void* sc, int kind, const float* x, int M, int N, int B,
+                           int M_stride, hipStream_t st);
 int ibh_launch_w4a8_batch(const MatDesc* d, int n, int kind, const int8_t* qx, const float* sa, int N, int B,
                           bool fused, hipStream_t st, int M_stride);
 
@@ -597,13 +539,9 @@ extern "C" int ibh_matmul_int8_batch(float* out, const void* w, const void* scal
         return IBH_ERROR_PARAM;
     }
     hipStream_t st = ibh_resolve_stream(stream);
-    if (N % 16 == 0 && aligned16(w) && aligned16(x)) {
-        if (scale_kind == IBH_SCALE_F16) launch_int8_batch<IBH_SCALE_F16>(out, w, scales, x, M, N, B, M_stride, st);
-        else launch_int8_batch<IBH_SCALE_F32>(out, w, scales, x, M, N, B, M_stride, st);
-        IBH_CHECK_LAUNCH("ibh_matmul_int8_batch");
-        return IBH_OK;
-    }
-    // Odd shapes: B independent matvecs into the strided output.
+    if (const int f = ibh_launch_int8_skinny(out, w, scales, scale_kind, x, M, N, B, M_stride, st))
+        return f < 0 ? IBH_ERROR_INTERNAL : IBH_OK;
+    // One column, or odd shapes: independent matvecs into the strided output.
     for (int b = 0; b < B; b++) {
         int rc = ibh_matmul(out + (size_t)b * M_stride, w, scales, scale_kind, x + (size_t)b * N, M, N, 8,
                             stream);

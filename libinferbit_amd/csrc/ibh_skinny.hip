@@ -289,6 +289,257 @@ __global__ __launch_bounds__(512) void w4a8_skinny(const BatchSet bs, const int8
     }
 }
 
+// ── INT8 rows x fp32 columns ────────────────────────────────────────────────
+// (kernels/scalar.c:70-84, within fp32 tolerance: sums in another order.)
+//
+// x becomes three int8 digit planes as in the one-column tile kernel, but per
+// (column, 128-column group): Q = rint(x * 4161400 / max|x|) in balanced
+// base-256 digits, so there is no second pass over x and an element keeps 23
+// bits of the group's largest.  Each group's exact int32 sums are combined,
+// scaled and added in fp32.  The 8 wavefronts of a block split K (their sums
+// meet in LDS, added in order).
+//
+// What bounds it is how its loads reach L1: neighbouring lanes in different
+// lines get one lane per clock.  With every lane loading its own 16 weights and
+// 16 floats of x in operand order (16 rows x 64 bytes an instruction), 4096 x
+// 4096 at 2 / 8 / 16 / 32 columns took 9.5 / 12.5 / 17.8 / 24.6 us.  So 8
+// neighbouring lanes load 128 contiguous bytes of a row of weights or of a
+// column, and both go through the wavefront's own LDS (no barrier; 16-byte
+// units swizzled to conflict-free) into the operands' order: x as digits, lane
+// 8 s + p holding columns 32 e + 4 p of slot s, 8 slots a pass, read back as
+// unit p = 4 m + q by lane (n, k quarter q) for MFMA m; the weights by the same
+// units of 16 columns, two lane swaps then giving them x's order of columns.
+// RT row tiles of a wavefront share its digits.
+// Measured in a graph, before (VALU, one wavefront per row) and here, at 2 / 8 /
+// 16 / 32 columns: 4096 x 4096 11.9 / 34.1 / 65 / 124 -> 8.6 / 9.1 / 11.4 / 16.6
+// us, 14336 x 4096 32.7 / 118 / 214 / 469 -> 21.8 / 23.1 / 28.9 / 38.5, 4096 x
+// 1024 5.0 / 12.2 / 21.5 / 40 -> 4.4 / 4.6 / 6.0 / 7.9.  Error against 64 bits
+// (relative to the outputs' norm): 4.5e-7 .. 6.7e-7 -> 4.2e-7 .. 4.8e-7.
+struct DigArgs {
+    const int8_t* W;
+    const void* sc;          // row scales
+    const float* x;          // [B][N]
+    float* y;
+    int M, N, B, ys, G, CPW; // G: 128-column groups of a row, CPW of them per wavefront
+};
+
+constexpr int kDigWaves = 8;
+// Q + 0x408080 in the low 23 bits of 2^23 + ..: bytes biased by 128, 128, 64
+constexpr float kDigMax = 4161400.f, kDigMagic = 8388608.f + 4227200.f;
+constexpr int kDigBytes = 3 * 1024;                            // digits of 8 slots x 128 columns
+
+// max that lets a NaN through (v_maximum3_f32)
+__device__ __forceinline__ float nmax(float a, float b) { return __builtin_elementwise_maximum(a, b); }
+
+template <int CTRL>
+__device__ __forceinline__ float dpp_nmax(float v) {
+    return nmax(v, __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), CTRL, 0xF, 0xF, false)));
+}
+
+// Lane (i, k quarter q) of unit 4 m' + q holds columns 64 m' + 16 q + 4 d .. + 3
+// in dword d: swapping dword and quarter gives lane q
+// dword j of unit half m' = columns 64 m' + 16 j + 4 q, which is element e = 2 m' +
+// (j >> 1) of unit p = 4 (j & 1) + q.
+__device__ __forceinline__ i4_t quarter_transpose(const uint4 w) {
+    typedef unsigned int u2_t __attribute__((ext_vector_type(2)));
+    const u2_t a = __builtin_amdgcn_permlane32_swap(w.x, w.z, false, false);
+    const u2_t b = __builtin_amdgcn_permlane32_swap(w.y, w.w, false, false);
+    const u2_t c = __builtin_amdgcn_permlane16_swap(a[0], b[0], false, false);
+    const u2_t d = __builtin_amdgcn_permlane16_swap(a[1], b[1], false, false);
+    return i4_t{(int)c[0], (int)c[1], (int)d[0], (int)d[1]};
+}
+
+// A row's sum over all columns in fp32, for a column that holds Inf or NaN:
+// both come out where they do without digits.
+__device__ __noinline__ float plain_dot(const int8_t* __restrict__ w, const float* __restrict__ x, int N) {
+    float y = 0.f;
+    for (int j = 0; j < N; j++) y = fmaf((float)w[j], x[j], y);
+    return y;
+}
+
+// SH: passes of 8 slots.
+template <int KIND, int RT, int SH>
+__global__ __launch_bounds__(64 * kDigWaves) void int8_skinny(const DigArgs a) {
+    constexpr int NT = (SH + 1) / 2;                           // column tiles
+    constexpr int RING = 4, XR = SH <= 2 ? 2 : 1;   // groups of weights and of x in flight
+    constexpr int WB = (SH * (kDigBytes + 32) + RT * 2048) / 4;   // a wavefront's LDS, in floats
+    static_assert(RT * NT * 256 <= WB, "the sums reuse the digits' LDS");
+    extern __shared__ __align__(16) unsigned char smem[];
+    const int N = a.N, B = a.B, M = a.M, G = a.G;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int kw = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int n = lane & 15, q = lane >> 4;
+    const int row0 = (int)blockIdx.x * 16 * RT;
+    const int g0 = kw * a.CPW, gn = max(0, min(a.CPW, G - g0));
+    float* mine = (float*)smem + (size_t)kw * WB;
+    uint4* ds = (uint4*)mine;                                  // [SH][3][64]
+    uint4* wl = ds + SH * 192;                                 // [RT][16 rows][8 units]
+    float* ss = (float*)(wl + RT * 128);                       // [SH][8] scales
+
+    float4 xr[XR][SH][4];
+    uint4 wr[RING][RT][2];
+    // columns past a row's end re-read its last 16 (same group): they leave the
+    // group's max as it is and meet zeroed weights
+    auto xload = [&](int u, int g) {
+        const int gc = min(g, G - 1);
+#pragma unroll
+        for (int h = 0; h < SH; h++) {
+            const uint32_t o = (uint32_t)min(8 * h + (lane >> 3), B - 1) * (uint32_t)N;
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                const int c = 128 * gc + 32 * e + 4 * (lane & 7);
+                xr[u][h][e] = *(const float4*)((const char*)a.x + 4 * (o + (uint32_t)(c < N ? c : N - 16 + (c & 15))));
+            }
+        }
+    };
+    const int8_t* wb = a.W + (size_t)row0 * N;
+    auto wload = [&](int u, int g) {
+        const int gc = min(g, G - 1);
+#pragma unroll
+        for (int t = 0; t < RT; t++) {
+#pragma unroll
+            for (int m = 0; m < 2; m++) {
+                const uint32_t o = (uint32_t)(min(row0 + 16 * t + 8 * m + (lane >> 3), M - 1) - row0) * (uint32_t)N;
+                wr[u][t][m] = ld_stream16((const uint8_t*)wb + (o + (uint32_t)min(128 * gc + 16 * (lane & 7), N - 16)));
+            }
+        }
+    };
+#pragma unroll
+    for (int u = 0; u < XR; u++) xload(u, g0 + u);
+#pragma unroll
+    for (int u = 0; u < RING; u++) wload(u, g0 + u);
+    __builtin_amdgcn_sched_barrier(0);
+
+    float acc[RT][NT][4];
+#pragma unroll
+    for (int t = 0; t < RT; t++)
+#pragma unroll
+        for (int nt = 0; nt < NT; nt++)
+#pragma unroll
+            for (int r = 0; r < 4; r++) acc[t][nt][r] = 0.f;
+
+    for (int c0 = 0; c0 < gn; c0 += RING) {
+#pragma unroll
+        for (int u = 0; u < RING; u++) {
+            const int c = c0 + u, g = g0 + c;
+            if (c >= gn) break;                                // wave-uniform
+            // 1. digits of the group, 8 slots a pass, to LDS
+#pragma unroll
+            for (int h = 0; h < SH; h++) {
+                float v[16];
+                float mx = 1e-31f;
+#pragma unroll
+                for (int e = 0; e < 4; e++) {
+                    const float4 f = xr[u % XR][h][e];
+                    v[4 * e] = f.x; v[4 * e + 1] = f.y; v[4 * e + 2] = f.z; v[4 * e + 3] = f.w;
+                }
+#pragma unroll
+                for (int e = 0; e < 16; e += 2) mx = nmax(nmax(mx, fabsf(v[e])), fabsf(v[e + 1]));
+                // the eight lanes of a slot share the scale, and with it that
+                // an element is not finite: the column's sums become NaN and
+                // are formed again in fp32 below.  The floor keeps 1 / mx
+                // finite (it rounds elements under 2e-38 in groups that hold
+                // nothing larger than 1e-31)
+                mx = dpp_nmax<0x141>(dpp_nmax<0x4E>(dpp_nmax<0xB1>(mx)));   // lane ^ 1, ^ 2, 7 - lane
+                const float inv = kDigMax / mx;
+                i4_t dg[3];
+#pragma unroll
+                for (int d = 0; d < 4; d++) {
+                    uint32_t b[4];
+#pragma unroll
+                    for (int e = 0; e < 4; e++)
+                        b[e] = __builtin_bit_cast(uint32_t, fmaf(v[4 * d + e], inv, kDigMagic));
+                    const uint32_t p01 = __builtin_amdgcn_perm(b[1], b[0], 0x05010400u);
+                    const uint32_t p23 = __builtin_amdgcn_perm(b[3], b[2], 0x05010400u);
+                    const uint32_t h01 = __builtin_amdgcn_perm(b[1], b[0], 0x0c0c0602u);
+                    const uint32_t h23 = __builtin_amdgcn_perm(b[3], b[2], 0x06020c0cu);
+                    dg[0][d] = (int)(__builtin_amdgcn_perm(p23, p01, 0x05040100u) ^ 0x80808080u);
+                    dg[1][d] = (int)(__builtin_amdgcn_perm(p23, p01, 0x07060302u) ^ 0x80808080u);
+                    dg[2][d] = (int)(((h01 | h23) << 1) ^ 0x80808080u);
+                }
+                const int s = lane >> 3, at = s * 8 + ((lane & 7) ^ s ^ (h & 1));
+#pragma unroll
+                for (int p = 0; p < 3; p++) *(i4_t*)(ds + (h * 3 + p) * 64 + at) = dg[p];
+                if ((lane & 7) == 0) ss[8 * h + s] = mx < __builtin_inff() ? mx * (1.0f / kDigMax) : __builtin_nanf("");
+            }
+            xload(u % XR, g + XR);
+#pragma unroll
+            for (int t = 0; t < RT; t++)
+#pragma unroll
+                for (int m = 0; m < 2; m++)
+                    wl[t * 128 + 64 * m + (lane & 56) + ((lane & 7) ^ (lane >> 3) ^ m)] = wr[u][t][m];
+            wload(u, g + RING);
+            // the wavefront's LDS operations run in order: the reads below see
+            // the writes above, the next group's writes come after these reads
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            i4_t av[RT][2];
+#pragma unroll
+            for (int t = 0; t < RT; t++) {
+#pragma unroll
+                for (int m = 0; m < 2; m++) {
+                    const i4_t T = quarter_transpose(wl[t * 128 + 8 * n + ((4 * m + q) ^ (n & 7) ^ (n >> 3))]);
+                    av[t][0][2 * m] = T[0]; av[t][1][2 * m] = T[1];
+                    av[t][0][2 * m + 1] = T[2]; av[t][1][2 * m + 1] = T[3];
+                }
+                if (128 * (g + 1) > N)                         // av[m][e]: columns 32 e + 16 m + 4 q
+#pragma unroll
+                    for (int e = 0; e < 8; e++)
+                        if (128 * g + 16 * e >= N) av[t][e & 1][e >> 1] = 0;
+            }
+            // 2. contraction and fold
+#pragma unroll
+            for (int nt = 0; nt < NT; nt++) {
+                // a last tile of 8 slots has them in both halves of its columns
+                const int h = 2 * nt + 1 < SH ? 2 * nt + (n >> 3) : 2 * nt, s = n & 7;
+                const uint4* src = ds + h * 192 + s * 8;
+                const int sw = s ^ (h & 1);
+                i4_t d[RT][3];
+#pragma unroll
+                for (int m = 0; m < 2; m++)
+#pragma unroll
+                    for (int p = 0; p < 3; p++) {
+                        const i4_t b = *(const i4_t*)(src + p * 64 + ((4 * m + q) ^ sw));
+#pragma unroll
+                        for (int t = 0; t < RT; t++)
+                            d[t][p] = __builtin_amdgcn_mfma_i32_16x16x64_i8(av[t][m], b, m ? d[t][p] : i4_t{0, 0, 0, 0}, 0, 0, 0);
+                    }
+                const float sc = ss[8 * h + s];
+#pragma unroll
+                for (int t = 0; t < RT; t++)
+#pragma unroll
+                    for (int r = 0; r < 4; r++) {
+                        // |d| <= 2^21: the low two planes join exactly in int32
+                        const float lo = (float)(d[t][0][r] + (d[t][1][r] << 8));
+                        acc[t][nt][r] = fmaf(fmaf((float)d[t][2][r], 32768.f, lo), sc, acc[t][nt][r]);
+                    }
+            }
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+        }
+    }
+
+    // 3. the wavefronts' sums, in order; thread -> (row fastest, column)
+#pragma unroll
+    for (int t = 0; t < RT; t++)
+#pragma unroll
+        for (int nt = 0; nt < NT; nt++)
+#pragma unroll
+            for (int r = 0; r < 4; r++) mine[(t * NT + nt) * 256 + r * 64 + lane] = acc[t][nt][r];
+    __syncthreads();
+    for (int e = tid; e < RT * NT * 256; e += 64 * kDigWaves) {
+        const int rr = e & 15, col = (e >> 4) & 15, tile = e >> 8, t = tile / NT, nt = tile - t * NT;
+        const int row = row0 + 16 * t + rr, s = 16 * nt + col;
+        if (row >= M || s >= B) continue;
+        const float* p = (const float*)smem + tile * 256 + (rr & 3) * 64 + (rr >> 2) * 16 + col;
+        float y = 0.f;
+#pragma unroll
+        for (int k = 0; k < kDigWaves; k++) y += p[(size_t)k * WB];
+        if (!(fabsf(y) <= 3.4e38f)) y = plain_dot(a.W + (size_t)row * N, a.x + (size_t)s * N, N);
+        a.y[(size_t)s * a.ys + row] = y * load_scale<KIND>(a.sc, row);
+    }
+}
+
 constexpr size_t kLds = 160 * 1024;
 
 bool lds_ok(const void* fn, size_t bytes) {
@@ -355,4 +606,30 @@ int ibh_launch_w4a8_batch(const MatDesc* d, int n, int kind, const int8_t* qx, c
 #undef IBH_SK
     IBH_CHECK_LAUNCH("w4a8 batch");
     return 1;
+}
+
+// INT8 rows x B fp32 columns (2 <= B <= 32).  Returns 1 if launched, 0 if the
+// shape is not taken, < 0 on a launch error.
+int ibh_launch_int8_skinny(float* out, const void* w, const void* sc, int kind, const float* x, int M, int N, int B,
+                           int M_stride, hipStream_t st) {
+    if (B < 2 || B > 32 || N % 16 || N < 16 || (((uintptr_t)w | (uintptr_t)x) & 15)) return 0;
+    const int G = (N + 127) / 128, T = (M + 15) / 16;
+    const DigArgs a{(const int8_t*)w, sc, x, out, M, N, B, M_stride, G, (G + kDigWaves - 1) / kDigWaves};
+    // two row tiles share the digits where that still leaves a block per CU
+    const int sh = (B + 7) / 8, rt = T > 256 ? 2 : 1;
+    const int blocks = (T + rt - 1) / rt;
+    const size_t lds = (size_t)kDigWaves * (sh * (kDigBytes + 32) + rt * 2048);
+#define IBH_I8L(K_, R_, H_) do { \
+        if (!lds_ok((const void*)int8_skinny<K_, R_, H_>, lds)) return 0; \
+        int8_skinny<K_, R_, H_><<<blocks, 64 * kDigWaves, lds, st>>>(a); } while (0)
+#define IBH_I8R(K_, H_) do { if (rt == 2) IBH_I8L(K_, 2, H_); else IBH_I8L(K_, 1, H_); } while (0)
+#define IBH_I8S(K_) do { if (sh == 1) IBH_I8R(K_, 1); else if (sh == 2) IBH_I8R(K_, 2); \
+                         else if (sh == 3) IBH_I8R(K_, 3); else IBH_I8R(K_, 4); } while (0)
+    if (kind == IBH_SCALE_F16) IBH_I8S(IBH_SCALE_F16); else IBH_I8S(IBH_SCALE_F32);
+#undef IBH_I8S
+#undef IBH_I8R
+#undef IBH_I8L
+    if (hipGetLastError() == hipSuccess) return 1;
+    ibh_set_error("int8 batch: launch failed");
+    return -1;
 }

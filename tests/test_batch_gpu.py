@@ -143,3 +143,46 @@ def test_w4a8_batch_columns_bit_exact(oracle_lib, M, N, B):
     for b in range(B):
         np.testing.assert_array_equal(got[b * ms + rows].view(np.uint32), want[b].view(np.uint32))
         assert (got[b * ms + M:(b + 1) * ms] == 7.0).all()
+
+
+# M, N, B, M_stride: part-filled row tiles and column tiles, one and two row
+# tiles per wavefront, rows that end inside a 128-column group or are shorter
+# than the wavefronts' split, both column-tile forms
+@pytest.mark.parametrize("M,N,B,ms", [(1, 16, 2, 1), (17, 144, 3, 20), (4100, 1040, 16, 4100), (4113, 4080, 9, 4113),
+                                      (100, 8192, 17, 100), (4112, 656, 32, 4120)])
+def test_int8_batch_digits(M, N, B, ms):
+    """Fast INT8 batch against float64.  An element keeps max|group| * 2^-22.9
+    of error (half a digit unit of max / 4161400), the group factor 2^-23, each
+    of the fp32 sums (N / 128 / 8 in a wavefront, 8 over them) 2^-24 of its
+    partial: bounded by 2^-24 * (N / 1024 + 13) of sum |w| * max|group|."""
+    import torch
+    import libinferbit_amd as L
+    L.ops.init(0)
+    print(f"case int8 digits M={M} N={N} B={B}", flush=True)
+    r = np.random.default_rng(M + N + B)
+    w = r.integers(-127, 128, (M, N), dtype=np.int8)
+    s = (r.random(M) * 0.01 + 1e-4).astype(np.float32)
+    x = r.standard_normal((B, N)).astype(np.float32)
+    x[0] *= np.float32(2.0) ** r.integers(-40, 30, N).astype(np.float32)
+    x[1] = 0
+    out = torch.full(((B - 1) * ms + M,), 7.0, device="cuda")
+    g = lambda a: torch.from_numpy(a).cuda()
+    L.ops.matmul_int8_batch(out, g(w), g(s), g(x), M, N, B, ms)
+    got = out.cpu().numpy()
+    pad = -N % 128
+    gm = np.abs(np.pad(x, ((0, 0), (0, pad)))).reshape(B, -1, 128).max(2).repeat(128, 1)[:, :N].astype(np.float64)
+    for b in range(B):
+        y = got[b * ms:b * ms + M].astype(np.float64)
+        want = (w.astype(np.float64) @ x[b].astype(np.float64)) * s
+        bound = 2.0 ** -24 * (N / 1024 + 13) * (np.abs(w.astype(np.float64)) @ gm[b]) * s
+        assert (np.abs(y - want) <= bound).all()
+        assert (got[b * ms + M:(b + 1) * ms] == 7.0).all()
+    # Inf and NaN stay in their own column and come out as in an fp32 sum
+    x[0, N // 2], x[B - 1, N - 1] = np.inf, np.nan
+    clean = got.copy()
+    L.ops.matmul_int8_batch(out, g(w), g(s), g(x), M, N, B, ms)
+    got = out.cpu().numpy()
+    y, wm = got[:M], w[:, N // 2]
+    assert (y[wm > 0] == np.inf).all() and (y[wm < 0] == -np.inf).all() and np.isnan(y[wm == 0]).all()
+    assert np.isnan(got[(B - 1) * ms:]).all()
+    np.testing.assert_array_equal(got[ms:(B - 1) * ms], clean[ms:(B - 1) * ms])
