@@ -22,9 +22,14 @@ typedef int i4_t __attribute__((ext_vector_type(4)));
 // order, times the row scale: bit-exact.
 //
 // The phases add up rather than overlap, since every wavefront's loads are in
-// flight at once (14336 x 4096, 16 columns, 13.0 us: 7.1 the weight loads
-// alone, 1.4 the columns, 1.5 the contraction, 1.4 the fold, 1.6 that a load
-// touches 16 rows x 64 bytes and not 4 x 256), so each is kept short.
+// flight at once, so each is kept short.
+//  - Loads: neighbouring lanes in different lines get one lane per clock from
+//    L1, so weights and codes come as 128 contiguous bytes per 8 lanes and are
+//    turned into operand order afterwards, the weights (8 rows x 128 bytes a
+//    load, two groups a pair of loads) between lanes, the codes on their way
+//    to LDS.  Loading both in operand order (16 rows x 64 bytes) took 13.1 us
+//    instead of 11.7 at 14336 x 4096 with 16 columns, 10.0 instead of 7.9 at
+//    4096 x 4096 with 32.
 //  - Columns: their codes are loaded ahead of the weights (loads return in
 //    order), permuted to the nibble order of the weight operand and, XLDS,
 //    staged in LDS in operand order for all row tiles of the block: a lane
@@ -35,9 +40,35 @@ typedef int i4_t __attribute__((ext_vector_type(4)));
 //    weights arrive; more of them (GATHER) put their sums in LDS over the codes
 //    and a thread per (column, row) folds, its reads independent.
 // Measured in a graph, before (4, 8 or 16 columns per pass, w4a8_mfma) and
-// here: 14336 x 4096 at 8 / 16 / 32 columns 13.7 / 17.5 / 35.4 -> 12.5 / 13.0 /
-// 17.2 us; 5632 x 2048 6.7 / 8.0 / 15.8 -> 5.8 / 6.2 / 8.2; 4096 x 4096 at 32
-// columns 13.5 -> 9.8, 2048 x 2048 at 16 / 32 5.3 / 10.3 -> 4.6 / 6.8.
+// here: 14336 x 4096 at 8 / 16 / 32 columns 13.7 / 17.5 / 35.4 -> 11.5 / 11.7 /
+// 14.6 us; 5632 x 2048 6.7 / 8.0 / 15.8 -> 5.7 / 5.9 / 7.3; 4096 x 4096 at 16 /
+// 32 columns 7.0 / 13.5 -> 6.0 / 7.9, 2048 x 2048 5.3 / 10.3 -> 4.6 / 6.0.
+
+// Two loads of 8 rows x 128 bytes, lane 8 r + u holding 16-byte unit u of row r
+// (a) or r + 8 (b): the lines of L1 are taken whole.  -> the operands of the two
+// 64-byte groups, lane (i, k quarter q) holding unit q of row i.  A lane and its
+// mirror in the 8 exchange the half that belongs to the other group, and one
+// lane permutation (p0, p1: turn_lanes) orders each group.
+__device__ __forceinline__ void turn_lanes(int lane, int& p0, int& p1) {
+    const int i = lane & 15, q = lane >> 4, b = i >> 3;
+    p0 = 4 * (8 * (i & 7) + (b ? 7 - q : q));
+    p1 = 4 * (8 * (i & 7) + (b ? 4 + q : 3 - q));
+}
+__device__ __forceinline__ void turn_pair(const uint4 a, const uint4 b, int p0, int p1, uint4& x0, uint4& x1) {
+    const uint32_t av[4] = {a.x, a.y, a.z, a.w}, bv[4] = {b.x, b.y, b.z, b.w};
+    uint32_t o0[4], o1[4];
+#pragma unroll
+    for (int e = 0; e < 4; e++) {
+        // row_half_mirror into lanes 4 .. 7 of each 8, or into lanes 0 .. 3
+        const int m0 = __builtin_amdgcn_update_dpp((int)av[e], (int)bv[e], 0x141, 0xF, 0xA, false);
+        const int m1 = __builtin_amdgcn_update_dpp((int)bv[e], (int)av[e], 0x141, 0xF, 0x5, false);
+        o0[e] = (uint32_t)__builtin_amdgcn_ds_bpermute(p0, m0);
+        o1[e] = (uint32_t)__builtin_amdgcn_ds_bpermute(p1, m1);
+    }
+    x0 = make_uint4(o0[0], o0[1], o0[2], o0[3]);
+    x1 = make_uint4(o1[0], o1[1], o1[2], o1[3]);
+}
+
 template <int KIND, bool FUSED, int NT, int MAXC, bool XLDS, bool GATHER>
 __global__ __launch_bounds__(512) void w4a8_skinny(const BatchSet bs, const int8_t* __restrict__ qx,
                                                    const float* __restrict__ sa, int N, int B, int G, int KW,
@@ -64,6 +95,23 @@ __global__ __launch_bounds__(512) void w4a8_skinny(const BatchSet bs, const int8
         a = *(const uint4*)p;
         b = *(const uint4*)(p + 16);
     };
+    // XLDS: unit lane & 7 of group g of slots (lane >> 3) (a) and + 8 (b), 128
+    // contiguous bytes per 8 lanes
+    auto codes8 = [&](int g, int nt, uint4& a, uint4& b) {
+        const int8_t* p = qx + min(128 * g + 16 * (lane & 7), N - 16);
+        a = *(const uint4*)(p + (size_t)min(16 * nt + (lane >> 3), B - 1) * N);
+        b = *(const uint4*)(p + (size_t)min(16 * nt + 8 + (lane >> 3), B - 1) * N);
+    };
+    // ... and where the contraction's lane (column, k quarter u >> 1) finds it
+    // as its half u & 1, conflict-free for both sides
+    auto stage = [&](int g, int nt, int s, const uint4& v) {
+        const int u = lane & 7;
+        const uint32_t on = 16 * nt + s < B && 128 * g + 16 * u < N ? 0xffffffffu : 0u;
+        xs[((size_t)g * NT + nt) * 128 + 64 * (u & 1) + 16 * (u >> 1) + (s ^ (2 * u))] =
+            make_uint4(__builtin_amdgcn_perm(v.y, v.x, 0x06040200u) & on, __builtin_amdgcn_perm(v.y, v.x, 0x07050301u) & on,
+                       __builtin_amdgcn_perm(v.w, v.z, 0x06040200u) & on, __builtin_amdgcn_perm(v.w, v.z, 0x07050301u) & on);
+    };
+    const int xl0 = 16 * q + (i ^ (4 * q)), xl1 = 64 + 16 * q + (i ^ (4 * q + 2));
     // codes in the order of the weight operand: even columns of each 8, then odd
     auto order = [&](int g, int nt, uint4& a, uint4& b) {
         const uint32_t on = 16 * nt + i < B && 128 * g + 32 * q < N ? 0xffffffffu : 0u;
@@ -85,8 +133,10 @@ __global__ __launch_bounds__(512) void w4a8_skinny(const BatchSet bs, const int8
 #pragma unroll
     for (int u = 0; u < XB; u++)
 #pragma unroll
-        for (int nt = 0; nt < NT; nt++)
-            codes(min(XLDS ? wave + nw * u : g0 + u, G - 1), nt, xa[u][nt], xb[u][nt]);
+        for (int nt = 0; nt < NT; nt++) {
+            if constexpr (XLDS) codes8(min(wave + nw * u, G - 1), nt, xa[u][nt], xb[u][nt]);
+            else codes(min(g0 + u, G - 1), nt, xa[u][nt], xb[u][nt]);
+        }
     const int nsc = G * 16 * NT;
     float sv[2];
 #pragma unroll
@@ -94,13 +144,14 @@ __global__ __launch_bounds__(512) void w4a8_skinny(const BatchSet bs, const int8
         const int e = min((int)threadIdx.x + u * (int)blockDim.x, nsc - 1);
         sv[u] = sa[(size_t)min(e % (16 * NT), B - 1) * G + e / (16 * NT)];
     }
-    // 2. every weight of the wavefront
-    const uint8_t* wrow = P.W + (size_t)min(row0 + i, P.M - 1) * rb;
+    // 2. every weight of the wavefront, two groups per pair of loads
     uint4 seg[MAXC];
 #pragma unroll
-    for (int c = 0; c < MAXC; c++) {
-        const size_t off = min((size_t)(g0 + min(c, max(gn - 1, 0))) * 64 + 16 * q, rb - 16);
-        seg[c] = ld_stream16(wrow + off);
+    for (int c = 0; c < MAXC; c += 2) {
+        const size_t off = min((size_t)(g0 + min(c, max(gn - 1, 0))) * 64 + 16 * (lane & 7), rb - 16);
+#pragma unroll
+        for (int h = 0; h < 2; h++)
+            seg[c + h] = ld_stream16(P.W + (size_t)min(row0 + 8 * h + (lane >> 3), P.M - 1) * rb + off);
     }
     float rsc[4];
     uint32_t rsb[4];
@@ -114,20 +165,18 @@ __global__ __launch_bounds__(512) void w4a8_skinny(const BatchSet bs, const int8
 #pragma unroll
             for (int nt = 0; nt < NT; nt++) {
                 const int g = wave + nw * u;
-                order(g, nt, xa[u][nt], xb[u][nt]);
                 if (g < G) {
-                    xs[((size_t)g * NT + nt) * 128 + lane] = xa[u][nt];
-                    xs[((size_t)g * NT + nt) * 128 + 64 + lane] = xb[u][nt];
+                    stage(g, nt, lane >> 3, xa[u][nt]);
+                    stage(g, nt, 8 + (lane >> 3), xb[u][nt]);
                 }
             }
         for (int g = wave + nw * XB; g < G; g += nw)
 #pragma unroll
             for (int nt = 0; nt < NT; nt++) {
                 uint4 a, b;
-                codes(g, nt, a, b);
-                order(g, nt, a, b);
-                xs[((size_t)g * NT + nt) * 128 + lane] = a;
-                xs[((size_t)g * NT + nt) * 128 + 64 + lane] = b;
+                codes8(g, nt, a, b);
+                stage(g, nt, lane >> 3, a);
+                stage(g, nt, 8 + (lane >> 3), b);
             }
     }
 #pragma unroll
@@ -141,6 +190,14 @@ __global__ __launch_bounds__(512) void w4a8_skinny(const BatchSet bs, const int8
 
     // 4. group sums: kept as floats (exact: below 2^18)
     float f[MAXC][NT][4];
+    int tp0, tp1;
+    turn_lanes(lane, tp0, tp1);
+    auto turn = [&](int c) {                                          // ahead of groups c and c + 1
+        uint4 x0, x1;
+        turn_pair(seg[c], seg[c + 1], tp0, tp1, x0, x1);
+        seg[c] = x0;
+        seg[c + 1] = x1;
+    };
     auto group = [&](int c, const uint4& x0, const uint4& x1, float (&o)[4]) {
         const uint32_t w[4] = {seg[c].x, seg[c].y, seg[c].z, seg[c].w};
         uint32_t av[8];
@@ -178,22 +235,26 @@ __global__ __launch_bounds__(512) void w4a8_skinny(const BatchSet bs, const int8
     if (XLDS && !GATHER && kw == 0) {
         // the first wavefront of a row folds as its groups arrive
 #pragma unroll
-        for (int c = 0; c < MAXC; c++)
+        for (int c = 0; c < MAXC; c++) {
+            if (c % 2 == 0) turn(c);
 #pragma unroll
             for (int nt = 0; nt < NT; nt++) {
-                const uint4* xg = xs + ((size_t)min(g0 + c, G - 1) * NT + nt) * 128 + lane;
+                const uint4* xg = xs + ((size_t)min(g0 + c, G - 1) * NT + nt) * 128;
                 float v[4];
-                group(c, xg[0], xg[64], v);
+                group(c, xg[xl0], xg[xl1], v);
                 fold(c, nt, v);
             }
+        }
     } else if constexpr (XLDS) {
 #pragma unroll
-        for (int c = 0; c < MAXC; c++)
+        for (int c = 0; c < MAXC; c++) {
+            if (c % 2 == 0) turn(c);
 #pragma unroll
             for (int nt = 0; nt < NT; nt++) {
-                const uint4* xg = xs + ((size_t)min(g0 + c, G - 1) * NT + nt) * 128 + lane;
-                group(c, xg[0], xg[64], f[c][nt]);
+                const uint4* xg = xs + ((size_t)min(g0 + c, G - 1) * NT + nt) * 128;
+                group(c, xg[xl0], xg[xl1], f[c][nt]);
             }
+        }
     } else {
 #pragma unroll
         for (int h = 0; h < 2; h++) {
@@ -209,6 +270,7 @@ __global__ __launch_bounds__(512) void w4a8_skinny(const BatchSet bs, const int8
                 for (int nt = 0; nt < NT; nt++) {
                     const int c = XB * h + u;
                     if (c >= MAXC) continue;
+                    if (c % 2 == 0 && nt == 0) turn(c);
                     order(min(g0 + c, G - 1), nt, xa[u][nt], xb[u][nt]);
                     group(c, xa[u][nt], xb[u][nt], f[c][nt]);
                 }
@@ -566,8 +628,10 @@ int ibh_launch_w4a8_batch(const MatDesc* d, int n, int kind, const int8_t* qx, c
     // on the running sum is handed on (2 wavefronts per row where 16 groups
     // each reach), one takes the gather with up to 8 wavefronts of 4 groups.
     // Fewer columns than these stay with the 4- to 16-column kernels, which
-    // stage nothing they do not need (measured crossings: tall matrices 5
-    // columns, short rows 9, others 17).
+    // stage nothing they do not need.  Both sides measured: at 4 and 6 columns
+    // 14336 x 4096 10.0 / 12.3 there and 11.5 / 11.5 here, 2048 x 2048 3.9 / 4.5
+    // and 4.4 / 4.4, 2048 x 5632 6.5 / 8.3 and 7.6 / 7.7; rows of 17 to 32 groups
+    // cross later, 4096 x 4096 at 8 / 12 columns 5.5 / 6.5 and 6.0 / 5.9.
     int rt = (T + 255) / 256;
     rt = rt > 4 ? 4 : rt;
     int KW = (G + 15) / 16 > 2 ? (G + 15) / 16 : 2;
@@ -575,7 +639,7 @@ int ibh_launch_w4a8_batch(const MatDesc* d, int n, int kind, const int8_t* qx, c
     if (rt < 1) return 0;
     const bool gather = rt == 1;
     if (gather) KW = (G + 3) / 4 < 8 ? (G + 3) / 4 : 8;
-    if (B <= (!gather ? 4 : G <= 16 ? 8 : 16)) return 0;
+    if (B <= (gather && G > 16 && G <= 32 ? 8 : 4)) return 0;
     const int CPW = (G + KW - 1) / KW;
     KW = (G + CPW - 1) / CPW;
     auto soff_of = [&](bool x) {
