@@ -21,6 +21,8 @@ int ibh_launch_rows_grp_multi(const IbhGrpMat* m, int n, const float* x, bool aw
 int ibh_launch_rows_grp(float* out, const uint8_t* q, const uint16_t* s, const float* x, bool awq, const float* xo,
                         const float* ia, const uint16_t* oi, const uint16_t* ov, int M, int N, int G, int K_out,
                         hipStream_t st);
+int ibh_launch_tile_grp_multi(const IbhGrpMat* m, int n, int mode, const float* x, const float* x2, int N, int G,
+                              const IbhGrpNorm* nrm, hipStream_t st, int B);
 void* ibh_workspace(size_t bytes);
 
 namespace {
@@ -216,7 +218,22 @@ extern "C" int ibh_int4g_matmul_batched(const ibh_int4g_tensor* t, int B, const 
     }
     if ((rc = int4g_ws_resolve(t, act_sparse_rel, &ws, ws_bytes, "ibh_int4g_matmul_batched"))) return rc;
     hipStream_t st = ibh_resolve_stream(stream);
-    for (int b = 0; b < B; b++)
+    // the quad-layout kernel takes the columns in one launch, each computed as
+    // a single call computes it
+    int b0 = 0;
+    if (!(act_sparse_rel > 0.f)) {
+        const IbhGrpMat m{t->q, t->s, t->inv_act, t->outl_idx, t->outl_val, out, t->M, t->K_out};
+        while (B - b0 > 1) {
+            const int nb = B - b0 < 1024 ? B - b0 : 1024;
+            IbhGrpMat c = m;
+            c.out = out + (size_t)b0 * t->M;
+            if (!ibh_launch_tile_grp_multi(&c, 1, t->inv_act ? 1 : 0, x + (size_t)b0 * t->N, nullptr, t->N, t->G, nullptr, st, nb))
+                break;
+            IBH_CHECK_LAUNCH("ibh_int4g_matmul_batched");
+            b0 += nb;
+        }
+    }
+    for (int b = b0; b < B; b++)
         if ((rc = int4g_one(t, x + (size_t)b * t->N, out + (size_t)b * t->M, act_sparse_rel, ws, st))) return rc;
     return IBH_OK;
 }

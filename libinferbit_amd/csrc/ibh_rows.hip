@@ -1087,7 +1087,7 @@ int ibh_launch_rows_x(float* out, const void* w, const void* scales, int kind, c
 // up: x is the MLP gate and xk = silu(x) * up (xo = x then; no AWQ).
 // Returns 1 if launched, 0 if not eligible (the caller runs its own path).
 int ibh_launch_tile_grp_multi(const IbhGrpMat* m, int n, int mode, const float* x, const float* x2, int N, int G,
-                              const IbhGrpNorm* nrm, hipStream_t st);
+                              const IbhGrpNorm* nrm, hipStream_t st, int B = 1);
 
 int ibh_launch_rows_grp_multi(const IbhGrpMat* m, int n, const float* x, bool awq, const float* xo, int N, int G,
                               hipStream_t st, const float* up, const IbhGrpNorm* nrm) {

@@ -119,3 +119,24 @@ def test_int4g_rejects_bad_tensors(ops):
     t = dict(q=rng.integers(0, 256, (4, 48), dtype=np.uint8), s=np.zeros((4, 5), np.uint16))    # 96 % 5 != 0
     with pytest.raises(IbhError):
         ops.Int4gDeviceTensor(t).matmul(x, out)
+
+
+# one launch for the columns: row blocks that are not whole rounds of 8, a row
+# block alone, ragged K-ranges, G = 256, outliers at and past the sidecar's limit
+@pytest.mark.parametrize("M,N,G,awq,K,B", [(1001, 4096, 128, 1, 3, 9), (3, 512 * 8, 128, 0, 0, 2), (333, 5632, 128, 1, 5, 4),
+                                           (100, 5632, 256, 1, 33, 3), (64, 14336, 128, 0, 32, 32), (2000, 2048, 128, 1, 8, 17)])
+def test_int4g_batched_columns_equal_single(ops, M, N, G, awq, K, B):
+    from gen_golden import make_int4g
+    print(f"case int4g batch {M}x{N} G={G} awq={awq} K={K} B={B}", flush=True)
+    rng = np.random.default_rng(M + N + B)
+    d = ops.Int4gDeviceTensor(make_int4g(rng, M, N, G, awq, K))
+    X = torch.from_numpy(rng.standard_normal((B, N)).astype(np.float32)).cuda()
+    X[1] *= 1e-3
+    Y = torch.full((B + 1, M), 7.0, device="cuda")
+    d.matmul_batched(X, Y[:B], 0.0)
+    for b in range(B):
+        y = torch.empty(M, device="cuda")
+        d.matmul(X[b].contiguous(), y, 0.0)
+        torch.cuda.synchronize()
+        np.testing.assert_array_equal(Y[b].cpu().numpy(), y.cpu().numpy())
+    assert (Y[B] == 7.0).all()
