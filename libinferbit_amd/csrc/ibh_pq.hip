@@ -465,8 +465,8 @@ __device__ __forceinline__ void table_tile(int K, const h8_t* cbs, const float* 
 }
 
 // A row's sum from the codebooks and x directly, no tables and no row words
-// (two-level calls with a non-finite x, sums past the fixed-point range, or a
-// workspace without the stamp, all of which the three-kernel path served): the
+// (two-level calls with a non-finite x or codeword, sums past the fixed-point
+// range, or a workspace without the stamp, all of which the three-kernel path served): the
 // entries in that path's order, so +-Inf and NaN come out where they do there.
 __device__ float plain_row(const PqDev& t, const float* __restrict__ x, int r, float gmax) {
     const int hf = t.G / 2;
@@ -585,7 +585,11 @@ __global__ __launch_bounds__(kFThreads) void pq_fused(PqDev t, const float* __re
     PQ_TT(0);
 
     // codebooks and the slab's x into LDS; the slab's max|x| and max|codeword|
+    // (fmaxf drops NaN, so what is not finite is flagged on its own: x below,
+    // and for two levels the codewords here, which the three-kernel path
+    // carries into the rows that use them)
     float mc = 0.f, ms = 0.f, mc2 = 0.f;
+    bool nonfin = false;
     if (tid < 2 * K) {
         h8_t h;
         if (cb16) h = __builtin_bit_cast(h8_t, cbv);
@@ -596,7 +600,10 @@ __global__ __launch_bounds__(kFThreads) void pq_fused(PqDev t, const float* __re
         }
         cbs[tid] = h;
 #pragma unroll
-        for (int i = 0; i < 8; i++) mc = fmaxf(mc, fabsf((float)h[i]));
+        for (int i = 0; i < 8; i++) {
+            mc = fmaxf(mc, fabsf((float)h[i]));
+            if (TWO) nonfin |= !(fabsf((float)h[i]) <= 65504.f);
+        }
     }
     if (TWO && tid < 2 * K2) {
         h8_t h;
@@ -609,7 +616,10 @@ __global__ __launch_bounds__(kFThreads) void pq_fused(PqDev t, const float* __re
         cbs[2 * K + tid] = h;
         float m2 = 0.f;
 #pragma unroll
-        for (int i = 0; i < 8; i++) m2 = fmaxf(m2, fabsf((float)h[i]));
+        for (int i = 0; i < 8; i++) {
+            m2 = fmaxf(m2, fabsf((float)h[i]));
+            nonfin |= !(fabsf((float)h[i]) <= 65504.f);
+        }
         mc2 = m2;
     }
     if (slab4) {
@@ -661,9 +671,7 @@ __global__ __launch_bounds__(kFThreads) void pq_fused(PqDev t, const float* __re
     }
     PQ_TT(1);
     // max|x| over the inner columns (the skipping rule's reference)
-    // (fmaxf drops NaN, so non-finite inputs are flagged on their own)
     float mx = 0.f;
-    bool nonfin = false;
     if (x4ok) {
 #pragma unroll
         for (int u = 0; u < 4; u++) {
@@ -687,7 +695,7 @@ __global__ __launch_bounds__(kFThreads) void pq_fused(PqDev t, const float* __re
     mx = wave_max_dpp(mx);
     __syncthreads();                                       // tables done; red[] read above
     if (lane == 0) red[wave] = mx;
-    const bool x_nonfinite = __syncthreads_or(nonfin) != 0;
+    const bool nonfinite = __syncthreads_or(nonfin) != 0;
     float gmax = 0.f;
 #pragma unroll
     for (int w = 0; w < kFThreads / 64; w++) gmax = fmaxf(gmax, red[w]);
@@ -706,7 +714,7 @@ __global__ __launch_bounds__(kFThreads) void pq_fused(PqDev t, const float* __re
     // <= 2^50; the same on every slab (cbmax, gmax and the flag are over the
     // whole tensor), so either every slab adds or none does
     const float bound = 2.0f * (float)ninner * cbmax * gmax;
-    const bool off = x_nonfinite || !(bound <= 3.4e38f) || (TWO && S > 1 && !wsok);
+    const bool off = nonfinite || !(bound <= 3.4e38f) || (TWO && S > 1 && !wsok);
     bool fin[NR];
     float sum[NR];
     uint16_t rs_bits[NR];

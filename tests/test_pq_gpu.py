@@ -389,3 +389,43 @@ def test_two_level_unprepared_workspace(ops):
     L._lib.check(L.lib().ibh_pq_matmul(ctypes.byref(d.s), x.data_ptr(), out.data_ptr(), ws.data_ptr(), ws.numel(),
                                        torch.cuda.current_stream().cuda_stream), "ibh_pq_matmul")
     assert relerr(out.cpu().numpy(), want.cpu().numpy()) <= 2e-6   # two orders of the same fp32 terms
+
+
+@pytest.mark.parametrize("book", ["cb1l", "cb1r", "cb2l", "cb2r"])
+@pytest.mark.parametrize("bad", [float("nan"), float("inf")])
+@pytest.mark.parametrize("M,C,K2", [(600, 70, 256), (520, 96, 16)])
+def test_two_level_nonfinite_codeword(ops, M, C, K2, book, bad):
+    """A NaN or Inf codeword reaches the rows that use it, and no others, as in
+    the three-kernel path; the workspace stays good for the next call."""
+    from gen_golden import make_pq
+    print(f"case two-level codeword {M}x{C} K2={K2} {book} {bad}", flush=True)
+    t = make_pq(np.random.default_rng(M + K2), M, C, 16, 256, 2, K2, 0)
+    if K2 == 16:
+        for i in ("i2l", "i2r"):                      # packed codes: every other row does without code 3
+            lo, hi = t[i][::2] & 15, t[i][::2] >> 4
+            t[i][::2] = np.where(lo == 3, 4, lo) | np.where(hi == 3, 4, hi) << 4
+    x = torch.randn(t["N"], generator=torch.Generator().manual_seed(C)).cuda()
+    good = ops.PqDeviceTensor(t)
+    cb = t[book].copy().view(np.float16).reshape(-1, 8)
+    cb[3, 5] = bad
+    d = ops.PqDeviceTensor({**t, book: cb.reshape(-1).view(np.uint16)})
+    d.ws = good.ws
+    out, want = torch.empty(M, device="cuda"), torch.empty(M, device="cuda")
+    good.matmul_streaming(x, want)
+    clean = want.clone()
+    try:
+        _fused(ops, 0)
+        d.matmul_streaming(x, want)
+    finally:
+        _fused(ops, 1)
+    for _ in range(2):
+        d.matmul_streaming(x, out)
+        g, w = out.cpu().numpy(), want.cpu().numpy()
+        assert 0 < np.isfinite(w).sum() < M
+        np.testing.assert_array_equal(np.isnan(g), np.isnan(w))
+        np.testing.assert_array_equal(g[np.isinf(w)], w[np.isinf(w)])
+        fin = np.isfinite(w)
+        # fp32 sums of 4 * 96 entries in two orders
+        assert np.abs(g - w)[fin].max() <= 2e-6 * np.abs(w[fin]).max()
+    good.matmul_streaming(x, out)
+    assert torch.equal(out, clean)
