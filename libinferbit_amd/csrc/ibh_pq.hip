@@ -52,6 +52,9 @@ struct PqDev {
     const int8_t* oside;
     const uint16_t* oscale;
     const int32_t* inner;    // inner (non-outlier) columns, null when n_outlier == 0
+    // what pq_fused may load 16 bytes at a time: the index rows (8 bytes of
+    // packed level-2 ones), the codebooks, x
+    int al_idx, al_cb, al_x;
 };
 
 __device__ __forceinline__ int inner_col(const PqDev& t, int j) { return t.inner ? t.inner[j] : j; }
@@ -400,6 +403,7 @@ constexpr int kFMaxRows = 131072;
 constexpr int kXS = 20;   // LDS floats per slab chunk: 8 per side (zero padded) + 4 (bank spread)
 __device__ unsigned long long pq_row_acc[kFMaxRows];   // ws == NULL calls: zero at load, each row's last slab clears it
 __device__ unsigned int ibh_pq_err;                    // IBH_DEVERR_* bits of this file's kernels
+__device__ uint4 pq_spare;                             // what a block without 16-byte index rows loads in their place
 constexpr unsigned long long kPqStamp = 0x49424850515753ull;   // "IBHPQWS"
 constexpr size_t kPqFront = 256 + (size_t)kFMaxRows * 8;       // stamp + row words at the front of a caller workspace
 
@@ -538,11 +542,11 @@ __global__ __launch_bounds__(kFThreads) void pq_fused(PqDev t, const float* __re
     // 1. loads: the slab's x, the codebooks, x for the max|x| scan, the index
     // bytes (in the order they are needed; loads complete in issue order)
     const int ninner = C * G;
-    const bool x4ok = !t.inner && (ninner & 3) == 0 && ninner <= 16 * kFThreads;
+    const bool x4ok = !t.inner && t.al_x && (ninner & 3) == 0 && ninner <= 16 * kFThreads;
     const bool slab4 = x4ok && G == 16;                    // the slab's x as float4s (c0 * 16 floats)
     float4 xsv = make_float4(0.f, 0.f, 0.f, 0.f);
     if (slab4) xsv = ((const float4*)x)[(size_t)c0 * 4 + min(tid, cn * 4 - 1)];
-    const bool cb16 = hf == 8;
+    const bool cb16 = hf == 8 && t.al_cb;
     uint4 cbv = make_uint4(0, 0, 0, 0);
     if (cb16) {
         const int ci = min(tid, 2 * K - 1);
@@ -561,25 +565,29 @@ __global__ __launch_bounds__(kFThreads) void pq_fused(PqDev t, const float* __re
 #pragma unroll
         for (int u = 0; u < 4; u++) xs4[u] = x4[min(u * kFThreads + tid, n4 - 1)];
     }
-    // the index bytes last, unconditionally (from a safe address when the
-    // slab is ragged; a load under a branch is waited for where it joins)
+    // the index bytes last, unconditionally (a load under a branch is waited
+    // for where it joins): a ragged slab's block, whose tensor may hold fewer
+    // than 16 of them, loads pq_spare and reads its bytes one by one below
     __builtin_amdgcn_sched_barrier(0);
-    const bool vec = cn == CS && (C & 15) == 0;
+    const bool vec = cn == CS && (C & 15) == 0 && t.al_idx;
+    const uint8_t* const spare = (const uint8_t*)&pq_spare;
+    const uint8_t *const b1l = vec ? t.i1l : spare, *const b1r = vec ? t.i1r : spare;
+    const uint8_t *const b2l = vec ? t.i2l : spare, *const b2r = vec ? t.i2r : spare;
     // level 2: 16 bytes a side, or 8 of packed 4-bit indices (C % 16 == 0: whole bytes)
     uint4 ivl[NR], ivr[NR], jvl[NR], jvr[NR];
 #pragma unroll
     for (int h = 0; h < NR; h++) {
         const size_t io = vec ? (size_t)min(r0 + h * kFRows, M - 1) * C + c0 + 16 * q : 0;
-        ivl[h] = *(const uint4*)(t.i1l + io);
-        ivr[h] = *(const uint4*)(t.i1r + io);
+        ivl[h] = *(const uint4*)(b1l + io);
+        ivr[h] = *(const uint4*)(b1r + io);
         jvl[h] = jvr[h] = make_uint4(0, 0, 0, 0);
         if constexpr (P4) {
-            const uint2 a = *(const uint2*)((vec ? t.i2l : t.i1l) + io / 2), b = *(const uint2*)((vec ? t.i2r : t.i1r) + io / 2);
+            const uint2 a = *(const uint2*)(b2l + io / 2), b = *(const uint2*)(b2r + io / 2);
             jvl[h] = make_uint4(a.x, a.y, 0, 0);
             jvr[h] = make_uint4(b.x, b.y, 0, 0);
         } else if constexpr (TWO) {
-            jvl[h] = *(const uint4*)((vec ? t.i2l : t.i1l) + io);
-            jvr[h] = *(const uint4*)((vec ? t.i2r : t.i1r) + io);
+            jvl[h] = *(const uint4*)(b2l + io);
+            jvr[h] = *(const uint4*)(b2r + io);
         }
     }
     PQ_TT(0);
@@ -1410,6 +1418,10 @@ static int pq_run(const ibh_pq_tensor_abi* t, const float* x, float* out, void* 
     const bool l2ok = !two || (!d.l2skip && d.l2_idx_bytes == 1 && d.K2 <= 256);
     if (l2ok && !md.q8 && !md.tq8 && t->G <= 16 && t->K <= 256 && S <= kFMaxS && t->M <= kFMaxRows && g_pq_fused) {
         const size_t flds = (size_t)kFCS * (2 * t->K + 4 + (two ? 2 * d.K2 + 4 : 0)) * sizeof(float);
+        const uintptr_t i2 = two ? (uintptr_t)d.i2l | (uintptr_t)d.i2r : 0;
+        d.al_idx = (((uintptr_t)d.i1l | (uintptr_t)d.i1r) & 15) == 0 && (i2 & (d.K2 == 16 ? 7 : 15)) == 0;
+        d.al_cb = (((uintptr_t)d.cb1l | (uintptr_t)d.cb1r | (two ? (uintptr_t)d.cb2l | (uintptr_t)d.cb2r : 0)) & 15) == 0;
+        d.al_x = ((uintptr_t)x & 15) == 0;
         unsigned long long* hdr = own_ws ? (unsigned long long*)ws : nullptr;
         unsigned long long* racc = own_ws ? hdr + 32 : nullptr;
         const bool ka = t->K % 32 == 0 && (!two || d.K2 % 32 == 0);

@@ -429,3 +429,31 @@ def test_two_level_nonfinite_codeword(ops, M, C, K2, book, bad):
         assert np.abs(g - w)[fin].max() <= 2e-6 * np.abs(w[fin]).max()
     good.matmul_streaming(x, out)
     assert torch.equal(out, clean)
+
+
+# fewer than 16 index bytes in all, and rows whose slabs hold 16-byte pieces
+@pytest.mark.parametrize("M,C,K2", [(1, 1, 0), (3, 5, 256), (7, 1, 16), (200, 64, 0), (200, 64, 256), (200, 64, 16)])
+def test_pq_operands_at_any_address(ops, oracle_lib, M, C, K2):
+    """Indices at odd addresses, codebooks at 2-byte and x at 4-byte ones: the
+    same rows as from aligned operands, and those the oracle's."""
+    from gen_golden import make_pq
+    print(f"case pq addresses {M}x{C} K2={K2}", flush=True)
+    t = make_pq(np.random.default_rng(M + C), M, C, 16, 256, 2 if K2 else 1, K2, 0)
+    x = np.random.default_rng(C).standard_normal(t["N"]).astype(np.float32)
+    d, e = ops.PqDeviceTensor(t), ops.PqDeviceTensor(t)
+    for k, f in ops.PqDeviceTensor._MAP.items():
+        if t.get(k) is None:
+            continue
+        raw = np.ascontiguousarray(t[k]).view(np.uint8).reshape(-1)
+        off = t[k].dtype.itemsize
+        b = torch.zeros(raw.size + off, dtype=torch.uint8, device="cuda")
+        b[off:] = torch.from_numpy(raw.copy()).cuda()
+        e.keep.append(b)
+        setattr(e.s, f, b.data_ptr() + off)
+    xb = torch.zeros(t["N"] + 1, device="cuda")
+    xb[1:] = torch.from_numpy(x).cuda()
+    a, b = torch.empty(M, device="cuda"), torch.empty(M, device="cuda")
+    d.matmul(torch.from_numpy(x).cuda(), a)
+    e.matmul(xb[1:], b)
+    assert torch.equal(a, b)
+    assert relerr(a.cpu().numpy(), oracle_lib.pq_matmul(t, x)) <= 1e-4
