@@ -52,9 +52,6 @@ struct PqDev {
     const int8_t* oside;
     const uint16_t* oscale;
     const int32_t* inner;    // inner (non-outlier) columns, null when n_outlier == 0
-    // what pq_fused may load 16 bytes at a time: the index rows (8 bytes of
-    // packed level-2 ones), the codebooks, x
-    int al_idx, al_cb, al_x;
 };
 
 __device__ __forceinline__ int inner_col(const PqDev& t, int j) { return t.inner ? t.inner[j] : j; }
@@ -416,6 +413,20 @@ __device__ unsigned long long ibh_pq_tt[4096][8];
 #define PQ_TT(i) ((void)0)
 #endif
 
+// 16 (8) bytes from any address in one load: indices lie where a file put
+// them, codebooks and x on multiples of their element
+typedef uint32_t u4a_t __attribute__((ext_vector_type(4), aligned(1)));
+typedef uint32_t u2a_t __attribute__((ext_vector_type(2), aligned(1)));
+typedef float f4a_t __attribute__((ext_vector_type(4), aligned(4)));
+__device__ __forceinline__ uint4 ld16(const void* p) {
+    const u4a_t v = *(const u4a_t*)p;
+    return make_uint4(v.x, v.y, v.z, v.w);
+}
+__device__ __forceinline__ float4 ld4f(const float* p) {
+    const f4a_t v = *(const f4a_t*)p;
+    return make_float4(v.x, v.y, v.z, v.w);
+}
+
 typedef _Float16 h8_t __attribute__((ext_vector_type(8)));
 typedef float f16x_t __attribute__((ext_vector_type(16)));
 
@@ -542,34 +553,33 @@ __global__ __launch_bounds__(kFThreads) void pq_fused(PqDev t, const float* __re
     // 1. loads: the slab's x, the codebooks, x for the max|x| scan, the index
     // bytes (in the order they are needed; loads complete in issue order)
     const int ninner = C * G;
-    const bool x4ok = !t.inner && t.al_x && (ninner & 3) == 0 && ninner <= 16 * kFThreads;
+    const bool x4ok = !t.inner && (ninner & 3) == 0 && ninner <= 16 * kFThreads;
     const bool slab4 = x4ok && G == 16;                    // the slab's x as float4s (c0 * 16 floats)
     float4 xsv = make_float4(0.f, 0.f, 0.f, 0.f);
-    if (slab4) xsv = ((const float4*)x)[(size_t)c0 * 4 + min(tid, cn * 4 - 1)];
-    const bool cb16 = hf == 8 && t.al_cb;
+    if (slab4) xsv = ld4f(x + 4 * ((size_t)c0 * 4 + min(tid, cn * 4 - 1)));
+    const bool cb16 = hf == 8;
     uint4 cbv = make_uint4(0, 0, 0, 0);
     if (cb16) {
         const int ci = min(tid, 2 * K - 1);
-        cbv = *(const uint4*)((ci < K ? t.cb1l : t.cb1r) + (size_t)(ci < K ? ci : ci - K) * 8);
+        cbv = ld16((ci < K ? t.cb1l : t.cb1r) + (size_t)(ci < K ? ci : ci - K) * 8);
     }
     uint4 cbv2 = make_uint4(0, 0, 0, 0);
     if (TWO && cb16) {
         const int ci = min(tid, 2 * K2 - 1);
-        cbv2 = *(const uint4*)((ci < K2 ? t.cb2l : t.cb2r) + (size_t)(ci < K2 ? ci : ci - K2) * 8);
+        cbv2 = ld16((ci < K2 ? t.cb2l : t.cb2r) + (size_t)(ci < K2 ? ci : ci - K2) * 8);
     }
     __builtin_amdgcn_sched_barrier(0);
     float4 xs4[4];
     if (x4ok) {
-        const float4* x4 = (const float4*)x;
         const int n4 = ninner >> 2;
 #pragma unroll
-        for (int u = 0; u < 4; u++) xs4[u] = x4[min(u * kFThreads + tid, n4 - 1)];
+        for (int u = 0; u < 4; u++) xs4[u] = ld4f(x + 4 * (size_t)min(u * kFThreads + tid, n4 - 1));
     }
     // the index bytes last, unconditionally (a load under a branch is waited
     // for where it joins): a ragged slab's block, whose tensor may hold fewer
     // than 16 of them, loads pq_spare and reads its bytes one by one below
     __builtin_amdgcn_sched_barrier(0);
-    const bool vec = cn == CS && (C & 15) == 0 && t.al_idx;
+    const bool vec = cn == CS && (C & 15) == 0;
     const uint8_t* const spare = (const uint8_t*)&pq_spare;
     const uint8_t *const b1l = vec ? t.i1l : spare, *const b1r = vec ? t.i1r : spare;
     const uint8_t *const b2l = vec ? t.i2l : spare, *const b2r = vec ? t.i2r : spare;
@@ -578,16 +588,16 @@ __global__ __launch_bounds__(kFThreads) void pq_fused(PqDev t, const float* __re
 #pragma unroll
     for (int h = 0; h < NR; h++) {
         const size_t io = vec ? (size_t)min(r0 + h * kFRows, M - 1) * C + c0 + 16 * q : 0;
-        ivl[h] = *(const uint4*)(b1l + io);
-        ivr[h] = *(const uint4*)(b1r + io);
+        ivl[h] = ld16(b1l + io);
+        ivr[h] = ld16(b1r + io);
         jvl[h] = jvr[h] = make_uint4(0, 0, 0, 0);
         if constexpr (P4) {
-            const uint2 a = *(const uint2*)(b2l + io / 2), b = *(const uint2*)(b2r + io / 2);
+            const u2a_t a = *(const u2a_t*)(b2l + io / 2), b = *(const u2a_t*)(b2r + io / 2);
             jvl[h] = make_uint4(a.x, a.y, 0, 0);
             jvr[h] = make_uint4(b.x, b.y, 0, 0);
         } else if constexpr (TWO) {
-            jvl[h] = *(const uint4*)(b2l + io);
-            jvr[h] = *(const uint4*)(b2r + io);
+            jvl[h] = ld16(b2l + io);
+            jvr[h] = ld16(b2r + io);
         }
     }
     PQ_TT(0);
@@ -1418,10 +1428,6 @@ static int pq_run(const ibh_pq_tensor_abi* t, const float* x, float* out, void* 
     const bool l2ok = !two || (!d.l2skip && d.l2_idx_bytes == 1 && d.K2 <= 256);
     if (l2ok && !md.q8 && !md.tq8 && t->G <= 16 && t->K <= 256 && S <= kFMaxS && t->M <= kFMaxRows && g_pq_fused) {
         const size_t flds = (size_t)kFCS * (2 * t->K + 4 + (two ? 2 * d.K2 + 4 : 0)) * sizeof(float);
-        const uintptr_t i2 = two ? (uintptr_t)d.i2l | (uintptr_t)d.i2r : 0;
-        d.al_idx = (((uintptr_t)d.i1l | (uintptr_t)d.i1r) & 15) == 0 && (i2 & (d.K2 == 16 ? 7 : 15)) == 0;
-        d.al_cb = (((uintptr_t)d.cb1l | (uintptr_t)d.cb1r | (two ? (uintptr_t)d.cb2l | (uintptr_t)d.cb2r : 0)) & 15) == 0;
-        d.al_x = ((uintptr_t)x & 15) == 0;
         unsigned long long* hdr = own_ws ? (unsigned long long*)ws : nullptr;
         unsigned long long* racc = own_ws ? hdr + 32 : nullptr;
         const bool ka = t->K % 32 == 0 && (!two || d.K2 % 32 == 0);
