@@ -239,16 +239,21 @@ typedef struct {
  * skipping rule, tables, gather and outlier sidecar; fp32 summation order
  * differs.  Returns 0 / negative like the reference (plus a message).
  * `ws` >= ibh_pq_workspace_bytes(t) bytes, NULL = library workspace.
- * Single-level work (one level, or level 1 only) with G <= 16 and K <= 256
- * runs in one launch whose blocks meet through one 64-bit word per row kept
- * at the front of the workspace (they return to zero at the end of every
- * call).  A caller workspace must be prepared ONCE, before its first use,
- * by ibh_pq_workspace_init; it then stays usable by every PQ call of any
- * tensor on that stream, but must not hold other data in between.  An
- * unprepared one gives NaN rows and IBH_DEVERR_PQ_WS (ibh_device_errors).
- * Calls that share a workspace must not overlap in time; different
- * workspaces are independent.  A non-finite x gives NaN rows on this path
- * (the CPU gives +-Inf or NaN). */
+ * One- and two-level work with G <= 16 and up to 256 codes a level (byte or
+ * packed level-2 indices; no L2SKIP, INT8 or q8lut) runs in one launch whose
+ * blocks meet through one 64-bit word per row kept at the front of the
+ * workspace (they return to zero at the end of every call).  A caller
+ * workspace must be prepared ONCE, before its first use, by
+ * ibh_pq_workspace_init; it then stays usable by every PQ call of any tensor
+ * on that stream, but must not hold other data in between.  On an unprepared
+ * one single-level work gives NaN rows and IBH_DEVERR_PQ_WS
+ * (ibh_device_errors); two-level work, which needs no words to be right, sums
+ * its rows from the codebooks instead, at a fraction of the speed, and raises
+ * nothing.  Calls that share a workspace must not overlap in time; different
+ * workspaces are independent.  A non-finite x gives NaN rows for single-level
+ * work (the CPU gives +-Inf or NaN); two-level work gives what the sums give,
+ * for codewords that are not finite too.  No alignment beyond that of the
+ * elements is required of the tensor's arrays or of x. */
 size_t ibh_pq_workspace_bytes(const ibh_pq_tensor* t);
 /* Stamps a caller PQ workspace and zeroes its row words (a kernel on
  * `stream`, so it may sit in a captured graph).  ws 256-byte aligned,

@@ -52,6 +52,7 @@ struct PqDev {
     const int8_t* oside;
     const uint16_t* oscale;
     const int32_t* inner;    // inner (non-outlier) columns, null when n_outlier == 0
+    int slab_sh;             // log2 of the three-kernel path's chunks per slab (two levels: 8 or 16)
 };
 
 __device__ __forceinline__ int inner_col(const PqDev& t, int j) { return t.inner ? t.inner[j] : j; }
@@ -387,7 +388,7 @@ __global__ __launch_bounds__(kThreads) void pq_reduce(PqDev t, const float* __re
 //     A non-finite x (or a bound that overflows) would make the fixed-point
 //     terms meaningless: every slab then writes NaN to its rows (the CPU
 //     gives +-Inf or NaN there); two-level calls, which had the three-kernel
-//     path's fp32 sums there, take them from plain_row.
+//     path's fp32 sums there, take them from direct_rows.
 //  Two levels double the tables, the lookups and the index bytes and keep the
 //  rest: 4096 x 14336, 256 + 256 codes, streaming: 75.3 us in three launches
 //  (68 of them the gather, 16 chunks' tables re-read by every block of 512
@@ -479,30 +480,108 @@ __device__ __forceinline__ void table_tile(int K, const h8_t* cbs, const float* 
     }
 }
 
-// A row's sum from the codebooks and x directly, no tables and no row words
-// (two-level calls with a non-finite x or codeword, sums past the fixed-point
-// range, or a workspace without the stamp, all of which the three-kernel path served): the
-// entries in that path's order, so +-Inf and NaN come out where they do there.
-__device__ float plain_row(const PqDev& t, const float* __restrict__ x, int r, float gmax) {
-    const int hf = t.G / 2;
+// Rows' sums from the codebooks and x directly, no tables and no row words:
+// two-level calls with a non-finite x or codeword, sums past the fixed-point
+// range, or a workspace without the stamp, all of which the three-kernel path
+// served.  The sums are that path's bit for bit: a lane sums the entries of
+// one of its slabs of 8 or 16 chunks, the slabs are added in order.  Rows
+// [lo, hi) of the block's tiles, two per group of lanes, into sums[row - tile
+// start].  Bound by the LDS reads of codewords at random (four of 16 bytes per
+// row and chunk) and of x, staged once with the slabs 4 floats apart so that
+// the lanes' reads spread over the banks.  A workspace without the stamp, 4096
+// x 14336, 256 + 256 codes: 53 us; 1024 x 3216 with 16 outliers, 256 + 64
+// codes: 42 us (the three kernels 79 and 45, a thread per row 10072 and 2299).
+constexpr int kDPad = 4;
+
+template <bool P4>
+__device__ __forceinline__ void direct_rows(const PqDev& t, const float* __restrict__ x, const h8_t* cbs, float* xd,
+                                            float* sums, int base, int lo, int hi, float gmax, int tid) {
+    const int hf = t.G / 2, C = t.C, K = t.K, K2 = t.K2, lane = tid & 63, wave = tid >> 6;
+    const int CS = 1 << t.slab_sh, dxs = 16 * CS + kDPad;
     const size_t l2s = l2_stride(t);
-    float acc = 0.f;
-    for (int c = 0; c < t.C; c++) {
-        float xv[16], cm = 0.f;
-        for (int i = 0; i < t.G; i++) {
-            xv[i] = x[inner_col(t, c * t.G + i)];
-            cm = fmaxf(cm, fabsf(xv[i]));
-        }
-        const bool keep = t.skip_mode == 1 ? (gmax > 0.f ? cm >= gmax * t.skip_val : true)
-                        : t.skip_mode == 2 ? (t.skip_val > 0.f ? cm > t.skip_val : true) : true;
-        if (!keep) continue;
-        const size_t io = (size_t)r * t.C + c;
-        acc = acc + (table_entry(t.cb1l + (size_t)t.i1l[io] * hf, xv, hf) +
-                     table_entry(t.cb1r + (size_t)t.i1r[io] * hf, xv + hf, hf));
-        acc = acc + (table_entry(t.cb2l + (size_t)l2_at(t, t.i2l + (size_t)r * l2s, c) * hf, xv, hf) +
-                     table_entry(t.cb2r + (size_t)l2_at(t, t.i2r + (size_t)r * l2s, c) * hf, xv + hf, hf));
+    for (int i = tid; i < C * 16; i += kFThreads) {
+        const int c = i >> 4, sd = (i >> 3) & 1, e = i & 7;
+        xd[(c >> t.slab_sh) * dxs + (i & (16 * CS - 1))] = e < hf ? x[inner_col(t, c * t.G + sd * hf + e)] : 0.f;
     }
-    return acc;
+    __syncthreads();
+    // sum_i cb[i] * x[i] in table_entry's order, over the hf values that exist
+    auto entry = [&](const h8_t cb, const float* xv) {
+        float s = 0.f;
+#pragma unroll
+        for (int i = 0; i < 8; i++) {
+            if (i >= hf) break;
+            const float c = (float)cb[i];
+            s = i < (hf & ~3) ? s + c * xv[i] : fmaf(c, xv[i], s);
+        }
+        return s;
+    };
+    const int ns = (C + CS - 1) >> t.slab_sh;
+    // lanes per row: the power of two that holds the slabs, up to 64
+    int lsh = 0;
+    while (lsh < 6 && (1 << lsh) < ns) lsh++;
+    const int sub = lane & ((1 << lsh) - 1), first = lane - sub, nrow = 2 << (6 - lsh);
+    for (int r0 = lo + nrow * wave; r0 < hi; r0 += nrow * (kFThreads / 64)) {
+        const int r = r0 + 2 * (lane >> lsh);
+        const uint8_t* ip[2][4];
+        float tot[2] = {0.f, 0.f};
+#pragma unroll
+        for (int u = 0; u < 2; u++) {
+            const size_t rr = (size_t)min(base + min(r + u, hi - 1), t.M - 1);
+            ip[u][0] = t.i1l + rr * C;
+            ip[u][1] = t.i1r + rr * C;
+            ip[u][2] = t.i2l + rr * l2s;
+            ip[u][3] = t.i2r + rr * l2s;
+        }
+        for (int s0 = 0; s0 < ns; s0 += 64) {
+            const int sl = min(s0 + sub, ns - 1);             // lanes past the last slab are not added
+            float acc[2] = {0.f, 0.f};
+            int k[2][4];
+            auto load = [&](int j) {                          // the chunk's codes
+                const int c = min(CS * sl + j, C - 1);
+#pragma unroll
+                for (int u = 0; u < 2; u++)
+#pragma unroll
+                    for (int i = 0; i < 4; i++)
+                        k[u][i] = P4 && i > 1 ? (ip[u][i][c >> 1] >> (4 * (c & 1))) & 15 : ip[u][i][c];
+            };
+            load(0);
+            for (int j = 0; j < CS; j++) {
+                h8_t cw[2][4];
+#pragma unroll
+                for (int u = 0; u < 2; u++) {
+                    cw[u][0] = cbs[k[u][0]];
+                    cw[u][1] = cbs[K + k[u][1]];
+                    cw[u][2] = cbs[2 * K + k[u][2]];
+                    cw[u][3] = cbs[2 * K + K2 + k[u][3]];
+                }
+                load(min(j + 1, CS - 1));                     // in flight during the sums
+                float xv[16], cm = 0.f;
+#pragma unroll
+                for (int v = 0; v < 4; v++) {
+                    const float4 f = *(const float4*)(xd + sl * dxs + 16 * j + 4 * v);
+                    xv[4 * v] = f.x; xv[4 * v + 1] = f.y; xv[4 * v + 2] = f.z; xv[4 * v + 3] = f.w;
+                }
+#pragma unroll
+                for (int v = 0; v < 16; v++) cm = fmaxf(cm, fabsf(xv[v]));
+                const bool keep = t.skip_mode == 1 ? (gmax > 0.f ? cm >= gmax * t.skip_val : true)
+                                : t.skip_mode == 2 ? (t.skip_val > 0.f ? cm > t.skip_val : true) : true;
+                if (!keep || CS * sl + j >= C) continue;
+#pragma unroll
+                for (int u = 0; u < 2; u++) {
+                    acc[u] = acc[u] + (entry(cw[u][0], xv) + entry(cw[u][1], xv + 8));
+                    acc[u] = acc[u] + (entry(cw[u][2], xv) + entry(cw[u][3], xv + 8));
+                }
+            }
+            const int n = min(64, ns - s0);
+#pragma unroll
+            for (int u = 0; u < 2; u++)
+                for (int l = 0; l < n; l++) tot[u] = tot[u] + __shfl(acc[u], first + l, 64);
+        }
+#pragma unroll
+        for (int u = 0; u < 2; u++)
+            if (sub == 0 && r + u < hi) sums[r + u] = tot[u];
+    }
+    __syncthreads();
 }
 
 // KA: every codebook a multiple of 32 codes (every table row of a tile is
@@ -736,81 +815,93 @@ __global__ __launch_bounds__(kFThreads) void pq_fused(PqDev t, const float* __re
     bool fin[NR];
     float sum[NR];
     uint16_t rs_bits[NR];
+    if (TWO && off) {
+        // rows that the tables cannot serve: every slab's block takes its share
+        // of the tile's rows whole (the tables' LDS is free now)
+        const int per = (kFRows * NR + S - 1) / S, lo = min(sl * per, kFRows * NR), hi = min(lo + per, kFRows * NR);
+        float* const dsum = T + ((C >> t.slab_sh) + 1) * ((16 << t.slab_sh) + kDPad);
+        direct_rows<P4>(t, x, cbs, T, dsum, rt * (kFRows * NR), lo, hi, gmax, tid);
 #pragma unroll
-    for (int h = 0; h < NR; h++) {
-        const int r = r0 + h * kFRows;
-        // 4. gather: the thread's 16 chunks, L then R per chunk (entries carry 2^-ex)
-        float acc = 0.f;
-        if (vec) {
-            const uint32_t wl[4] = {ivl[h].x, ivl[h].y, ivl[h].z, ivl[h].w}, wr[4] = {ivr[h].x, ivr[h].y, ivr[h].z, ivr[h].w};
-            const uint32_t vl[4] = {jvl[h].x, jvl[h].y, jvl[h].z, jvl[h].w}, vr[4] = {jvr[h].x, jvr[h].y, jvr[h].z, jvr[h].w};
-            const float* Tq = T + (size_t)(16 * q) * TS;
-            const float* Tq2 = T2 + (size_t)(16 * q) * TS2;
-            auto term = [&](int j) {
-                const int il = (wl[j >> 2] >> (8 * (j & 3))) & 0xff, ir = (wr[j >> 2] >> (8 * (j & 3))) & 0xff;
-                float v = Tq[j * TS + il] + Tq[j * TS + K + ir];
-                if constexpr (TWO) {
-                    const int jl = P4 ? (vl[j >> 3] >> (4 * (j & 7))) & 0xf : (vl[j >> 2] >> (8 * (j & 3))) & 0xff;
-                    const int jr = P4 ? (vr[j >> 3] >> (4 * (j & 7))) & 0xf : (vr[j >> 2] >> (8 * (j & 3))) & 0xff;
-                    v = v + (Tq2[j * TS2 + jl] + Tq2[j * TS2 + K2 + jr]);
-                }
-                return v;
-            };
-            if (keepm == full) {
-#pragma unroll
-                for (int j = 0; j < 16; j++) acc = acc + term(j);
-            } else {
-#pragma unroll
-                for (int j = 0; j < 16; j++) {
-                    const float val = term(j);
-                    acc = acc + (((keepm >> (16 * q + j)) & 1) ? val : 0.f);
-                }
-            }
-        } else if (r < M) {
-            const uint8_t* pl = t.i1l + (size_t)r * C + c0;
-            const uint8_t* pr = t.i1r + (size_t)r * C + c0;
-            const size_t l2s = TWO ? l2_stride(t) : 0;
-            for (int c = 16 * q; c < min(16 * q + 16, cn); c++) {
-                const float* Tc = T + (size_t)c * TS;
-                float val = Tc[pl[c]] + Tc[K + pr[c]];
-                if constexpr (TWO) {
-                    const float* Tc2 = T2 + (size_t)c * TS2;
-                    val = val + (Tc2[l2_at(t, t.i2l + (size_t)r * l2s, c0 + c)] +
-                                 Tc2[K2 + l2_at(t, t.i2r + (size_t)r * l2s, c0 + c)]);
-                }
-                acc = acc + (((keepm >> c) & 1) ? val : 0.f);
-            }
+        for (int h = 0; h < NR; h++) {
+            const int r = r0 + h * kFRows, i = (tid >> 1) + h * kFRows;
+            fin[h] = q == 0 && r < M && i >= lo && i < hi;
+            sum[h] = dsum[i];
+            rs_bits[h] = t.row_scale[min(r, M - 1)];
         }
-        // the row's two partials, lanes 2i, 2i+1
-        acc += __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, acc), 0xB1, 0xF, 0xF, false));
-        PQ_TT(3);
+    } else {
+#pragma unroll
+        for (int h = 0; h < NR; h++) {
+            const int r = r0 + h * kFRows;
+            // 4. gather: the thread's 16 chunks, L then R per chunk (entries carry 2^-ex)
+            float acc = 0.f;
+            if (vec) {
+                const uint32_t wl[4] = {ivl[h].x, ivl[h].y, ivl[h].z, ivl[h].w}, wr[4] = {ivr[h].x, ivr[h].y, ivr[h].z, ivr[h].w};
+                const uint32_t vl[4] = {jvl[h].x, jvl[h].y, jvl[h].z, jvl[h].w}, vr[4] = {jvr[h].x, jvr[h].y, jvr[h].z, jvr[h].w};
+                const float* Tq = T + (size_t)(16 * q) * TS;
+                const float* Tq2 = T2 + (size_t)(16 * q) * TS2;
+                auto term = [&](int j) {
+                    const int il = (wl[j >> 2] >> (8 * (j & 3))) & 0xff, ir = (wr[j >> 2] >> (8 * (j & 3))) & 0xff;
+                    float v = Tq[j * TS + il] + Tq[j * TS + K + ir];
+                    if constexpr (TWO) {
+                        const int jl = P4 ? (vl[j >> 3] >> (4 * (j & 7))) & 0xf : (vl[j >> 2] >> (8 * (j & 3))) & 0xff;
+                        const int jr = P4 ? (vr[j >> 3] >> (4 * (j & 7))) & 0xf : (vr[j >> 2] >> (8 * (j & 3))) & 0xff;
+                        v = v + (Tq2[j * TS2 + jl] + Tq2[j * TS2 + K2 + jr]);
+                    }
+                    return v;
+                };
+                if (keepm == full) {
+#pragma unroll
+                    for (int j = 0; j < 16; j++) acc = acc + term(j);
+                } else {
+#pragma unroll
+                    for (int j = 0; j < 16; j++) {
+                        const float val = term(j);
+                        acc = acc + (((keepm >> (16 * q + j)) & 1) ? val : 0.f);
+                    }
+                }
+            } else if (r < M) {
+                const uint8_t* pl = t.i1l + (size_t)r * C + c0;
+                const uint8_t* pr = t.i1r + (size_t)r * C + c0;
+                const size_t l2s = TWO ? l2_stride(t) : 0;
+                for (int c = 16 * q; c < min(16 * q + 16, cn); c++) {
+                    const float* Tc = T + (size_t)c * TS;
+                    float val = Tc[pl[c]] + Tc[K + pr[c]];
+                    if constexpr (TWO) {
+                        const float* Tc2 = T2 + (size_t)c * TS2;
+                        val = val + (Tc2[l2_at(t, t.i2l + (size_t)r * l2s, c0 + c)] +
+                                     Tc2[K2 + l2_at(t, t.i2r + (size_t)r * l2s, c0 + c)]);
+                    }
+                    acc = acc + (((keepm >> c) & 1) ? val : 0.f);
+                }
+            }
+            // the row's two partials, lanes 2i, 2i+1
+            acc += __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, acc), 0xB1, 0xF, 0xF, false));
+            PQ_TT(3);
 
-        // 5. the rows' words
-        const bool own = q == 0 && r < M;
-        fin[h] = own;
-        sum[h] = ldexpf(acc, ex);
-        rs_bits[h] = t.row_scale[min(r, M - 1)];   // in flight with the atomic below
-        if (TWO && off) {
-            fin[h] = own && sl == 0;
-            if (fin[h]) sum[h] = plain_row(t, x, r, gmax);
-        } else if (S > 1 && off) {
-            if (own) out[r] = __builtin_nanf("");
-            fin[h] = false;
-        }
-        if (S > 1 && own && !off) {
-            int eb = 0;
-            if (bound > 0.f) frexpf(bound, &eb);               // bound < 2^eb
-            const int qe = 50 - eb;
-            const long long v = llrint((double)acc * ldexp(1.0, qe + ex));
-            const unsigned long long add = (1ull << 58) + (unsigned long long)(v + (1ll << 50));
-            const unsigned long long old =
-                __hip_atomic_fetch_add(&words[r], add, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            const unsigned long long tot = old + add;
-            fin[h] = (tot >> 58) == (unsigned long long)S;
-            if (fin[h]) {
-                const long long val = (long long)(tot & ((1ull << 58) - 1)) - (long long)S * (1ll << 50);
-                sum[h] = (float)((double)val * ldexp(1.0, -qe));
-                __hip_atomic_store(&words[r], 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            // 5. the rows' words
+            const bool own = q == 0 && r < M;
+            fin[h] = own;
+            sum[h] = ldexpf(acc, ex);
+            rs_bits[h] = t.row_scale[min(r, M - 1)];   // in flight with the atomic below
+            if (S > 1 && off) {
+                if (own) out[r] = __builtin_nanf("");
+                fin[h] = false;
+            }
+            if (S > 1 && own && !off) {
+                int eb = 0;
+                if (bound > 0.f) frexpf(bound, &eb);               // bound < 2^eb
+                const int qe = 50 - eb;
+                const long long v = llrint((double)acc * ldexp(1.0, qe + ex));
+                const unsigned long long add = (1ull << 58) + (unsigned long long)(v + (1ll << 50));
+                const unsigned long long old =
+                    __hip_atomic_fetch_add(&words[r], add, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                const unsigned long long tot = old + add;
+                fin[h] = (tot >> 58) == (unsigned long long)S;
+                if (fin[h]) {
+                    const long long val = (long long)(tot & ((1ull << 58) - 1)) - (long long)S * (1ll << 50);
+                    sum[h] = (float)((double)val * ldexp(1.0, -qe));
+                    __hip_atomic_store(&words[r], 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                }
             }
         }
     }
@@ -1425,9 +1516,14 @@ static int pq_run(const ibh_pq_tensor_abi* t, const float* x, float* out, void* 
     // the level-2 skip and the int8 tables take the three-kernel path below
     int tiles = (t->M + kFRows - 1) / kFRows;
     const int S = (t->C + kFCS - 1) / kFCS;
-    const bool l2ok = !two || (!d.l2skip && d.l2_idx_bytes == 1 && d.K2 <= 256);
+    const bool l2ok = !two || (!d.l2skip && d.l2_idx_bytes == 1 && d.K2 <= 256 && (CS == 8 || CS == 16));
     if (l2ok && !md.q8 && !md.tq8 && t->G <= 16 && t->K <= 256 && S <= kFMaxS && t->M <= kFMaxRows && g_pq_fused) {
-        const size_t flds = (size_t)kFCS * (2 * t->K + 4 + (two ? 2 * d.K2 + 4 : 0)) * sizeof(float);
+        size_t flds = (size_t)kFCS * (2 * t->K + 4 + (two ? 2 * d.K2 + 4 : 0)) * sizeof(float);
+        // direct_rows' x and sums (a block of 1024 threads has a CU to itself,
+        // so more LDS costs no block its place)
+        d.slab_sh = CS == 8 ? 3 : 4;
+        const size_t dlds = ((size_t)(t->C / CS + 1) * (16 * CS + kDPad) + 2 * kFRows) * sizeof(float);
+        if (two && dlds > flds) flds = dlds;
         unsigned long long* hdr = own_ws ? (unsigned long long*)ws : nullptr;
         unsigned long long* racc = own_ws ? hdr + 32 : nullptr;
         const bool ka = t->K % 32 == 0 && (!two || d.K2 % 32 == 0);

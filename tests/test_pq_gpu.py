@@ -457,3 +457,39 @@ def test_pq_operands_at_any_address(ops, oracle_lib, M, C, K2):
     e.matmul(xb[1:], b)
     assert torch.equal(a, b)
     assert relerr(a.cpu().numpy(), oracle_lib.pq_matmul(t, x)) <= 1e-4
+
+
+@pytest.mark.parametrize("M,C,G,K,K2,no", TWO_LEVEL + [(40, 2016, 16, 256, 256, 0), (1100, 700, 8, 64, 16, 8)])
+def test_two_level_direct_rows(ops, M, C, G, K, K2, no):
+    """The sums that need neither tables nor row words (a workspace that was
+    not prepared, a non-finite x) are the three-kernel path's bit for bit."""
+    import ctypes
+
+    import libinferbit_amd as L
+    from gen_golden import make_pq
+    print(f"case two-level direct {M}x{C} G={G} K={K}/{K2} no={no}", flush=True)
+    t = make_pq(np.random.default_rng(M + C), M, C, G, K, 2, K2, no)
+    d = ops.PqDeviceTensor(t)
+    x = torch.randn(t["N"], generator=torch.Generator().manual_seed(C))
+    x[torch.rand(t["N"], generator=torch.Generator().manual_seed(M)) < 0.3] *= 1e-4
+    inf = x.clone()
+    inf[t["N"] // 3] = float("inf")
+    raw = torch.full((d.ws.numel(),), 0x5A, dtype=torch.uint8, device="cuda")
+    out, want = torch.empty(M, device="cuda"), torch.empty(M, device="cuda")
+    for v, ws in ((x, raw), (inf, d.ws)):
+        for skip in (True, False):
+            v = v.cuda()
+            try:
+                _fused(ops, 0)
+                d.matmul(v, want) if skip else d.matmul_streaming(v, want)
+            finally:
+                _fused(ops, 1)
+            f = L.lib().ibh_pq_matmul if skip else L.lib().ibh_pq_matmul_streaming
+            out.fill_(7.0)
+            L._lib.check(f(ctypes.byref(d.s), v.data_ptr(), out.data_ptr(), ws.data_ptr(), ws.numel(),
+                           torch.cuda.current_stream().cuda_stream), "two-level direct")
+            if C > 32 or ws is d.ws:      # one slab needs no words: the tables serve it
+                np.testing.assert_array_equal(out.cpu().numpy(), want.cpu().numpy())
+            else:
+                assert (out - want).abs().max() <= 2e-6 * want.abs().max()
+    assert L.lib().ibh_device_errors(0) == 0
