@@ -481,8 +481,8 @@ __device__ __forceinline__ void table_tile(int K, const h8_t* cbs, const float* 
 }
 
 // Rows' sums from the codebooks and x directly, no tables and no row words:
-// two-level calls with a non-finite x or codeword, sums past the fixed-point
-// range, or a workspace without the stamp, all of which the three-kernel path
+// two-level calls with a non-finite or tiny x or a non-finite codeword, sums
+// past the fixed-point range, or a workspace without the stamp, all of which the three-kernel path
 // served.  The sums are that path's bit for bit: a lane sums the entries of
 // one of its slabs of 8 or 16 chunks, the slabs are added in order.  Rows
 // [lo, hi) of the block's tiles, two per group of lanes, into sums[row - tile
@@ -811,7 +811,10 @@ __global__ __launch_bounds__(kFThreads) void pq_fused(PqDev t, const float* __re
     // <= 2^50; the same on every slab (cbmax, gmax and the flag are over the
     // whole tensor), so either every slab adds or none does
     const float bound = 2.0f * (float)ninner * cbmax * gmax;
-    const bool off = nonfinite || !(bound <= 3.4e38f) || (TWO && S > 1 && !wsok);
+    // (two levels: neither does an x so small that its fp16 parts, scaled by at
+    // most 2^115, or the bound would lose bits)
+    const bool off = nonfinite || !(bound <= 3.4e38f) ||
+                     (TWO && ((S > 1 && !wsok) || (gmax > 0.f && gmax < 1e-30f)));
     bool fin[NR];
     float sum[NR];
     uint16_t rs_bits[NR];

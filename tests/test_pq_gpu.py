@@ -462,7 +462,7 @@ def test_pq_operands_at_any_address(ops, oracle_lib, M, C, K2):
 @pytest.mark.parametrize("M,C,G,K,K2,no", TWO_LEVEL + [(40, 2016, 16, 256, 256, 0), (1100, 700, 8, 64, 16, 8)])
 def test_two_level_direct_rows(ops, M, C, G, K, K2, no):
     """The sums that need neither tables nor row words (a workspace that was
-    not prepared, a non-finite x) are the three-kernel path's bit for bit."""
+    not prepared, a non-finite or tiny x) are the three-kernel path's bit for bit."""
     import ctypes
 
     import libinferbit_amd as L
@@ -474,9 +474,10 @@ def test_two_level_direct_rows(ops, M, C, G, K, K2, no):
     x[torch.rand(t["N"], generator=torch.Generator().manual_seed(M)) < 0.3] *= 1e-4
     inf = x.clone()
     inf[t["N"] // 3] = float("inf")
+    tiny = x * 2.0 ** -127                    # rows and table entries are subnormal
     raw = torch.full((d.ws.numel(),), 0x5A, dtype=torch.uint8, device="cuda")
     out, want = torch.empty(M, device="cuda"), torch.empty(M, device="cuda")
-    for v, ws in ((x, raw), (inf, d.ws)):
+    for v, ws in ((x, raw), (inf, d.ws), (tiny, d.ws)):
         for skip in (True, False):
             v = v.cuda()
             try:
