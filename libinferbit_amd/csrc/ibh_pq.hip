@@ -601,7 +601,7 @@ __global__ __launch_bounds__(kFThreads) void pq_fused(PqDev t, const float* __re
     __shared__ float red[kFThreads / 64], redc[kFThreads / 64], redc2[TWO ? kFThreads / 64 : 1];
     __shared__ float cmax_s[2][CS];
     __shared__ int8_t qq_s[1024];
-    __shared__ float meta_s;
+    __shared__ float ox_s[32], os_s[32];                   // fewer than 32 outliers: their x and scales
     __shared__ h8_t cbs[(TWO ? 4 : 2) * 256];              // the codebooks, fp16 rows padded to 8
     __shared__ __align__(16) float xsl[CS * kXS];          // the slab's x: [chunk][side][8], zero padded
     const int K = t.K, C = t.C, G = t.G, M = t.M, hf = G / 2;
@@ -769,6 +769,12 @@ __global__ __launch_bounds__(kFThreads) void pq_fused(PqDev t, const float* __re
     PQ_TT(1);
     // max|x| over the inner columns (the skipping rule's reference)
     float mx = 0.f;
+    float ox = 0.f, osc = 0.f;                             // thread j: outlier j's x and scale
+    if (t.n_outlier > 0) {
+        const int j = min(tid, t.n_outlier - 1);
+        ox = x[t.ocols[j]];
+        osc = f16_to_f32(t.oscale[j]);
+    }
     if (x4ok) {
 #pragma unroll
         for (int u = 0; u < 4; u++) {
@@ -913,27 +919,32 @@ __global__ __launch_bounds__(kFThreads) void pq_fused(PqDev t, const float* __re
     // outliers, fp32 otherwise
     const int no = t.n_outlier;
     const bool quant = no >= 32;
+    float meta = 1.f;
     if (no > 0) {
         bool any = false;
 #pragma unroll
         for (int h = 0; h < NR; h++) any |= fin[h];
         if (__syncthreads_or(any) == 0) return;
+        // (the largest product by a reduction over the threads, one product each:
+        // thread 0 walking 128 of them took 20 us)
+        const float ov = ox * osc;
         if (quant) {
-            if (tid == 0) {
-                float m = 0.f;
-                for (int j = 0; j < no; j++) {
-                    const float v = x[t.ocols[j]] * f16_to_f32(t.oscale[j]);
-                    const float av = v < 0 ? -v : v;
-                    if (av > m) m = av;
-                }
-                meta_s = m > 0.f ? m / 127.0f : 1.0f;
-            }
-            __syncthreads();
-            const float inv = 1.0f / meta_s;
-            for (int j = tid; j < no; j += kFThreads) {
-                const float sv = (x[t.ocols[j]] * f16_to_f32(t.oscale[j])) * inv;
+            const float m = wave_max_dpp(tid < no ? fabsf(ov) : 0.f);
+            if (lane == 0) red[wave] = m;
+        } else if (tid < no) {
+            ox_s[tid] = ox;
+            os_s[tid] = osc;
+        }
+        __syncthreads();
+        if (quant) {
+            float m = 0.f;
+#pragma unroll
+            for (int w = 0; w < kFThreads / 64; w++) m = fmaxf(m, red[w]);
+            meta = m > 0.f ? m / 127.0f : 1.0f;
+            if (tid < no) {
+                const float sv = ov * (1.0f / meta);
                 const int v = (int)(sv >= 0 ? sv + 0.5f : sv - 0.5f);
-                qq_s[j] = (int8_t)(v > 127 ? 127 : (v < -128 ? -128 : v));
+                qq_s[tid] = (int8_t)(v > 127 ? 127 : (v < -128 ? -128 : v));
             }
             __syncthreads();
         }
@@ -947,10 +958,12 @@ __global__ __launch_bounds__(kFThreads) void pq_fused(PqDev t, const float* __re
             const int8_t* sdc = t.oside + (size_t)r * no;
             if (quant) {
                 int32_t isum = 0;
+#pragma unroll 8
                 for (int j = 0; j < no; j++) isum += (int32_t)sdc[j] * (int32_t)qq_s[j];
-                y = fmaf((float)isum, meta_s, y);
+                y = fmaf((float)isum, meta, y);
             } else {
-                for (int j = 0; j < no; j++) y = fmaf((float)sdc[j] * f16_to_f32(t.oscale[j]), x[t.ocols[j]], y);
+#pragma unroll 8
+                for (int j = 0; j < no; j++) y = fmaf((float)sdc[j] * os_s[j], ox_s[j], y);
             }
         }
         out[r] = y;
