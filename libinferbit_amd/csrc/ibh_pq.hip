@@ -655,23 +655,31 @@ __global__ __launch_bounds__(kFThreads) void pq_fused(PqDev t, const float* __re
         for (int u = 0; u < 4; u++) xs4[u] = ld4f(x + 4 * (size_t)min(u * kFThreads + tid, n4 - 1));
     }
     // the index bytes last, unconditionally (a load under a branch is waited
-    // for where it joins): a ragged slab's block, whose tensor may hold fewer
-    // than 16 of them, loads pq_spare and reads its bytes one by one below
+    // for where it joins): 16 chunks from w0 on, the thread's own or, where the
+    // row ends before, its last 16.  A row of fewer loads pq_spare and its
+    // bytes one by one below (64 lanes' bytes lie in 64 lines, and a load takes
+    // a clock for each: 1024 x 3200, 256 + 256 codes 24.3 us with byte loads
+    // for every C that is not a multiple of 16, 11.2 so).
     __builtin_amdgcn_sched_barrier(0);
-    const bool vec = cn == CS && (C & 15) == 0;
+    const bool vec = C >= 16;
+    const int w0 = min(c0 + 16 * q, max(C - 16, 0));
     const uint8_t* const spare = (const uint8_t*)&pq_spare;
     const uint8_t *const b1l = vec ? t.i1l : spare, *const b1r = vec ? t.i1r : spare;
     const uint8_t *const b2l = vec ? t.i2l : spare, *const b2r = vec ? t.i2r : spare;
-    // level 2: 16 bytes a side, or 8 of packed 4-bit indices (C % 16 == 0: whole bytes)
+    // level 2: 16 bytes a side, or 8 of packed 4-bit indices (from the even
+    // chunk e0; a last piece of an odd C starts one behind w0, whose own index
+    // is then another thread's)
+    const int e0 = min(c0 + 16 * q, max(((C + 1) & ~1) - 16, 0));
     uint4 ivl[NR], ivr[NR], jvl[NR], jvr[NR];
 #pragma unroll
     for (int h = 0; h < NR; h++) {
-        const size_t io = vec ? (size_t)min(r0 + h * kFRows, M - 1) * C + c0 + 16 * q : 0;
+        const size_t rr = min(r0 + h * kFRows, M - 1), io = vec ? rr * C + w0 : 0;
         ivl[h] = ld16(b1l + io);
         ivr[h] = ld16(b1r + io);
         jvl[h] = jvr[h] = make_uint4(0, 0, 0, 0);
         if constexpr (P4) {
-            const u2a_t a = *(const u2a_t*)(b2l + io / 2), b = *(const u2a_t*)(b2r + io / 2);
+            const size_t po = vec ? rr * ((C + 1) >> 1) + (e0 >> 1) : 0;
+            const u2a_t a = *(const u2a_t*)(b2l + po), b = *(const u2a_t*)(b2r + po);
             jvl[h] = make_uint4(a.x, a.y, 0, 0);
             jvr[h] = make_uint4(b.x, b.y, 0, 0);
         } else if constexpr (TWO) {
@@ -845,27 +853,40 @@ __global__ __launch_bounds__(kFThreads) void pq_fused(PqDev t, const float* __re
             float acc = 0.f;
             if (vec) {
                 const uint32_t wl[4] = {ivl[h].x, ivl[h].y, ivl[h].z, ivl[h].w}, wr[4] = {ivr[h].x, ivr[h].y, ivr[h].z, ivr[h].w};
-                const uint32_t vl[4] = {jvl[h].x, jvl[h].y, jvl[h].z, jvl[h].w}, vr[4] = {jvr[h].x, jvr[h].y, jvr[h].z, jvr[h].w};
-                const float* Tq = T + (size_t)(16 * q) * TS;
-                const float* Tq2 = T2 + (size_t)(16 * q) * TS2;
-                auto term = [&](int j) {
+                uint32_t vl[4] = {jvl[h].x, jvl[h].y, jvl[h].z, jvl[h].w}, vr[4] = {jvr[h].x, jvr[h].y, jvr[h].z, jvr[h].w};
+                if (P4 && w0 != e0) {                          // nibble j: chunk w0 + j
+                    vl[1] = vl[1] << 4 | vl[0] >> 28; vl[0] <<= 4;
+                    vr[1] = vr[1] << 4 | vr[0] >> 28; vr[0] <<= 4;
+                }
+                // entry sum of the j-th loaded chunk, tables at Tc (and T2c)
+                auto term = [&](int j, const float* Tc, const float* T2c) {
                     const int il = (wl[j >> 2] >> (8 * (j & 3))) & 0xff, ir = (wr[j >> 2] >> (8 * (j & 3))) & 0xff;
-                    float v = Tq[j * TS + il] + Tq[j * TS + K + ir];
+                    float v = Tc[il] + Tc[K + ir];
                     if constexpr (TWO) {
                         const int jl = P4 ? (vl[j >> 3] >> (4 * (j & 7))) & 0xf : (vl[j >> 2] >> (8 * (j & 3))) & 0xff;
                         const int jr = P4 ? (vr[j >> 3] >> (4 * (j & 7))) & 0xf : (vr[j >> 2] >> (8 * (j & 3))) & 0xff;
-                        v = v + (Tq2[j * TS2 + jl] + Tq2[j * TS2 + K2 + jr]);
+                        v = v + (T2c[jl] + T2c[K2 + jr]);
                     }
                     return v;
                 };
-                if (keepm == full) {
+                const float* Tq = T + (size_t)(16 * q) * TS;
+                const float* Tq2 = T2 + (size_t)(16 * q) * TS2;
+                if (cn == CS && keepm == full) {
 #pragma unroll
-                    for (int j = 0; j < 16; j++) acc = acc + term(j);
+                    for (int j = 0; j < 16; j++) acc = acc + term(j, Tq + j * TS, Tq2 + j * TS2);
+                } else if (cn == CS) {
+#pragma unroll
+                    for (int j = 0; j < 16; j++) {
+                        const float val = term(j, Tq + j * TS, Tq2 + j * TS2);
+                        acc = acc + (((keepm >> (16 * q + j)) & 1) ? val : 0.f);
+                    }
                 } else {
 #pragma unroll
                     for (int j = 0; j < 16; j++) {
-                        const float val = term(j);
-                        acc = acc + (((keepm >> (16 * q + j)) & 1) ? val : 0.f);
+                        // chunks of the other thread or slab are loaded and not added
+                        const int c = w0 - c0 + j, cc = max(c, 0);
+                        const float val = term(j, T + cc * TS, T2 + cc * TS2);
+                        acc = acc + (c >= 16 * q && ((keepm >> cc) & 1) ? val : 0.f);
                     }
                 }
             } else if (r < M) {

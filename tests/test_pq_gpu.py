@@ -494,3 +494,28 @@ def test_two_level_direct_rows(ops, M, C, G, K, K2, no):
             else:
                 assert (out - want).abs().max() <= 2e-6 * want.abs().max()
     assert L.lib().ibh_device_errors(0) == 0
+
+
+# a slab's last 16-byte pieces: whole, part-filled, reaching into the slab or
+# row before, of odd rows whose packed codes start a half-byte later
+@pytest.mark.parametrize("K2", [0, 16, 64])
+@pytest.mark.parametrize("C", [15, 16, 17, 18, 30, 31, 32, 34, 47, 49, 63, 79, 94, 95])
+def test_pq_ragged_chunk_counts(ops, oracle_lib, C, K2):
+    from gen_golden import make_pq
+    print(f"case pq ragged C={C} K2={K2}", flush=True)
+    M = 70
+    t = make_pq(np.random.default_rng(C + K2), M, C, 16, 256, 2 if K2 else 1, K2, 5)
+    x = np.random.default_rng(C).standard_normal(t["N"]).astype(np.float32)
+    x[:: 3] *= 1e-4
+    d = ops.PqDeviceTensor(t)
+    v = torch.from_numpy(x).cuda()
+    a, b = torch.empty(M, device="cuda"), torch.empty(M, device="cuda")
+    for f in (d.matmul, d.matmul_streaming):
+        f(v, a)
+        try:
+            _fused(ops, 0)
+            f(v, b)
+        finally:
+            _fused(ops, 1)
+        # fp32 sums of up to 4 * 95 entries in two orders, entries of 23 bits of x
+        assert (a - b).abs().max() <= 1e-6 * b.abs().max()
