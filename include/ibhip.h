@@ -145,7 +145,10 @@ int ibh_matmul_w4a8_x_noalloc(float* out, const void* w, const void* scales, int
  * ibh_matmul_w4a8_batch is bit-identical to the x86 build's scalar kernel
  * (src/kernels/scalar.c:86-124: per-group multiply and add rounded apart);
  * ibh_matmul_int8_batch follows src/kernels/scalar.c:70-84 within fp32
- * tolerance.  B <= 32 (IB_BATCH_MAX, src/inferbit_internal.h:287). */
+ * tolerance: from 2 columns on x may be held to 2^-29 of the largest of each
+ * 128 columns (exactly from 2^-6 of it up) and summed as integers there, one
+ * column is an fp32 dot product.  B <= 32 (IB_BATCH_MAX,
+ * src/inferbit_internal.h:287). */
 int ibh_matmul_w4a8_batch(float* out, const void* w, const void* scales, int scale_kind,
                           const int8_t* qx, const float* sa, int M, int N, int B,
                           int M_stride, void* stream);

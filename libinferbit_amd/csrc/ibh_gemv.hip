@@ -541,7 +541,7 @@ extern "C" int ibh_matmul_int8_batch(float* out, const void* w, const void* scal
     hipStream_t st = ibh_resolve_stream(stream);
     if (const int f = ibh_launch_int8_skinny(out, w, scales, scale_kind, x, M, N, B, M_stride, st))
         return f < 0 ? IBH_ERROR_INTERNAL : IBH_OK;
-    // One column, or odd shapes: independent matvecs into the strided output.
+    // Odd shapes: independent matvecs into the strided output.
     for (int b = 0; b < B; b++) {
         int rc = ibh_matmul(out + (size_t)b * M_stride, w, scales, scale_kind, x + (size_t)b * N, M, N, 8,
                             stream);

@@ -354,12 +354,15 @@ __global__ __launch_bounds__(512) void w4a8_skinny(const BatchSet bs, const int8
 // ── INT8 rows x fp32 columns ────────────────────────────────────────────────
 // (kernels/scalar.c:70-84, within fp32 tolerance: sums in another order.)
 //
-// x becomes three int8 digit planes as in the one-column tile kernel, but per
-// (column, 128-column group): Q = rint(x * 4161400 / max|x|) in balanced
-// base-256 digits, so there is no second pass over x and an element keeps 23
-// bits of the group's largest.  Each group's exact int32 sums are combined,
-// scaled and added in fp32.  The 8 wavefronts of a block split K (their sums
-// meet in LDS, added in order).
+// x becomes four int8 digit planes per (column, 128-column group): Q =
+// trunc(x * 2^(30 - e)), e the exponent of the group's max|x|, in balanced
+// base-256 digits, so there is no second pass over x and an element is held to
+// 2^-29 of the group's largest: exactly down to 2^-6 of it.  (Three planes, 2^-23
+// of the largest, left elements that lie far below it fewer bits than an fp32
+// product has, which shows in rows whose weights on the large channels are 0.)
+// Each group's exact integer sum is rounded to fp32 once, scaled by the power of
+// two and added.  The 8 wavefronts of a block split K (their sums meet in LDS,
+// added in order).
 //
 // What bounds it is how its loads reach L1: neighbouring lanes in different
 // lines get one lane per clock.  With every lane loading its own 16 weights and
@@ -372,11 +375,12 @@ __global__ __launch_bounds__(512) void w4a8_skinny(const BatchSet bs, const int8
 // unit p = 4 m + q by lane (n, k quarter q) for MFMA m; the weights by the same
 // units of 16 columns, two lane swaps then giving them x's order of columns.
 // RT row tiles of a wavefront share its digits.
-// Measured in a graph, before (VALU, one wavefront per row) and here, at 2 / 8 /
-// 16 / 32 columns: 4096 x 4096 11.9 / 34.1 / 65 / 124 -> 8.6 / 9.1 / 11.4 / 16.6
-// us, 14336 x 4096 32.7 / 118 / 214 / 469 -> 21.8 / 23.1 / 28.9 / 38.5, 4096 x
-// 1024 5.0 / 12.2 / 21.5 / 40 -> 4.4 / 4.6 / 6.0 / 7.9.  Error against 64 bits
-// (relative to the outputs' norm): 4.5e-7 .. 6.7e-7 -> 4.2e-7 .. 4.8e-7.
+// Measured in a graph, one wavefront per row on the VALU (biased weights) and
+// here, at 3 / 8 / 16 / 32 columns: 4096 x 4096 15.6 / 34 / 65 / 124 -> 9.5 / 9.7 /
+// 11.7 / 18.2 us, 14336 x 4096 46 / 118 / 214 / 467 -> 23.5 / 24.5 / 30.1 / 41.7,
+// 4096 x 1024 6.2 / 11.9 / 21.5 / 40 -> 4.7 / 4.7 / 6.1 / 8.2 (three planes 4 to 8
+// % less).  Error against 64 bits relative to the outputs' norm: 5e-7 .. 1.1e-6
+// -> 7e-8 .. 9e-8 (three planes 3.3e-7 .. 5.2e-7).
 struct DigArgs {
     const int8_t* W;
     const void* sc;          // row scales
@@ -385,10 +389,10 @@ struct DigArgs {
     int M, N, B, ys, G, CPW; // G: 128-column groups of a row, CPW of them per wavefront
 };
 
-constexpr int kDigWaves = 8;
-// Q + 0x408080 in the low 23 bits of 2^23 + ..: bytes biased by 128, 128, 64
-constexpr float kDigMax = 4161400.f, kDigMagic = 8388608.f + 4227200.f;
-constexpr int kDigBytes = 3 * 1024;                            // digits of 8 slots x 128 columns
+constexpr int kDigWaves = 8, kDigPlanes = 4;
+constexpr int kDigBytes = kDigPlanes * 1024;                   // digits of 8 slots x 128 columns
+constexpr int kDigBits = 30;                                   // |Q| < 2^30
+constexpr int kDigMinExp = -119;                               // 2^(e - 30) stays a (subnormal) number: exact below it
 
 // max that lets a NaN through (v_maximum3_f32)
 __device__ __forceinline__ float nmax(float a, float b) { return __builtin_elementwise_maximum(a, b); }
@@ -398,10 +402,15 @@ __device__ __forceinline__ float dpp_nmax(float v) {
     return nmax(v, __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), CTRL, 0xF, 0xF, false)));
 }
 
-// Lane (i, k quarter q) of unit 4 m' + q holds columns 64 m' + 16 q + 4 d .. + 3
-// in dword d: swapping dword and quarter gives lane q
-// dword j of unit half m' = columns 64 m' + 16 j + 4 q, which is element e = 2 m' +
-// (j >> 1) of unit p = 4 (j & 1) + q.
+// orders a wavefront's LDS writes before its reads (no wait: they run in order)
+__device__ __forceinline__ void wave_fence() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
+// Lane (i, k quarter q) of unit 4 m + q holds columns 64 m + 16 q + 4 d .. + 3 in
+// dword d.  Swapping dword and quarter gives it columns 64 m + 16 j + 4 q in
+// dword j, which is element 2 m + (j >> 1) of x's unit 4 (j & 1) + q.
 __device__ __forceinline__ i4_t quarter_transpose(const uint4 w) {
     typedef unsigned int u2_t __attribute__((ext_vector_type(2)));
     const u2_t a = __builtin_amdgcn_permlane32_swap(w.x, w.z, false, false);
@@ -411,20 +420,17 @@ __device__ __forceinline__ i4_t quarter_transpose(const uint4 w) {
     return i4_t{(int)c[0], (int)c[1], (int)d[0], (int)d[1]};
 }
 
-// A row's sum over all columns in fp32, for a column that holds Inf or NaN:
-// both come out where they do without digits.
-__device__ __noinline__ float plain_dot(const int8_t* __restrict__ w, const float* __restrict__ x, int N) {
-    float y = 0.f;
-    for (int j = 0; j < N; j++) y = fmaf((float)w[j], x[j], y);
-    return y;
-}
+// Row tiles staged in LDS at a time: both, except where 4 passes' digits leave
+// room for one (they take turns then).
+constexpr int dig_row_bufs(int rt, int sh) { return rt == 2 && sh == 4 ? 1 : rt; }
 
 // SH: passes of 8 slots.
 template <int KIND, int RT, int SH>
 __global__ __launch_bounds__(64 * kDigWaves) void int8_skinny(const DigArgs a) {
     constexpr int NT = (SH + 1) / 2;                           // column tiles
     constexpr int RING = 4, XR = SH <= 2 ? 2 : 1;   // groups of weights and of x in flight
-    constexpr int WB = (SH * (kDigBytes + 32) + RT * 2048) / 4;   // a wavefront's LDS, in floats
+    constexpr int RB = dig_row_bufs(RT, SH);
+    constexpr int WB = (SH * (kDigBytes + 32) + RB * 2048) / 4;   // a wavefront's LDS, in floats
     static_assert(RT * NT * 256 <= WB, "the sums reuse the digits' LDS");
     extern __shared__ __align__(16) unsigned char smem[];
     const int N = a.N, B = a.B, M = a.M, G = a.G;
@@ -434,9 +440,9 @@ __global__ __launch_bounds__(64 * kDigWaves) void int8_skinny(const DigArgs a) {
     const int row0 = (int)blockIdx.x * 16 * RT;
     const int g0 = kw * a.CPW, gn = max(0, min(a.CPW, G - g0));
     float* mine = (float*)smem + (size_t)kw * WB;
-    uint4* ds = (uint4*)mine;                                  // [SH][3][64]
-    uint4* wl = ds + SH * 192;                                 // [RT][16 rows][8 units]
-    float* ss = (float*)(wl + RT * 128);                       // [SH][8] scales
+    uint4* ds = (uint4*)mine;                                  // [SH][4][64]
+    uint4* wl = ds + SH * 64 * kDigPlanes;                     // [RB][16 rows][8 units]
+    float* ss = (float*)(wl + RB * 128);                       // [SH][8] scales
 
     float4 xr[XR][SH][4];
     uint4 wr[RING][RT][2];
@@ -489,7 +495,7 @@ __global__ __launch_bounds__(64 * kDigWaves) void int8_skinny(const DigArgs a) {
 #pragma unroll
             for (int h = 0; h < SH; h++) {
                 float v[16];
-                float mx = 1e-31f;
+                float mx = 0.f;
 #pragma unroll
                 for (int e = 0; e < 4; e++) {
                     const float4 f = xr[u % XR][h][e];
@@ -499,68 +505,70 @@ __global__ __launch_bounds__(64 * kDigWaves) void int8_skinny(const DigArgs a) {
                 for (int e = 0; e < 16; e += 2) mx = nmax(nmax(mx, fabsf(v[e])), fabsf(v[e + 1]));
                 // the eight lanes of a slot share the scale, and with it that
                 // an element is not finite: the column's sums become NaN and
-                // are formed again in fp32 below.  The floor keeps 1 / mx
-                // finite (it rounds elements under 2e-38 in groups that hold
-                // nothing larger than 1e-31)
+                // are formed again in fp32 below
                 mx = dpp_nmax<0x141>(dpp_nmax<0x4E>(dpp_nmax<0xB1>(mx)));   // lane ^ 1, ^ 2, 7 - lane
-                const float inv = kDigMax / mx;
-                i4_t dg[3];
+                const int sh = kDigBits - max(__builtin_amdgcn_frexp_expf(mx), kDigMinExp);
+                i4_t dg[kDigPlanes];
 #pragma unroll
                 for (int d = 0; d < 4; d++) {
-                    uint32_t b[4];
+                    uint32_t b[4];                             // biased digits, least significant first
 #pragma unroll
                     for (int e = 0; e < 4; e++)
-                        b[e] = __builtin_bit_cast(uint32_t, fmaf(v[4 * d + e], inv, kDigMagic));
-                    const uint32_t p01 = __builtin_amdgcn_perm(b[1], b[0], 0x05010400u);
-                    const uint32_t p23 = __builtin_amdgcn_perm(b[3], b[2], 0x05010400u);
-                    const uint32_t h01 = __builtin_amdgcn_perm(b[1], b[0], 0x0c0c0602u);
-                    const uint32_t h23 = __builtin_amdgcn_perm(b[3], b[2], 0x06020c0cu);
-                    dg[0][d] = (int)(__builtin_amdgcn_perm(p23, p01, 0x05040100u) ^ 0x80808080u);
-                    dg[1][d] = (int)(__builtin_amdgcn_perm(p23, p01, 0x07060302u) ^ 0x80808080u);
-                    dg[2][d] = (int)(((h01 | h23) << 1) ^ 0x80808080u);
+                        b[e] = (uint32_t)(int)__builtin_amdgcn_ldexpf(v[4 * d + e], sh) + 0x80808080u;
+                    const uint32_t l01 = __builtin_amdgcn_perm(b[1], b[0], 0x05010400u);
+                    const uint32_t l23 = __builtin_amdgcn_perm(b[3], b[2], 0x05010400u);
+                    const uint32_t h01 = __builtin_amdgcn_perm(b[1], b[0], 0x07030602u);
+                    const uint32_t h23 = __builtin_amdgcn_perm(b[3], b[2], 0x07030602u);
+                    dg[0][d] = (int)(__builtin_amdgcn_perm(l23, l01, 0x05040100u) ^ 0x80808080u);
+                    dg[1][d] = (int)(__builtin_amdgcn_perm(l23, l01, 0x07060302u) ^ 0x80808080u);
+                    dg[2][d] = (int)(__builtin_amdgcn_perm(h23, h01, 0x05040100u) ^ 0x80808080u);
+                    dg[3][d] = (int)(__builtin_amdgcn_perm(h23, h01, 0x07060302u) ^ 0x80808080u);
                 }
                 const int s = lane >> 3, at = s * 8 + ((lane & 7) ^ s ^ (h & 1));
 #pragma unroll
-                for (int p = 0; p < 3; p++) *(i4_t*)(ds + (h * 3 + p) * 64 + at) = dg[p];
-                if ((lane & 7) == 0) ss[8 * h + s] = mx < __builtin_inff() ? mx * (1.0f / kDigMax) : __builtin_nanf("");
+                for (int p = 0; p < kDigPlanes; p++) *(i4_t*)(ds + (h * kDigPlanes + p) * 64 + at) = dg[p];
+                if ((lane & 7) == 0) ss[8 * h + s] = mx < __builtin_inff() ? __builtin_amdgcn_ldexpf(1.0f, -sh) : __builtin_nanf("");
             }
             xload(u % XR, g + XR);
-#pragma unroll
-            for (int t = 0; t < RT; t++)
-#pragma unroll
-                for (int m = 0; m < 2; m++)
-                    wl[t * 128 + 64 * m + (lane & 56) + ((lane & 7) ^ (lane >> 3) ^ m)] = wr[u][t][m];
-            wload(u, g + RING);
-            // the wavefront's LDS operations run in order: the reads below see
-            // the writes above, the next group's writes come after these reads
-            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-            __builtin_amdgcn_wave_barrier();
+            // the wavefront's LDS operations run in order: reads see the writes
+            // above them, later writes come after these reads
             i4_t av[RT][2];
 #pragma unroll
-            for (int t = 0; t < RT; t++) {
+            for (int t0 = 0; t0 < RT; t0 += RB) {
+                if (t0) wave_fence();
 #pragma unroll
-                for (int m = 0; m < 2; m++) {
-                    const i4_t T = quarter_transpose(wl[t * 128 + 8 * n + ((4 * m + q) ^ (n & 7) ^ (n >> 3))]);
-                    av[t][0][2 * m] = T[0]; av[t][1][2 * m] = T[1];
-                    av[t][0][2 * m + 1] = T[2]; av[t][1][2 * m + 1] = T[3];
+                for (int t = t0; t < t0 + RB; t++)
+#pragma unroll
+                    for (int m = 0; m < 2; m++)
+                        wl[(t - t0) * 128 + 64 * m + (lane & 56) + ((lane & 7) ^ (lane >> 3) ^ m)] = wr[u][t][m];
+                if (t0 + RB == RT) wload(u, g + RING);
+                wave_fence();
+#pragma unroll
+                for (int t = t0; t < t0 + RB; t++) {
+#pragma unroll
+                    for (int m = 0; m < 2; m++) {
+                        const i4_t T = quarter_transpose(wl[(t - t0) * 128 + 8 * n + ((4 * m + q) ^ (n & 7) ^ (n >> 3))]);
+                        av[t][0][2 * m] = T[0]; av[t][1][2 * m] = T[1];
+                        av[t][0][2 * m + 1] = T[2]; av[t][1][2 * m + 1] = T[3];
+                    }
+                    if (128 * (g + 1) > N)                     // av[m][e]: columns 32 e + 16 m + 4 q
+#pragma unroll
+                        for (int e = 0; e < 8; e++)
+                            if (128 * g + 16 * e >= N) av[t][e & 1][e >> 1] = 0;
                 }
-                if (128 * (g + 1) > N)                         // av[m][e]: columns 32 e + 16 m + 4 q
-#pragma unroll
-                    for (int e = 0; e < 8; e++)
-                        if (128 * g + 16 * e >= N) av[t][e & 1][e >> 1] = 0;
             }
             // 2. contraction and fold
 #pragma unroll
             for (int nt = 0; nt < NT; nt++) {
                 // a last tile of 8 slots has them in both halves of its columns
                 const int h = 2 * nt + 1 < SH ? 2 * nt + (n >> 3) : 2 * nt, s = n & 7;
-                const uint4* src = ds + h * 192 + s * 8;
+                const uint4* src = ds + h * 64 * kDigPlanes + s * 8;
                 const int sw = s ^ (h & 1);
-                i4_t d[RT][3];
+                i4_t d[RT][kDigPlanes];
 #pragma unroll
                 for (int m = 0; m < 2; m++)
 #pragma unroll
-                    for (int p = 0; p < 3; p++) {
+                    for (int p = 0; p < kDigPlanes; p++) {
                         const i4_t b = *(const i4_t*)(src + p * 64 + ((4 * m + q) ^ sw));
 #pragma unroll
                         for (int t = 0; t < RT; t++)
@@ -571,13 +579,14 @@ __global__ __launch_bounds__(64 * kDigWaves) void int8_skinny(const DigArgs a) {
                 for (int t = 0; t < RT; t++)
 #pragma unroll
                     for (int r = 0; r < 4; r++) {
-                        // |d| <= 2^21: the low two planes join exactly in int32
-                        const float lo = (float)(d[t][0][r] + (d[t][1][r] << 8));
-                        acc[t][nt][r] = fmaf(fmaf((float)d[t][2][r], 32768.f, lo), sc, acc[t][nt][r]);
+                        // |d| <= 2^21, so two planes join exactly in int32;
+                        // the low pair's carry moves up, so that one rounding
+                        // of the high pair and one of the sum remain
+                        const int lo = d[t][0][r] + (d[t][1][r] << 8), hi = d[t][2][r] + (d[t][3][r] << 8) + (lo >> 16);
+                        acc[t][nt][r] = fmaf(fmaf((float)hi, 65536.f, (float)(lo & 0xffff)), sc, acc[t][nt][r]);
                     }
             }
-            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-            __builtin_amdgcn_wave_barrier();
+            wave_fence();
         }
     }
 
@@ -589,16 +598,73 @@ __global__ __launch_bounds__(64 * kDigWaves) void int8_skinny(const DigArgs a) {
 #pragma unroll
             for (int r = 0; r < 4; r++) mine[(t * NT + nt) * 256 + r * 64 + lane] = acc[t][nt][r];
     __syncthreads();
-    for (int e = tid; e < RT * NT * 256; e += 64 * kDigWaves) {
+    for (int e = tid; e < RT * NT * 256; e += 64 * kDigWaves) {    // whole wavefronts
         const int rr = e & 15, col = (e >> 4) & 15, tile = e >> 8, t = tile / NT, nt = tile - t * NT;
         const int row = row0 + 16 * t + rr, s = 16 * nt + col;
-        if (row >= M || s >= B) continue;
+        const bool live = row < M && s < B;
         const float* p = (const float*)smem + tile * 256 + (rr & 3) * 64 + (rr >> 2) * 16 + col;
         float y = 0.f;
 #pragma unroll
         for (int k = 0; k < kDigWaves; k++) y += p[(size_t)k * WB];
-        if (!(fabsf(y) <= 3.4e38f)) y = plain_dot(a.W + (size_t)row * N, a.x + (size_t)s * N, N);
-        a.y[(size_t)s * a.ys + row] = y * load_scale<KIND>(a.sc, row);
+        // a column that holds Inf or NaN: the sum in fp32, by the whole
+        // wavefront, so that both come out where they do without digits
+        for (unsigned long long bad = __ballot(live && !(fabsf(y) <= 3.4e38f)); bad; bad &= bad - 1) {
+            const int l = __builtin_ctzll(bad);
+            const int8_t* w = a.W + (size_t)__builtin_amdgcn_readlane(row, l) * N;
+            const float* x = a.x + (size_t)__builtin_amdgcn_readlane(s, l) * N;
+            float v = 0.f;
+#pragma unroll 8
+            for (int j = lane; j < N; j += 64) v = fmaf((float)w[j], x[j], v);
+            v = wave_sum(v);
+            if (lane == l) y = v;
+        }
+        if (live) a.y[(size_t)s * a.ys + row] = y * load_scale<KIND>(a.sc, row);
+    }
+}
+
+// One column, or few beside a small matrix: a wavefront a row on the vector
+// units, which take x in fp32 and have no digits to make.  A signed weight is
+// the byte's float less 128: one operation more than the unsigned one, and none
+// for a sum of x that takes the bias out again and would round at 128 times the
+// largest x.  Bound by the L1 reads of x, made again for every row: 4096 x 4096
+// at 1 / 2 columns 7.1 / 10.5 us with both forms.
+template <int KIND, int B>
+__global__ __launch_bounds__(256) void int8_rows(const DigArgs a) {
+    const int lane = threadIdx.x & 63, row = (int)blockIdx.x * 4 + (threadIdx.x >> 6);
+    if (row >= a.M) return;
+    const uint8_t* w = (const uint8_t*)a.W + (size_t)row * a.N;
+    float acc[B];
+#pragma unroll
+    for (int b = 0; b < B; b++) acc[b] = 0.f;
+    for (int j = 16 * lane; j < a.N; j += 16 * 64) {
+        const uint4 q = ld_stream16(w + j);
+        const uint32_t d[4] = {q.x ^ 0x80808080u, q.y ^ 0x80808080u, q.z ^ 0x80808080u, q.w ^ 0x80808080u};
+        float f[16];
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            f[4 * e] = ubyte<0>(d[e]) - 128.f;
+            f[4 * e + 1] = ubyte<1>(d[e]) - 128.f;
+            f[4 * e + 2] = ubyte<2>(d[e]) - 128.f;
+            f[4 * e + 3] = ubyte<3>(d[e]) - 128.f;
+        }
+#pragma unroll
+        for (int b = 0; b < B; b++) {
+            const float4* xp = (const float4*)(a.x + (size_t)b * a.N + j);
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                const float4 v = xp[e];
+                acc[b] = fmaf(f[4 * e], v.x, acc[b]);
+                acc[b] = fmaf(f[4 * e + 1], v.y, acc[b]);
+                acc[b] = fmaf(f[4 * e + 2], v.z, acc[b]);
+                acc[b] = fmaf(f[4 * e + 3], v.w, acc[b]);
+            }
+        }
+    }
+    const float scale = load_scale<KIND>(a.sc, row);
+#pragma unroll
+    for (int b = 0; b < B; b++) {
+        const float v = wave_sum(acc[b]);
+        if (lane == 0) a.y[(size_t)b * a.ys + row] = v * scale;
     }
 }
 
@@ -672,17 +738,43 @@ int ibh_launch_w4a8_batch(const MatDesc* d, int n, int kind, const int8_t* qx, c
     return 1;
 }
 
-// INT8 rows x B fp32 columns (2 <= B <= 32).  Returns 1 if launched, 0 if the
+// INT8 rows x B fp32 columns (1 <= B <= 32).  Returns 1 if launched, 0 if the
 // shape is not taken, < 0 on a launch error.
 int ibh_launch_int8_skinny(float* out, const void* w, const void* sc, int kind, const float* x, int M, int N, int B,
                            int M_stride, hipStream_t st) {
-    if (B < 2 || B > 32 || N % 16 || N < 16 || (((uintptr_t)w | (uintptr_t)x) & 15)) return 0;
+    if (B < 1 || B > 32 || N % 16 || N < 16 || (((uintptr_t)w | (uintptr_t)x) & 15)) return 0;
+    // offsets within a launch's columns and a block's rows are 32 bits
+    if (N > 1 << 26) return 0;
+    const int most = (1 << 30) / N;
+    if (B > most) {
+        for (int b = 0; b < B; b += most) {
+            const int rc = ibh_launch_int8_skinny(out + (size_t)b * M_stride, w, sc, kind, x + (size_t)b * N, M, N,
+                                                  B - b < most ? B - b : most, M_stride, st);
+            if (rc <= 0) return rc;
+        }
+        return 1;
+    }
     const int G = (N + 127) / 128, T = (M + 15) / 16;
-    const DigArgs a{(const int8_t*)w, sc, x, out, M, N, B, M_stride, G, (G + kDigWaves - 1) / kDigWaves};
+        const DigArgs a{(const int8_t*)w, sc, x, out, M, N, B, M_stride, G, (G + kDigWaves - 1) / kDigWaves};
+    // One column has no digits to share: 14336 x 4096 19.0 us here, 23.5 there.
+    // Two cross at 2048 rows or 1024 columns (2048 x 8192 9.9 and 11.6, 4096 x
+    // 4096 10.5 and 9.3, 14336 x 512 7.9 and 8.4), three and four where few
+    // short rows leave the digits' kernel its latency (1000 x 2048 5.0 and 5.4
+    // at four, 1024 x 4096 7.6 and 7.4).
+    if (B == 1 || (B == 2 && (M <= 2048 || N <= 1024)) || (B <= 4 && M <= 1024 && N <= 2048)) {
+#define IBH_I8V(K_) do { const int g_ = (M + 3) / 4; \
+        if (B == 1) int8_rows<K_, 1><<<g_, 256, 0, st>>>(a); else if (B == 2) int8_rows<K_, 2><<<g_, 256, 0, st>>>(a); \
+        else if (B == 3) int8_rows<K_, 3><<<g_, 256, 0, st>>>(a); else int8_rows<K_, 4><<<g_, 256, 0, st>>>(a); } while (0)
+        if (kind == IBH_SCALE_F16) IBH_I8V(IBH_SCALE_F16); else IBH_I8V(IBH_SCALE_F32);
+#undef IBH_I8V
+        if (hipGetLastError() == hipSuccess) return 1;
+        ibh_set_error("int8 batch: launch failed");
+        return -1;
+    }
     // two row tiles share the digits where that still leaves a block per CU
     const int sh = (B + 7) / 8, rt = T > 256 ? 2 : 1;
     const int blocks = (T + rt - 1) / rt;
-    const size_t lds = (size_t)kDigWaves * (sh * (kDigBytes + 32) + rt * 2048);
+    const size_t lds = (size_t)kDigWaves * (sh * (kDigBytes + 32) + dig_row_bufs(rt, sh) * 2048);
 #define IBH_I8L(K_, R_, H_) do { \
         if (!lds_ok((const void*)int8_skinny<K_, R_, H_>, lds)) return 0; \
         int8_skinny<K_, R_, H_><<<blocks, 64 * kDigWaves, lds, st>>>(a); } while (0)

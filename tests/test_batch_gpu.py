@@ -151,10 +151,9 @@ def test_w4a8_batch_columns_bit_exact(oracle_lib, M, N, B):
 @pytest.mark.parametrize("M,N,B,ms", [(1, 16, 2, 1), (17, 144, 3, 20), (4100, 1040, 16, 4100), (4113, 4080, 9, 4113),
                                       (100, 8192, 17, 100), (4112, 656, 32, 4120)])
 def test_int8_batch_digits(M, N, B, ms):
-    """Fast INT8 batch against float64.  An element keeps max|group| * 2^-22.9
-    of error (half a digit unit of max / 4161400), the group factor 2^-23, each
-    of the fp32 sums (N / 128 / 8 in a wavefront, 8 over them) 2^-24 of its
-    partial: bounded by 2^-24 * (N / 1024 + 13) of sum |w| * max|group|."""
+    """Fast INT8 batch against float64.  An element keeps at most max|group| *
+    2^-29 of error (a digit unit), the group's sum 2^-23, each of the fp32 sums
+    (N / 128 / 8 in a wavefront, 8 over them) 2^-24 of its partial: bounded by 2^-24 * (N / 1024 + 13) of sum |w| * max|group|."""
     import torch
     import libinferbit_amd as L
     L.ops.init(0)
@@ -186,3 +185,68 @@ def test_int8_batch_digits(M, N, B, ms):
     assert (y[wm > 0] == np.inf).all() and (y[wm < 0] == -np.inf).all() and np.isnan(y[wm == 0]).all()
     assert np.isnan(got[(B - 1) * ms:]).all()
     np.testing.assert_array_equal(got[ms:(B - 1) * ms], clean[ms:(B - 1) * ms])
+
+
+def _int8_batch(w, s, x, ms=None):
+    import torch
+    import libinferbit_amd as L
+    L.ops.init(0)
+    B, N = x.shape
+    M = w.shape[0]
+    out = torch.empty(B * M, device="cuda")
+    g = lambda a: torch.from_numpy(a).cuda()
+    L.ops.matmul_int8_batch(out, g(w), g(s), g(x), M, N, B, M)
+    return out.cpu().numpy().reshape(B, M).astype(np.float64)
+
+
+# one column and several; rows on both sides of the split over row tiles
+@pytest.mark.parametrize("M,N,B", [(4096, 4096, 1), (100, 14336, 1), (300, 2048, 2), (4112, 1040, 8), (64, 8192, 32)])
+def test_int8_batch_small_beside_large(M, N, B):
+    """An element far below its group's largest keeps its bits: rows whose
+    weights on the large channels are 0, against float64.  A group's x is held
+    to 2^-29 of its largest (30 bits and sign, truncated); its integer sum is
+    rounded twice and each fp32 partial sum once (N / 1024 + 8 of them) to
+    2^-24, the row scale once more."""
+    print(f"case int8 range M={M} N={N} B={B}", flush=True)
+    r = np.random.default_rng(M + N + B)
+    w = r.integers(-127, 128, (M, N), dtype=np.int8)
+    s = (r.random(M) * 0.01 + 1e-4).astype(np.float32)
+    x = r.standard_normal((B, N)).astype(np.float32)
+    big = r.random(N) < 1 / 128
+    x[:, big] *= np.float32(2.0 ** 14)
+    w[: M // 2, big] = 0
+    got = _int8_batch(w, s, x)
+    gm = np.abs(np.pad(x, ((0, 0), (0, -N % 128)))).reshape(B, -1, 128).max(2).repeat(128, 1)[:, :N].astype(np.float64)
+    a = np.abs(w.astype(np.float64))
+    for b in range(B):
+        want = (w.astype(np.float64) @ x[b].astype(np.float64)) * s
+        bound = (2.0 ** -29 * (a @ gm[b]) + 2.0 ** -24 * (N / 1024 + 12) * (a @ np.abs(x[b]).astype(np.float64))) * s
+        assert (np.abs(got[b] - want) <= bound).all()
+
+
+def test_int8_batch_tiny_x():
+    """Groups of subnormal and just normal numbers, exactly held."""
+    r = np.random.default_rng(5)
+    w = r.integers(-127, 128, (40, 512), dtype=np.int8)
+    x = (r.integers(-(1 << 22), 1 << 22, (3, 512)) * 2.0 ** -149).astype(np.float32)
+    got = _int8_batch(w, np.ones(40, np.float32), x)
+    want = x.astype(np.float64) @ w.T.astype(np.float64)
+    assert (np.abs(got - want) <= 2.0 ** -24 * 8 * (np.abs(x).astype(np.float64) @ np.abs(w.T.astype(np.float64)))).all()
+
+
+def test_int8_batch_long_rows():
+    """Columns whose offsets pass 32 bits of bytes together."""
+    import torch
+    import libinferbit_amd as L
+    L.ops.init(0)
+    M, N, B = 2, (1 << 25) + 16, 32
+    print(f"case int8 long rows N={N} B={B}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(3)
+    w = torch.randint(-127, 128, (M, N), dtype=torch.int8, device="cuda", generator=g)
+    x = torch.randn(B, N, device="cuda", generator=g)
+    out = torch.empty(B, M, device="cuda")
+    L.ops.matmul_int8_batch(out, w, torch.ones(M, device="cuda"), x, M, N, B, M)
+    for b in range(B):
+        want = (w.double() * x[b].double()).sum(1)
+        # sums of 2^25 / 1024 + 8 fp32 steps in 8 wavefronts, each within 2^-24 of the partial sum
+        assert ((out[b].double() - want).abs() <= 2.0 ** -24 * N / 128 * 8 * want.abs().clamp(min=73 * N ** 0.5)).all()
