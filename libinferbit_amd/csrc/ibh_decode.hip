@@ -290,14 +290,16 @@ struct ibh_model {
     void* attn_ws = nullptr;
     size_t attn_ws_bytes = 0;
     int* dstate = nullptr;   // [0] pos, [1] prompt_end, [2..] tokens[capacity + 1]
-    // batched positions (prompts, forward_positions), allocated with the model
-    // or, where that found no memory, on first use, for kMaxBatch slots: activations [slot][dim], the attention's score rows or
-    // partials per slot
+    // batched positions (prompts, forward_positions) of kMaxBatch slots:
+    // activations [slot][dim], exact mode's score rows per slot.  Allocated
+    // with the model; where that found no memory prompts run as single steps
+    // and forward_positions asks again.  Fast mode's attention partials come
+    // when the mode is chosen; without them attn_ws serves slot by slot
     float *bx = nullptr, *bxb = nullptr, *bxb2 = nullptr, *bq = nullptr, *bk = nullptr, *bv = nullptr;
     float *bhb = nullptr, *bhb2 = nullptr, *blogits = nullptr, *bsa = nullptr;
     int8_t* bqx = nullptr;
-    void* battn = nullptr;
-    size_t battn_bytes = 0;
+    void *battn = nullptr, *bpart = nullptr;
+    size_t battn_bytes = 0, bpart_bytes = 0;
     int hpos = 0;
     hipGraphExec_t exec = nullptr;
     hipGraphExec_t bexec[2][33] = {};   // forward_batch graphs per (exact, B)
@@ -309,10 +311,10 @@ struct ibh_model {
 
 namespace {
 
-int dalloc(ibh_model* m, void** p, size_t bytes) {
+int dalloc(ibh_model* m, void** p, size_t bytes, bool quiet = false) {
     if (hipMalloc(p, bytes ? bytes : 16) != hipSuccess) {
         (void)hipGetLastError();   // reported here; the next launch check must not see it
-        ibh_set_error("ibh_model: device allocation of %zu bytes failed", bytes);
+        if (!quiet) ibh_set_error("ibh_model: device allocation of %zu bytes failed", bytes);
         return IBH_ERROR_MEMORY;
     }
     m->allocs.push_back(*p);
@@ -685,17 +687,14 @@ int step(ibh_model* m) {
 constexpr int kMaxBatch = 32;   // IB_BATCH_MAX (inferbit_internal.h:287)
 constexpr int kPromptMin = 3;   // fewer prompt positions run as single steps
 
-// The batched passes' buffers, one allocation on first use.
-int alloc_batch(ibh_model* m) {
+// The batched passes' buffers, one allocation (quiet: its failure is no error
+// of the caller's and leaves no message).
+int alloc_batch(ibh_model* m, bool quiet = false) {
     if (m->bx) return IBH_OK;
     const size_t B = kMaxBatch, H = m->hidden, KV = (size_t)m->n_kv * m->head_dim, I = m->inter, V = m->vocab;
     const size_t NM = H > I ? H : I;
-    // attention: exact mode (up to 8192 positions) keeps every slot's score
-    // rows, fast mode as many slots' partials as fit 256 MB
-    const size_t ex = m->max_pos + 1 <= 8192 ? B * ibh_attn_exact_scratch(m->n_heads, m->max_pos) : 0;
-    const size_t one = m->attn_ws_bytes, fit = ((size_t)256 << 20) / one;
-    const size_t fast = one * (fit < 1 ? 1 : fit < B ? fit : B);
-    m->battn_bytes = ex > fast ? ex : fast;
+    // exact attention (up to 8192 positions) keeps every slot's score rows
+    m->battn_bytes = m->max_pos + 1 <= 8192 ? B * ibh_attn_exact_scratch(m->n_heads, m->max_pos) : 0;
     size_t off = 0;
     auto take = [&](size_t bytes) {
         const size_t at = off;
@@ -707,7 +706,7 @@ int alloc_batch(ibh_model* m) {
     const size_t olg = take(B * V * 4), oqx = take(B * NM + 64), osa = take(B * (NM / 128 + 2) * 4);
     const size_t oat = take(m->battn_bytes);
     uint8_t* p = nullptr;
-    if (const int rc = dalloc(m, (void**)&p, off)) return rc;
+    if (const int rc = dalloc(m, (void**)&p, off, quiet)) return rc;
     m->bxb = (float*)(p + oxb);
     m->bxb2 = (float*)(p + oxb2);
     m->bq = (float*)(p + oq);
@@ -721,6 +720,17 @@ int alloc_batch(ibh_model* m) {
     m->battn = p + oat;
     m->bx = (float*)(p + ox);
     return IBH_OK;
+}
+
+// Fast mode's attention partials of as many slots as fit 256 MB, taken when
+// the mode is first chosen (64 MB, three slots a launch at 32768 positions of
+// 32 heads of 128, took 10 % longer for 8 to 32 of them).
+void alloc_partials(ibh_model* m) {
+    if (m->bpart || m->exact) return;
+    const size_t one = m->attn_ws_bytes, fit = ((size_t)256 << 20) / one, B = kMaxBatch;
+    const size_t bytes = one * (fit < 1 ? 1 : fit < B ? fit : B);
+    if (dalloc(m, &m->bpart, bytes, true) != IBH_OK) m->bpart = nullptr;
+    else m->bpart_bytes = bytes;
 }
 
 // int8 activation codes and group scales of B vectors.  Rows of whole groups
@@ -844,7 +854,8 @@ int forward_batch(ibh_model* m, int B, Pass pass) {
                                                  m->n_heads, m->n_kv, m->head_dim, m->kv_bits, (float*)m->battn,
                                                  m->battn_bytes, m->st)
                    : ibh_launch_attn_batch(m->bxb2, m->bq, L.kd, L.vd, L.ks, L.vs, m->dpos(), B, m->max_pos, m->n_heads,
-                                           m->n_kv, m->head_dim, m->kv_bits, m->battn, m->battn_bytes, m->st);
+                                           m->n_kv, m->head_dim, m->kv_bits, m->bpart ? m->bpart : m->attn_ws,
+                                           m->bpart ? m->bpart_bytes : m->attn_ws_bytes, m->st);
         if (rc || (rc = mm_batch1(m, L.o, m->bxb, m->bxb2, H, H, B, exact, pass)) ||
             (rc = norm_batch(m, m->bxb2, m->bx, m->bxb, L.post_norm, B, exact)))
             return rc;
@@ -958,9 +969,8 @@ int run_steps(ibh_model* m, int n) {
 // TinyLlama-width layers take 0.60 ms, as 32 steps 5.35 ms.
 int run_prompt(ibh_model* m, int n) {
     int rc, done = 0;
-    // (without memory for the batch buffers: single steps, which need none)
-    const bool batch = n >= kPromptMin && alloc_batch(m) == IBH_OK;
-    while (batch && n - done >= kPromptMin) {
+    // (without the batch buffers: single steps, which need none)
+    while (m->bx && n - done >= kPromptMin) {
         const int B = n - done < kMaxBatch ? n - done : kMaxBatch;
         if ((rc = forward_batch(m, B, done + B == n ? Pass::kPromptLast : Pass::kPrompt))) return rc;
         done += B;
@@ -1246,7 +1256,8 @@ int load(ibh_model* m, const char* path, int context_length) {
         IBH_HIP(hipMemcpy(m->rope, tab.data(), tab.size() * 4, hipMemcpyHostToDevice), "ibh_model_load: rope");
     }
     // with the model, not in the first prompt's time (0.8 ms of its 1.4)
-    (void)alloc_batch(m);
+    (void)alloc_batch(m, true);
+    alloc_partials(m);
     return set_state(m, 0, 0);
 }
 
@@ -1298,6 +1309,7 @@ extern "C" int ibh_model_set_exact(ibh_model* m, int exact) {
         m->exec = nullptr;
     }
     m->exact = exact != 0;
+    alloc_partials(m);
     return IBH_OK;
 }
 
