@@ -301,6 +301,9 @@ struct ibh_model {
     void *battn = nullptr, *bpart = nullptr;
     size_t battn_bytes = 0, bpart_bytes = 0;
     int hpos = 0;
+    // the device position is hpos: false while queued work moves it, and after
+    // a call that failed in between, until the next one uploads it
+    bool synced = false;
     hipGraphExec_t exec = nullptr;
     hipGraphExec_t bexec[2][33] = {};   // forward_batch graphs per (exact, B)
     std::vector<void*> allocs;
@@ -966,7 +969,8 @@ int run_steps(ibh_model* m, int n) {
 // of up to kMaxBatch positions; ends as n single steps would.  A pass reads
 // every weight once for all its positions and its serial fp32 chains run side
 // by side, where n steps read and run them n times: 32 tokens through four
-// TinyLlama-width layers take 0.60 ms, as 32 steps 5.35 ms.
+// TinyLlama-width layers take 0.46 ms, as 32 steps 5.35 ms.  Like the steps, it
+// moves hpos only when all of it is queued.
 int run_prompt(ibh_model* m, int n) {
     int rc, done = 0;
     // (without the batch buffers: single steps, which need none)
@@ -974,15 +978,17 @@ int run_prompt(ibh_model* m, int n) {
         const int B = n - done < kMaxBatch ? n - done : kMaxBatch;
         if ((rc = forward_batch(m, B, done + B == n ? Pass::kPromptLast : Pass::kPrompt))) return rc;
         done += B;
-        m->hpos += B;
     }
-    return done < n ? run_steps(m, n - done) : IBH_OK;
+    if (done < n && (rc = run_steps(m, n - done))) return rc;   // moves hpos by n - done
+    m->hpos += done;
+    return IBH_OK;
 }
 
 int set_state(ibh_model* m, int pos, int prompt_end) {
     const int s[2] = {pos, prompt_end};
     IBH_HIP(hipMemcpyAsync(m->dstate, s, sizeof s, hipMemcpyHostToDevice, m->st), "ibh_model: state upload");
     IBH_HIP(hipStreamSynchronize(m->st), "ibh_model: state upload");
+    m->synced = true;
     return IBH_OK;
 }
 
@@ -1385,12 +1391,13 @@ extern "C" int ibh_model_forward(ibh_model* m, const int32_t* tokens, int n, flo
         return IBH_ERROR_CONTEXT;
     }
     int rc;
-    if ((rc = check_tokens(m, tokens, n, "ibh_model_forward")) || (rc = put_tokens(m, tokens, n)) ||
-        (rc = run_prompt(m, n)))
-        return rc;
+    if ((rc = check_tokens(m, tokens, n, "ibh_model_forward")) || (rc = put_tokens(m, tokens, n))) return rc;
+    m->synced = false;
+    if ((rc = run_prompt(m, n))) return rc;
     IBH_HIP(hipMemcpyAsync(logits, m->logits, (size_t)vocab * 4, hipMemcpyDeviceToHost, m->st),
             "ibh_model_forward: logits");
     IBH_HIP(hipStreamSynchronize(m->st), "ibh_model_forward");
+    m->synced = true;
     return IBH_OK;
 }
 
@@ -1415,7 +1422,9 @@ extern "C" int ibh_model_forward_positions(ibh_model* m, const int32_t* tokens, 
         return IBH_ERROR_PARAM;
     }
     int rc;
-    if ((rc = check_tokens(m, tokens, n, "ibh_model_forward_positions")) || (rc = alloc_batch(m))) return rc;
+    if ((rc = check_tokens(m, tokens, n, "ibh_model_forward_positions")) || (rc = alloc_batch(m)) ||
+        (!m->synced && (rc = set_state(m, m->hpos, m->hpos))))
+        return rc;
     IBH_HIP(hipMemcpyAsync(m->dtokens() + m->hpos, tokens, (size_t)n * 4, hipMemcpyHostToDevice, m->st),
             "ibh_model_forward_positions: tokens");
     // one captured graph per (mode, B): the positions and tokens are device
@@ -1438,6 +1447,7 @@ extern "C" int ibh_model_forward_positions(ibh_model* m, const int32_t* tokens, 
         }
         hipGraphDestroy(g);
     }
+    m->synced = false;
     if (ge) {
         IBH_HIP(hipGraphLaunch(ge, m->st), "ibh_model_forward_positions: graph launch");
     } else if ((rc = forward_batch(m, n, Pass::kVerify))) {
@@ -1447,6 +1457,7 @@ extern "C" int ibh_model_forward_positions(ibh_model* m, const int32_t* tokens, 
             "ibh_model_forward_positions: logits");
     IBH_HIP(hipStreamSynchronize(m->st), "ibh_model_forward_positions");
     m->hpos += n;   // the pass advanced the device position itself
+    m->synced = true;
     return IBH_OK;
 }
 
@@ -1463,12 +1474,16 @@ extern "C" int ibh_model_generate_greedy(ibh_model* m, const int32_t* in, int n_
     }
     const int start = m->hpos;
     int rc;
-    if ((rc = check_tokens(m, in, n_in, "ibh_model_generate_greedy")) || (rc = put_tokens(m, in, n_in)) ||
-        (rc = run_prompt(m, n_in)) || (max_out > 1 && (rc = run_steps(m, max_out - 1))))
+    if ((rc = check_tokens(m, in, n_in, "ibh_model_generate_greedy")) || (rc = put_tokens(m, in, n_in))) return rc;
+    m->synced = false;
+    if ((rc = run_prompt(m, n_in)) || (max_out > 1 && (rc = run_steps(m, max_out - 1)))) {
+        m->hpos = start;
         return rc;
+    }
     IBH_HIP(hipMemcpyAsync(out, m->dtokens() + start + n_in, (size_t)max_out * 4, hipMemcpyDeviceToHost, m->st),
             "ibh_model_generate_greedy: tokens");
     IBH_HIP(hipStreamSynchronize(m->st), "ibh_model_generate_greedy");
+    m->synced = true;
     // the reference stops at the first end-of-sequence token (generate.c:283-297)
     int n = max_out;
     for (int i = 0; i < max_out; i++)
@@ -1490,7 +1505,12 @@ extern "C" int ibh_model_decode_steps(ibh_model* m, int n) {
         ibh_set_error("ibh_model_decode_steps: invalid step count");
         return IBH_ERROR_PARAM;
     }
-    return run_steps(m, n);
+    int rc;
+    if (!m->synced && (rc = set_state(m, m->hpos, m->hpos))) return rc;
+    m->synced = false;
+    if ((rc = run_steps(m, n))) return rc;
+    m->synced = true;
+    return IBH_OK;
 }
 
 extern "C" int ibh_model_synchronize(ibh_model* m) {

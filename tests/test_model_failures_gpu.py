@@ -108,3 +108,37 @@ def test_load_without_memory_for_batches(tmp_path):
         assert v("shim_mallocs").value == n + 2
         print("checked")
         """)
+
+
+def test_position_after_a_failed_call(tmp_path):
+    """A call whose pass ran but whose logits did not arrive leaves the length
+    as it was, and what follows starts from that length: the same results as
+    from a model that never saw it, also at the end of the context."""
+    run(tmp_path, """
+        def fails(f):
+            v("shim_fail_d2h").value = 1
+            try:
+                f()
+            except IbhError:
+                assert v("shim_fail_d2h").value == 0         # the copy was reached and failed
+                return
+            raise SystemExit("the copy did not fail")
+
+        a, b = Model(sys.argv[2]), Model(sys.argv[2])
+        for m in (a, b):
+            m.forward(toks[:20])
+        for n in (5, 32, 1):
+            fails(lambda: a.forward_positions(toks[:n]))
+            assert a.kv_length() == b.kv_length()
+            assert same(a.forward_positions(toks[3:7]), b.forward_positions(toks[3:7]))
+            assert same(a.forward(toks[9:10]), b.forward(toks[9:10]))
+        # up to the last position of the context
+        while b.kv_length() < 199:
+            n = min(32, 199 - b.kv_length())
+            fails(lambda: a.forward_positions(toks[:n]))
+            assert same(a.forward_positions(toks[:n]), b.forward_positions(toks[:n]))
+        fails(lambda: a.forward_positions(toks[:1]))
+        assert same(a.forward_positions(toks[:1]), b.forward_positions(toks[:1]))
+        assert a.kv_length() == b.kv_length() == 200
+        print("checked")
+        """)
