@@ -79,6 +79,26 @@ PROMPT_MODELS = {
 }
 
 
+def _add_masks(path, inter, keep):
+    """Append a sparsity mask to every layer of an IBF file: a share of `keep`
+    of the MLP rows active, other rows in each layer."""
+    import json
+
+    from libinferbit_amd import ibf
+    raw = open(path, "rb").read()
+    n = int(np.frombuffer(raw[8:16], np.uint32)[1])
+    head, data = json.loads(raw[32:32 + n]), raw[ibf._align(32 + n):]
+    for i, layer in enumerate(head["layers"]):
+        data += bytes(ibf._align(len(data)) - len(data))
+        layer["sparsity_mask"] = {"offset": len(data), "size": inter}
+        data += (np.random.default_rng(i).random(inter) < keep).astype(np.uint8).tobytes()
+    head["data"]["weight_data_size"] = len(data)
+    js = json.dumps(head, separators=(",", ":")).encode()
+    with open(path, "wb") as f:
+        f.write(raw[:8] + np.array([1, len(js), 0], np.uint32).tobytes() + bytes(12) + js)
+        f.write(bytes(ibf._align(32 + len(js)) - 32 - len(js)) + data)
+
+
 @pytest.mark.parametrize("name", list(PROMPT_MODELS))
 def test_prompt_equals_single_steps(tmp_path, name):
     """A prompt in batched passes leaves the logits, the cache and the greedy
@@ -250,3 +270,65 @@ def test_int8_batch_long_rows():
         want = (w.double() * x[b].double()).sum(1)
         # sums of 2^25 / 1024 + 8 fp32 steps in 8 wavefronts, each within 2^-24 of the partial sum
         assert ((out[b].double() - want).abs() <= 2.0 ** -24 * N / 128 * 8 * want.abs().clamp(min=73 * N ** 0.5)).all()
+
+
+@pytest.mark.parametrize("keep", [0.5, 0.9])                  # the sparse row path, and above its limit of 80 %
+@pytest.mark.parametrize("bits", [None, dict(gate_proj=8, up_proj=8, down_proj=8)])
+def test_prompt_with_sparsity_masks(tmp_path, keep, bits):
+    """Prompts through layers with a sparsity mask: the logits, the cache and
+    what follows of single steps, bit for bit, and other ones than unmasked."""
+    from libinferbit_amd import ibf
+    from libinferbit_amd.model import Model
+    cfg = dict(ibf.TINYLLAMA, num_layers=2, hidden_size=256, num_heads=4, num_kv_heads=2, head_dim=64,
+               intermediate_size=512, vocab_size=1000, max_context_length=200, kv_bits=8)
+    path = str(tmp_path / "m.ibf")
+    ibf.write_synthetic(path, cfg, seed=31, bits=bits)
+    plain = Model(path)
+    _add_masks(path, 512, keep)
+    one, many = Model(path), Model(path)
+    toks = np.random.default_rng(7).integers(0, 1000, 60).astype(np.int32)
+    print(f"case prompt mask {keep} {bits}", flush=True)
+    at = 0
+    for n in (7, 33):
+        for t in toks[at:at + n]:
+            a = one.forward([t])
+        b = many.forward(toks[at:at + n])
+        np.testing.assert_array_equal(a.view(np.uint32), b.view(np.uint32))
+        assert not np.array_equal(plain.forward(toks[at:at + n]), b)
+        at += n
+    np.testing.assert_array_equal(one.forward_positions(toks[:5]).view(np.uint32),
+                                  many.forward_positions(toks[:5]).view(np.uint32))
+
+
+@pytest.mark.parametrize("w4a8", [False, True])
+@pytest.mark.parametrize("name", ["int8kv", "all_int8", "all_int4", "mixed_qkv"])
+def test_fast_prompt_near_single_steps(tmp_path, monkeypatch, name, w4a8):
+    """Fast mode: a prompt's projections run on the batch kernels, so its
+    logits differ from single steps by fp32 rounding (1e-4 of the largest, as
+    fast and exact mode do), and with int8 activation codes by the codes that
+    such rounding moves by one (up to 1/127 of a group's largest, a few in a
+    thousand: 2e-2 at this width)."""
+    from libinferbit_amd import ibf
+    from libinferbit_amd.model import Model
+    monkeypatch.setenv("IB_W4A8", "1" if w4a8 else "0")
+    spec = dict(PROMPT_MODELS[name])
+    bits = spec.pop("bits", None)
+    cfg = dict(ibf.TINYLLAMA, num_layers=2, hidden_size=256, num_heads=4, num_kv_heads=2, head_dim=64,
+               intermediate_size=512, vocab_size=1000, max_context_length=200)
+    cfg.update(spec)
+    path = str(tmp_path / "m.ibf")
+    ibf.write_synthetic(path, cfg, seed=31, bits=bits)
+    one, many = Model(path), Model(path)
+    one.set_exact(False)
+    many.set_exact(False)
+    toks = np.random.default_rng(7).integers(0, 1000, 60).astype(np.int32)
+    print(f"case fast prompt {name} w4a8={w4a8}", flush=True)
+    at = 0
+    for n in (3, 33, 16):
+        for t in toks[at:at + n]:
+            a = one.forward([t])
+        b = many.forward(toks[at:at + n])
+        d = np.abs(a.astype(np.float64) - b).max() / np.abs(a).max()
+        print(f"  {n}: {d:.2e}", flush=True)
+        assert d <= (2e-2 if w4a8 else 1e-4)
+        at += n
