@@ -22,7 +22,8 @@ def table():
 
     k = Kernels()
     L.lib().ib_init_kernels_hip(C.byref(k))
-    return {"matmul_int8_batch": C.CFUNCTYPE(None, P, P, P, P, I, I, I, I)(k.matmul_int8_batch)}
+    return {"matmul_int8_batch": C.CFUNCTYPE(None, P, P, P, P, I, I, I, I)(k.matmul_int8_batch),
+            "matmul_int8": C.CFUNCTYPE(None, P, P, P, P, I, I)(k.matmul_int8)}
 
 
 # M, N, B, M_stride: one row and column block; partial row and column tiles;
@@ -332,3 +333,107 @@ def test_fast_prompt_near_single_steps(tmp_path, monkeypatch, name, w4a8):
         print(f"  {n}: {d:.2e}", flush=True)
         assert d <= (2e-2 if w4a8 else 1e-4)
         at += n
+
+
+# decoders of real widths, whose launches take the forms of many row blocks: 8
+# slots a block of the fused INT8 chains (40 row blocks and more), the W4A8 fold
+# handed on between wavefronts, and columns that do not fit LDS
+@pytest.mark.parametrize("I,bits", [(5632, None), (5600, None), (5600, dict(o_proj=8, gate_proj=8, up_proj=8, down_proj=8))])
+def test_wide_prompt_equals_single_steps(tmp_path, I, bits):
+    from libinferbit_amd import ibf
+    from libinferbit_amd.model import Model
+    cfg = dict(ibf.TINYLLAMA, num_layers=2, intermediate_size=I, vocab_size=1000, max_context_length=200)
+    path = str(tmp_path / "m.ibf")
+    ibf.write_synthetic(path, cfg, seed=31, bits=bits)
+    toks = np.random.default_rng(7).integers(0, 1000, 100).astype(np.int32)
+    one, many = Model(path), Model(path)
+    at = 0
+    for n in (32, 25, 31, 7):
+        print(f"case wide prompt {I} {bits} {at}+{n}", flush=True)
+        for t in toks[at:at + n]:
+            a = one.forward([t])
+        b = many.forward(toks[at:at + n])
+        np.testing.assert_array_equal(a.view(np.uint32), b.view(np.uint32))
+        at += n
+    np.testing.assert_array_equal(one.forward_positions(toks[:5]).view(np.uint32),
+                                  many.forward_positions(toks[:5]).view(np.uint32))
+
+
+class _Mat(C.Structure):                                       # MatDesc (ibh_common.h)
+    _fields_ = [("out", C.c_void_p), ("w", C.c_void_p), ("s", C.c_void_p), ("M", C.c_int)]
+
+
+def _internal(name, *args):
+    """A C++ launcher of the library that only its own files call."""
+    import libinferbit_amd as L
+    f = getattr(L.lib(), name)
+    f.restype, f.argtypes = C.c_int, args
+    return f
+
+
+# rows of 1 to 3 matrices, columns, slots: partial row blocks, 4 and 8 slots a
+# block with a remainder, a last tile of 16 columns
+@pytest.mark.parametrize("Ms,N,B", [((2000, 300, 260), 2048, 31), ((2000, 300, 260), 272, 7), ((2560,), 1040, 25),
+                                    ((4100,), 400, 17), ((70, 64), 16, 3), ((1,), 144, 1)])
+def test_fused_int8_chains_bit_exact(table, Ms, N, B):
+    """The prompt's INT8 products against the one-vector exact kernel, bit for
+    bit: normal numbers, subnormal ones, and sums that cancel to nothing."""
+    import torch
+
+    import libinferbit_amd as L
+    launch = _internal("_Z27ibh_launch_int8_batch_exactPKN3ibh7MatDescEiiPKfiibP12ihipStream_ti", C.c_void_p, C.c_int,
+                       C.c_int, C.c_void_p, C.c_int, C.c_int, C.c_bool, C.c_void_p, C.c_int)
+    r = np.random.default_rng(sum(Ms) + N + B)
+    ws = [r.integers(-127, 128, (M, N), dtype=np.int8) for M in Ms]
+    ss = [(r.random(M) * 0.01 + 1e-4).astype(np.float32) for M in Ms]
+    x = r.standard_normal((B, N)).astype(np.float32)
+    x[B // 3] *= np.float32(2.0) ** -135                       # products and sums subnormal or lost
+    x[2 * B // 3] *= np.float32(2.0) ** r.integers(-149, 100, N).astype(np.float32)
+    h = N // 32 * 16
+    for w in ws:                                               # a chain's second half takes its first away again
+        w[::2, h:2 * h] = -w[::2, :h]
+    x[B - 1, h:2 * h] = x[B - 1, :h]
+    dw = [torch.from_numpy(w).cuda() for w in ws]
+    ds = [torch.from_numpy(s).cuda() for s in ss]
+    dx = torch.from_numpy(x).cuda()
+    out = [torch.full((B, M), 7.0, device="cuda") for M in Ms]
+    d = (_Mat * len(Ms))(*[_Mat(o.data_ptr(), w.data_ptr(), s.data_ptr(), M) for o, w, s, M in zip(out, dw, ds, Ms)])
+    print(f"case fused chains {Ms} N={N} B={B}", flush=True)
+    assert launch(C.addressof(d), len(Ms), 1, dx.data_ptr(), N, B, True, torch.cuda.current_stream().cuda_stream, 0) == 0
+    p = lambda a: a.ctypes.data_as(C.c_void_p)
+    for o, w, s, M in zip(out, ws, ss, Ms):
+        got = o.cpu().numpy()
+        for b in range(B):
+            want = np.empty(M, np.float32)
+            table["matmul_int8"](p(want), p(w), p(s), p(np.ascontiguousarray(x[b])), M, N)
+            np.testing.assert_array_equal(got[b].view(np.uint32), want.view(np.uint32))
+
+
+# the fused fold handed on (tall), gathered, with codes from L2, and rows that
+# end inside a group; 2 matrices in a launch
+@pytest.mark.parametrize("Ms,N,B", [((8200,), 4096, 5), ((8200,), 4096, 17), ((5632, 5632), 2048, 32), ((2048,), 5632, 31),
+                                    ((1000, 500), 6176, 20), ((500,), 2080, 9), ((40,), 64, 17), ((1003,), 2048, 16)])
+def test_fused_w4a8_columns_bit_exact(Ms, N, B):
+    """The prompt's W4A8 products against the one-vector product, bit for bit."""
+    import torch
+
+    import libinferbit_amd as L
+    L.ops.init(0)
+    launch = _internal("_Z21ibh_launch_w4a8_batchPKN3ibh7MatDescEiiPKaPKfiibP12ihipStream_ti", C.c_void_p, C.c_int, C.c_int,
+                       C.c_void_p, C.c_void_p, C.c_int, C.c_int, C.c_bool, C.c_void_p, C.c_int)
+    r = np.random.default_rng(sum(Ms) + N + B)
+    g = lambda a: torch.from_numpy(a).cuda()
+    dw = [g(r.integers(0, 256, (M, N // 2), dtype=np.uint8)) for M in Ms]
+    ds = [g((r.random(M) * 0.01 + 1e-3).astype(np.float16)) for M in Ms]
+    q = g(r.integers(-127, 128, (B, N), dtype=np.int8))
+    sa = g((r.random((B, (N + 127) // 128)) * 0.02 + 1e-3).astype(np.float32))
+    out = [torch.full((B, M), 7.0, device="cuda") for M in Ms]
+    d = (_Mat * len(Ms))(*[_Mat(o.data_ptr(), w.data_ptr(), s.data_ptr(), M) for o, w, s, M in zip(out, dw, ds, Ms)])
+    print(f"case fused w4a8 {Ms} N={N} B={B}", flush=True)
+    assert launch(C.addressof(d), len(Ms), 0, q.data_ptr(), sa.data_ptr(), N, B, True,
+                  torch.cuda.current_stream().cuda_stream, 0) == 1
+    for o, w, s, M in zip(out, dw, ds, Ms):
+        y = torch.empty(M, device="cuda")
+        for b in range(B):
+            L.ops.parallel_matmul_w4a8(y, w, s, q[b].contiguous(), sa[b].contiguous(), M, N)
+            assert torch.equal(o[b].view(torch.int32), y.view(torch.int32))
