@@ -255,7 +255,9 @@ typedef struct {
  * nothing.  Calls that share a workspace must not overlap in time; different
  * workspaces are independent.  A non-finite x gives NaN rows for single-level
  * work (the CPU gives +-Inf or NaN); two-level work gives what the sums give,
- * for codewords that are not finite too.  No alignment beyond that of the
+ * for codewords that are not finite too.  x is held there to 2^-23 of each
+ * element down to 2^-17 of the largest of the codeword's own columns, sums to
+ * 2^-49 of sum|x| times the largest codeword element.  No alignment beyond that of the
  * elements is required of the tensor's arrays or of x. */
 size_t ibh_pq_workspace_bytes(const ibh_pq_tensor* t);
 /* Stamps a caller PQ workspace and zeroes its row words (a kernel on

@@ -363,19 +363,23 @@ __global__ __launch_bounds__(kThreads) void pq_reduce(PqDev t, const float* __re
 //     v_mfma_f32_32x32x16_f16 with A = [cb | cb] (the fp16 codewords, exact)
 //     and B = [x_hi ; x_lo], x scaled per (chunk, side) by a power of two
 //     (exact) and split into two fp16 parts; products are exact and sums
-//     fp32.  x is scaled by one power of two per slab that takes its max|x|
-//     to the top of fp16: an element's two parts then keep 2^-23 of the
-//     element itself down to 2^-17 of the slab's max (scaled to 1 instead,
-//     small elements lost their low parts: error against 64 bits 3.0e-7 ->
-//     1.5e-7, 3489 rows of 201 chunks).
+//     fp32.  The power of two takes the 8 elements' max|x| to the top of fp16:
+//     an element's two parts then keep 2^-23 of the element itself down to
+//     2^-17 of that max.  (Scaled to 1 instead, small elements lost their low
+//     parts: error against 64 bits 3.0e-7 -> 1.5e-7, 3489 rows of 201 chunks.
+//     With one power of two a slab, one large channel took bits from every
+//     other chunk of it: 520 x 1536, rows whose codewords are 0 on a channel
+//     2^20 / 2^26 / 2^32 times the others, error 6e-7 / 4e-5 / 3e-3 -> 1.1e-7 /
+//     1.1e-7 / 6e-7, the three kernels 1.1e-7.)
 //  3. Max|x| over the inner columns (the skipping rule of
-//     pq_decode.c:1569-1616), the slab's chunk maxima, max|codeword|.
+//     pq_decode.c:1569-1616) and sum|x|, the slab's chunk maxima.
 //  4. Gather: 32 LDS lookups per thread, the row's two partials summed.
 //  5. Slabs meet per row in one 64-bit word: each slab adds
 //     2^58 + round(partial * 2^q) + 2^50 (an agent-scope atomic with return,
 //     performed where every XCD sees it).  2^q maps the largest sum the
-//     inputs allow (N * max|cb| * max|x|, doubled) to 2^50, so every term is
-//     an exact integer below 2^51 and the sum of at most 63 slabs stays
+//     inputs allow (max|cb| * sum|x|, doubled; with N * max|x| in place of
+//     the sum one large channel cost the other rows bits) to 2^50, so every
+//     term is an exact integer below 2^51 and the sum of at most 63 slabs stays
 //     below 2^58; the count sits above.  The slab whose add completes the
 //     count has the whole row in the returned value: it applies the row scale
 //     and the outliers, writes y and clears the word for the next call.
@@ -392,12 +396,13 @@ __global__ __launch_bounds__(kThreads) void pq_reduce(PqDev t, const float* __re
 //  Two levels double the tables, the lookups and the index bytes and keep the
 //  rest: 4096 x 14336, 256 + 256 codes, streaming: 75.3 us in three launches
 //  (68 of them the gather, 16 chunks' tables re-read by every block of 512
-//  rows and two byte loads per lookup) -> 13.1 us, error 2.1e-7 -> 1.2e-7.
+//  rows and two byte loads per lookup) -> 12.4 us, error 2.1e-7 -> 1.2e-7.
 constexpr int kFThreads = 1024;
 constexpr int kFRows = 512;
 constexpr int kFCS = 32;
 constexpr int kFMaxS = 63;
 constexpr int kFMaxRows = 131072;
+constexpr int kMinExp = -100;   // exponents of x below it share its scale
 constexpr int kXS = 20;   // LDS floats per slab chunk: 8 per side (zero padded) + 4 (bank spread)
 __device__ unsigned long long pq_row_acc[kFMaxRows];   // ws == NULL calls: zero at load, each row's last slab clears it
 __device__ unsigned int ibh_pq_err;                    // IBH_DEVERR_* bits of this file's kernels
@@ -431,29 +436,27 @@ __device__ __forceinline__ float4 ld4f(const float* p) {
 typedef _Float16 h8_t __attribute__((ext_vector_type(8)));
 typedef float f16x_t __attribute__((ext_vector_type(16)));
 
-// One table tile (side sd, codes 32*kt.., chunks 32*ct.. of the slab; the
-// item index is wave-uniform, so its decomposition is scalar work) from the
-// block's LDS copies of the codebooks (fp16, rows padded to 8) and of the
-// slab's x, scaled by 2^-e (e: exponent of max|x|, one per call, so the
-// entries are T * 2^-e and the row sums are rescaled once).  Tiles with
-// kt == 0 also record each (chunk, side)'s max|x|.
-template <bool KA, int CS, bool CMAX>
-__device__ __forceinline__ void table_tile(int K, const h8_t* cbs, const float* xsl, int it, int KT, int CT, int cn,
-                                           int lane, int TS, float xscale, float* T, float (*cmax_s)[CS]) {
-    const int sd = it / (KT * CT), rest = it - sd * KT * CT, kt = rest / CT, ct = rest - kt * CT;
-    const int k = min(kt * 32 + (lane & 31), K - 1);
-    const int cc = ct * 32 + (lane & 31);
-    const int ccl = min(cc, cn - 1);
-    const h8_t a = cbs[sd * K + k];
-    const float4* xp = (const float4*)(xsl + ccl * kXS + sd * 8);
+// The slab's tables from the block's LDS copies of the codebooks (fp16, rows
+// padded to 8) and of the slab's x.  A wavefront has one side: it scales and
+// splits that side's x once (a lane has a chunk's whole) and takes every eighth
+// 32-code tile of both levels.  (Split again for each tile, 4096 x 14336 at 256
+// + 256 codes: 13.3 us; 12.4 so.)  Scales are a power of two of each (chunk,
+// side); the entries leave as T * 2^-ex, so that the row sums are rescaled once.
+// Records each (chunk, side)'s max|x|.
+template <bool KA, bool TWO>
+__device__ __forceinline__ void slab_tables(int K, int K2, const h8_t* cbs, const float* xsl, int cn, int wave, int lane,
+                                            int ex, float* T1, float* T2, float (*cmax_s)[kFCS]) {
+    static_assert(kFCS == 32);
+    const int sd = wave & 1, cc = lane & 31;
+    const float4* xp = (const float4*)(xsl + min(cc, cn - 1) * kXS + sd * 8);
     const float4 x0 = xp[0], x1 = xp[1];
     const float xv[8] = {x0.x, x0.y, x0.z, x0.w, x1.x, x1.y, x1.z, x1.w};
-    if (CMAX && kt == 0) {
-        float m = 0.f;
+    float m = 0.f;
 #pragma unroll
-        for (int i = 0; i < 8; i++) m = fmaxf(m, fabsf(xv[i]));
-        if (lane < 32 && cc < cn) cmax_s[sd][cc] = m;        // this (chunk, side)'s max|x|
-    }
+    for (int i = 0; i < 8; i++) m = fmaxf(m, fabsf(xv[i]));
+    if (wave < 2 && lane < cn) cmax_s[sd][lane] = m;
+    const int ec = m > 0.f ? max(__builtin_amdgcn_frexp_expf(m), kMinExp) - 15 : ex;   // m < 2^(ec + 15)
+    const float xscale = ldexpf(1.0f, -ec), es = ldexpf(1.0f, ec - ex);
     const bool lo = lane >= 32;
     h8_t b;
 #pragma unroll
@@ -462,19 +465,25 @@ __device__ __forceinline__ void table_tile(int K, const h8_t* cbs, const float* 
         const _Float16 h = (_Float16)v;
         b[i] = lo ? (_Float16)(v - (float)h) : h;
     }
-    const f16x_t d = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, f16x_t{}, 0, 0, 0);
-    // D[k][n]: lane (n = lane & 31), register r: row 8*(r>>2) + 4*(lane>>5) + (r&3)
-    if (cc < cn) {
-        float* dst = T + (size_t)cc * TS + sd * K + kt * 32 + 4 * (lane >> 5);
+    const int KT1 = (K + 31) / 32, KT = KT1 + (TWO ? (K2 + 31) / 32 : 0);
+    for (int j = wave >> 1; j < KT; j += kFThreads / 128) {
+        const bool second = TWO && j >= KT1;
+        const int k0 = 32 * (second ? j - KT1 : j), Kj = second ? K2 : K;
+        const h8_t a = cbs[(second ? 2 * K : 0) + sd * Kj + min(k0 + (lane & 31), Kj - 1)];
+        const f16x_t d = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, f16x_t{}, 0, 0, 0) * es;
+        // D[k][n]: lane (n = lane & 31), register r: row 8*(r>>2) + 4*(lane>>5) + (r&3)
+        if (cc < cn) {
+            float* dst = (second ? T2 : T1) + (size_t)cc * (2 * Kj + 4) + sd * Kj + k0 + 4 * (lane >> 5);
 #pragma unroll
-        for (int g = 0; g < 4; g++) {
-            const int kk = kt * 32 + 8 * g + 4 * (lane >> 5);
-            const float4 v = make_float4(d[4 * g], d[4 * g + 1], d[4 * g + 2], d[4 * g + 3]);
-            if (KA || kk + 3 < K) *(float4*)(dst + 8 * g) = v;
-            else {
-                const float vv[4] = {v.x, v.y, v.z, v.w};
-                for (int u = 0; u < 4; u++)
-                    if (kk + u < K) dst[8 * g + u] = vv[u];
+            for (int g = 0; g < 4; g++) {
+                const int kk = k0 + 8 * g + 4 * (lane >> 5);
+                const float4 v = make_float4(d[4 * g], d[4 * g + 1], d[4 * g + 2], d[4 * g + 3]);
+                if (KA || kk + 3 < Kj) *(float4*)(dst + 8 * g) = v;
+                else {
+                    const float vv[4] = {v.x, v.y, v.z, v.w};
+                    for (int u = 0; u < 4; u++)
+                        if (kk + u < Kj) dst[8 * g + u] = vv[u];
+                }
             }
         }
     }
@@ -757,26 +766,16 @@ __global__ __launch_bounds__(kFThreads) void pq_fused(PqDev t, const float* __re
         if (TWO) cbmax2 = fmaxf(cbmax2, redc2[w]);
     }
     if (TWO) cbmax += cbmax2;
-    // the tables carry 2^-ex: x scaled so that the slab's max|x| sits just
-    // below 2^15, the top of fp16, and the low halves of its elements stay
-    // normal numbers down to 2^-17 of it
+    // the tables carry 2^-ex, the slab's max|x| below 2^15
     int ex = 0;
     if (smax > 0.f) frexpf(smax, &ex);                     // smax < 2^ex
-    ex = max(ex, -100) - 15;
-    const float xscale = ldexpf(1.0f, -ex);
+    ex = max(ex, kMinExp) - 15;
 
-    // 2. tables: items (side, 32-code tile, 32-chunk tile), <= 32
-    const int KT = (K + 31) / 32, CT = (cn + 31) / 32, items = 2 * KT * CT;
-    for (int it = wave; it < items; it += kFThreads / 64)
-        table_tile<KA, CS, true>(K, cbs, xsl, it, KT, CT, cn, lane, TS, xscale, T, cmax_s);
-    if constexpr (TWO) {
-        const int KT2 = (K2 + 31) / 32;
-        for (int it = wave; it < 2 * KT2 * CT; it += kFThreads / 64)
-            table_tile<KA, CS, false>(K2, cbs + 2 * K, xsl, it, KT2, CT, cn, lane, TS2, xscale, T2, cmax_s);
-    }
+    // 2. tables
+    slab_tables<KA, TWO>(K, K2, cbs, xsl, cn, wave, lane, ex, T, T2, cmax_s);
     PQ_TT(1);
-    // max|x| over the inner columns (the skipping rule's reference)
-    float mx = 0.f;
+    // max|x| over the inner columns (the skipping rule's reference) and sum|x|
+    float mx = 0.f, sx = 0.f;
     float ox = 0.f, osc = 0.f;                             // thread j: outlier j's x and scale
     if (t.n_outlier > 0) {
         const int j = min(tid, t.n_outlier - 1);
@@ -787,7 +786,9 @@ __global__ __launch_bounds__(kFThreads) void pq_fused(PqDev t, const float* __re
 #pragma unroll
         for (int u = 0; u < 4; u++) {
             const float a = fmaxf(fmaxf(fabsf(xs4[u].x), fabsf(xs4[u].y)), fmaxf(fabsf(xs4[u].z), fabsf(xs4[u].w)));
+            const float b = (fabsf(xs4[u].x) + fabsf(xs4[u].y)) + (fabsf(xs4[u].z) + fabsf(xs4[u].w));
             mx = fmaxf(mx, a);
+            sx += u * kFThreads + tid < ninner >> 2 ? b : 0.f;
             nonfin |= !(fabsf(xs4[u].x) <= 3.4e38f && fabsf(xs4[u].y) <= 3.4e38f && fabsf(xs4[u].z) <= 3.4e38f &&
                         fabsf(xs4[u].w) <= 3.4e38f);
         }
@@ -799,17 +800,26 @@ __global__ __launch_bounds__(kFThreads) void pq_fused(PqDev t, const float* __re
 #pragma unroll
             for (int u = 0; u < 16; u++) {
                 mx = fmaxf(mx, fabsf(v[u]));
+                sx += j0 + u * kFThreads + tid < ninner ? fabsf(v[u]) : 0.f;
                 nonfin |= !(fabsf(v[u]) <= 3.4e38f);
             }
         }
     }
     mx = wave_max_dpp(mx);
+    sx = wave_sum_dpp(sx);
     __syncthreads();                                       // tables done; red[] read above
-    if (lane == 0) red[wave] = mx;
+    if (lane == 0) {
+        red[wave] = mx;
+        redc[wave] = sx;
+    }
     const bool nonfinite = __syncthreads_or(nonfin) != 0;
-    float gmax = 0.f;
+    
+    float gmax = 0.f, gsum = 0.f;
 #pragma unroll
-    for (int w = 0; w < kFThreads / 64; w++) gmax = fmaxf(gmax, red[w]);
+    for (int w = 0; w < kFThreads / 64; w += 4) {
+        gmax = fmaxf(fmaxf(gmax, fmaxf(red[w], red[w + 1])), fmaxf(red[w + 2], red[w + 3]));
+        gsum += (redc[w] + redc[w + 1]) + (redc[w + 2] + redc[w + 3]);
+    }
     // the slab's kept chunks as a mask, made by every wavefront (lane = chunk)
     bool keep = false;
     if (lane < cn) {
@@ -821,10 +831,10 @@ __global__ __launch_bounds__(kFThreads) void pq_fused(PqDev t, const float* __re
     const unsigned long long full = cn == 64 ? ~0ull : ((1ull << cn) - 1);
     PQ_TT(2);
 
-    // 2^qe maps 2 * N_inner * max|cb| * max|x| (a bound on |row sum|) to
-    // <= 2^50; the same on every slab (cbmax, gmax and the flag are over the
-    // whole tensor), so either every slab adds or none does
-    const float bound = 2.0f * (float)ninner * cbmax * gmax;
+    // 2^qe maps 2 * max|cb| * sum|x| (a bound on |row sum|) to <= 2^50; the
+    // same on every slab (cbmax, gsum and the flag are over the whole tensor,
+    // summed in the same order), so either every slab adds or none does
+    const float bound = 2.0f * cbmax * gsum;
     // (two levels: neither does an x so small that its fp16 parts, scaled by at
     // most 2^115, or the bound would lose bits)
     const bool off = nonfinite || !(bound <= 3.4e38f) ||

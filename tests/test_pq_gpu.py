@@ -519,3 +519,51 @@ def test_pq_ragged_chunk_counts(ops, oracle_lib, C, K2):
             _fused(ops, 1)
         # fp32 sums of up to 4 * 95 entries in two orders, entries of 23 bits of x
         assert (a - b).abs().max() <= 1e-6 * b.abs().max()
+
+
+# slabs of 32 chunks: the large channel's own, others, a ragged last one; x read
+# as float4s (G = 16) and element by element (95 chunks of 6)
+@pytest.mark.parametrize("M,C,G,K2", [(520, 96, 16, 0), (520, 96, 16, 16), (520, 96, 16, 256), (1100, 95, 6, 64),
+                                      (300, 20, 16, 0)])
+def test_pq_rows_without_the_large_channel(ops, M, C, G, K2):
+    """A channel 2^32 times the others: rows whose codewords are 0 there keep
+    the bits of the others."""
+    from gen_golden import make_pq
+    print(f"case pq large channel {M}x{C} G={G} K2={K2}", flush=True)
+    K, hf, big = 256, G // 2, 3
+    rng = np.random.default_rng(M + C + K2)
+    t = make_pq(rng, M, C, G, K, 2 if K2 else 1, K2, 0)
+    books = [("cb1l", "cb1r", "i1l", "i1r")] + ([("cb2l", "cb2r", "i2l", "i2r")] if K2 else [])
+    x = rng.standard_normal(C * G).astype(np.float32)
+    x[big * G + 1] = 2.0 ** 32
+    want, size = np.zeros(M), np.zeros(M)
+    for names in books:
+        for side, (cb, ix) in enumerate(zip(names[:2], names[2:])):
+            t[cb] = t[cb].copy()
+            t[ix] = t[ix].copy()
+            words = t[cb].reshape(-1, hf)
+            words[0] = 0
+            idx = t[ix].reshape(M, -1)
+            if ix[1] == "2" and K2 == 16:
+                codes = np.stack([idx & 15, idx >> 4], -1).reshape(M, -1)[:, :C]
+                if side == 0:
+                    idx[:, big // 2] &= 15                  # chunk 3: the high half
+                    codes[:, big] = 0
+            else:
+                codes = idx
+                if side == 0:
+                    idx[:, big] = 0
+            tab = np.einsum("kh,ch->ck", words.view(np.float16).astype(np.float64),
+                            x.astype(np.float64).reshape(C, 2, hf)[:, side])
+            terms = tab[np.arange(C)[None], codes]
+            want += terms.sum(1)
+            size += np.abs(np.einsum("kh,ch->ck", np.abs(words.view(np.float16).astype(np.float64)),
+                                     np.abs(x.astype(np.float64)).reshape(C, 2, hf)[:, side])[np.arange(C)[None], codes]).sum(1)
+    scale = t["row_scale"].view(np.float16).astype(np.float64)
+    d = ops.PqDeviceTensor(t)
+    out = torch.empty(M, device="cuda")
+    d.matmul_streaming(torch.from_numpy(x).cuda(), out)
+    got = out.cpu().numpy().astype(np.float64)
+    # x to 2^-22 of each element (down to 2^-17 of its 8), chains of up to 16 + 16
+    # fp32 adds of 2^-24 each
+    assert (np.abs(got - want * scale) <= 2.0 ** -18 * size * np.abs(scale)).all()
