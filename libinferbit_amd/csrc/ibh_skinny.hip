@@ -627,7 +627,9 @@ __global__ __launch_bounds__(64 * kDigWaves) void int8_skinny(const DigArgs a) {
 // the byte's float less 128: one operation more than the unsigned one, and none
 // for a sum of x that takes the bias out again and would round at 128 times the
 // largest x.  Bound by the L1 reads of x, made again for every row: 4096 x 4096
-// at 1 / 2 columns 7.1 / 10.5 us with both forms.
+// at 1 / 2 columns 7.1 / 10.5 us with both forms.  All columns' loads are issued
+// ahead of the products (with each column's in front of its own, 1000 x 4096 at
+// 3 columns 5.8 us, 5.0 so).
 template <int KIND, int B>
 __global__ __launch_bounds__(256) void int8_rows(const DigArgs a) {
     const int lane = threadIdx.x & 63, row = (int)blockIdx.x * 4 + (threadIdx.x >> 6);
@@ -647,12 +649,16 @@ __global__ __launch_bounds__(256) void int8_rows(const DigArgs a) {
             f[4 * e + 2] = ubyte<2>(d[e]) - 128.f;
             f[4 * e + 3] = ubyte<3>(d[e]) - 128.f;
         }
+        float4 xv[B][4];                                       // every column's loads ahead of its products
 #pragma unroll
-        for (int b = 0; b < B; b++) {
-            const float4* xp = (const float4*)(a.x + (size_t)b * a.N + j);
+        for (int b = 0; b < B; b++)
 #pragma unroll
-            for (int e = 0; e < 4; e++) {
-                const float4 v = xp[e];
+            for (int e = 0; e < 4; e++) xv[b][e] = ((const float4*)(a.x + (size_t)b * a.N + j))[e];
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+#pragma unroll
+            for (int b = 0; b < B; b++) {
+                const float4 v = xv[b][e];
                 acc[b] = fmaf(f[4 * e], v.x, acc[b]);
                 acc[b] = fmaf(f[4 * e + 1], v.y, acc[b]);
                 acc[b] = fmaf(f[4 * e + 2], v.z, acc[b]);
@@ -755,13 +761,16 @@ int ibh_launch_int8_skinny(float* out, const void* w, const void* sc, int kind, 
         return 1;
     }
     const int G = (N + 127) / 128, T = (M + 15) / 16;
-        const DigArgs a{(const int8_t*)w, sc, x, out, M, N, B, M_stride, G, (G + kDigWaves - 1) / kDigWaves};
+    const DigArgs a{(const int8_t*)w, sc, x, out, M, N, B, M_stride, G, (G + kDigWaves - 1) / kDigWaves};
     // One column has no digits to share: 14336 x 4096 19.0 us here, 23.5 there.
     // Two cross at 2048 rows or 1024 columns (2048 x 8192 9.9 and 11.6, 4096 x
-    // 4096 10.5 and 9.3, 14336 x 512 7.9 and 8.4), three and four where few
-    // short rows leave the digits' kernel its latency (1000 x 2048 5.0 and 5.4
-    // at four, 1024 x 4096 7.6 and 7.4).
-    if (B == 1 || (B == 2 && (M <= 2048 || N <= 1024)) || (B <= 4 && M <= 1024 && N <= 2048)) {
+    // 4096 10.5 and 9.3, 14336 x 512 7.9 and 8.4), three and four where the
+    // wavefront-a-row blocks pass one per CU (in a graph, 1000 rows of 4096 5.0
+    // and 6.6 at three, 6.2 and 6.9 at four, of 14336 11.7 and 16.3, 15.5 and
+    // 16.3; 1500 rows of 4096 8.2 and 6.7, 9.6 and 6.6); a few long rows at four
+    // leave most CUs idle here (256 x 8192 11.9 and 10.7, 256 x 4096 6.0 and 6.4).
+    if (B == 1 || (B == 2 && (M <= 2048 || N <= 1024)) || (B == 3 && M <= 1024) ||
+        (B == 4 && M <= 1024 && (M > 256 || N <= 4096))) {
 #define IBH_I8V(K_) do { const int g_ = (M + 3) / 4; \
         if (B == 1) int8_rows<K_, 1><<<g_, 256, 0, st>>>(a); else if (B == 2) int8_rows<K_, 2><<<g_, 256, 0, st>>>(a); \
         else if (B == 3) int8_rows<K_, 3><<<g_, 256, 0, st>>>(a); else int8_rows<K_, 4><<<g_, 256, 0, st>>>(a); } while (0)

@@ -245,6 +245,26 @@ def test_int8_batch_small_beside_large(M, N, B):
         assert (np.abs(got[b] - want) <= bound).all()
 
 
+# two to four columns on either side of the rows and lengths where the vector
+# form hands over to the digits
+@pytest.mark.parametrize("M,N,B", [(1024, 4096, 3), (1025, 4096, 3), (1024, 2064, 4), (256, 4112, 4), (257, 4112, 4),
+                                   (256, 4096, 4), (2049, 1024, 2), (2049, 1040, 2), (3, 14336, 3)])
+def test_int8_batch_few_columns(M, N, B):
+    """Both forms against float64: a lane's chain of N / 64 products, rounded
+    up, and six folds, each to 2^-24 of its partial sum (the digits' bound is
+    smaller), the row scale once more."""
+    print(f"case int8 few columns M={M} N={N} B={B}", flush=True)
+    r = np.random.default_rng(M + N + B)
+    w = r.integers(-128, 128, (M, N), dtype=np.int8)
+    s = (r.random(M) * 0.01 + 1e-4).astype(np.float32)
+    x = r.standard_normal((B, N)).astype(np.float32)
+    got = _int8_batch(w, s, x)
+    for b in range(B):
+        want = (w.astype(np.float64) @ x[b].astype(np.float64)) * s
+        bound = 2.0 ** -24 * (N / 64 + 16 + 7) * (np.abs(w.astype(np.float64)) @ np.abs(x[b]).astype(np.float64)) * s
+        assert (np.abs(got[b] - want) <= bound).all()
+
+
 def test_int8_batch_tiny_x():
     """Groups of subnormal and just normal numbers, exactly held."""
     r = np.random.default_rng(5)
