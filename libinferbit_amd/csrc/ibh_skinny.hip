@@ -674,6 +674,36 @@ __global__ __launch_bounds__(256) void int8_rows(const DigArgs a) {
     }
 }
 
+// The most columns that stay with the 4- to 16-column kernels of ibh_mfma.hip,
+// which stage nothing that they do not need, for rows of G groups in `blocks`
+// blocks of rt row tiles.  Both sides measured in a graph at 256 to 32000 rows
+// of 128 to 14336 columns (the sums are the same bits); there and here:
+//  - at 4 columns every shape (14336 x 4096 10.0 and 11.5 us, 2048 x 2048 3.9
+//    and 4.4), at 6 most are here (12.3 and 11.5, 4.5 and 4.4);
+//  - rows of up to 7 groups give a block one or two wavefronts here: 1024 x 512
+//    at 8 / 16 columns 3.4 / 3.8 and 4.2 / 4.5, 1024 x 768 3.5 / 3.9 and 3.9 /
+//    4.0 (one group or eight: even at 5); 2 and 3 groups cross where the
+//    other kernels need a second pass, 8192 x 256 at 8 / 9 3.4 / 6.0 and 3.8;
+//  - 17 to 32 groups with one block per CU: the codes staged and the hand-on
+//    show, 4096 x 4096 at 8 / 12 5.5 / 6.5 and 6.0 / 5.9, 8192 x 4096 at 8 / 10
+//    / 12 7.6 / 8.4 / 8.9 and 8.8;
+//  - blocks that fill their last round of the CUs badly: 9216 x 8192 (288
+//    blocks) at 8 / 12 19.5 / 22.6 and 22.5, 20000 x 2048 at 8 8.4 and 9.6.
+// Rows that end inside a group take a pass per 4 columns there.
+int w4a8_stay(int N, int rt, int blocks) {
+    const int G = N / 128, rounds = (blocks + 255) / 256;
+    if (N % 128) return 4;
+    if (G == 2 || G == 3) return 8;
+    if (rounds > 1 && rt > 1 && 8 * blocks < 7 * 256 * rounds) {
+        if (rt == 2) return rounds > 2 ? (G > 48 ? 8 : 4) : G <= 48 ? 8 : G < 64 ? 12 : 10;
+        return G < 9 ? 4 : G < 12 ? 12 : 9;
+    }
+    if (rt == 1) return G > 3 && G < 8 ? 16 : (G > 8 && G < 12) || (G > 16 && G <= 32) ? 8 : 4;
+    if (rt == 2) return G < 17 ? 4 : G < 24 ? 9 : G <= 32 ? 10 : G < 64 ? 4 : 5;
+    if (rt == 3) return G > 16 && G <= 32 ? 8 : 4;
+    return G > 8 && G <= 16 ? 8 : 4;
+}
+
 constexpr size_t kLds = 160 * 1024;
 
 bool lds_ok(const void* fn, size_t bytes) {
@@ -699,11 +729,6 @@ int ibh_launch_w4a8_batch(const MatDesc* d, int n, int kind, const int8_t* qx, c
     // Row tiles per block: as many as make one block per CU, up to 4; from two
     // on the running sum is handed on (2 wavefronts per row where 16 groups
     // each reach), one takes the gather with up to 8 wavefronts of 4 groups.
-    // Fewer columns than these stay with the 4- to 16-column kernels, which
-    // stage nothing they do not need.  Both sides measured: at 4 and 6 columns
-    // 14336 x 4096 10.0 / 12.3 there and 11.5 / 11.5 here, 2048 x 2048 3.9 / 4.5
-    // and 4.4 / 4.4, 2048 x 5632 6.5 / 8.3 and 7.6 / 7.7; rows of 17 to 32 groups
-    // cross later, 4096 x 4096 at 8 / 12 columns 5.5 / 6.5 and 6.0 / 5.9.
     int rt = (T + 255) / 256;
     rt = rt > 4 ? 4 : rt;
     int KW = (G + 15) / 16 > 2 ? (G + 15) / 16 : 2;
@@ -711,7 +736,8 @@ int ibh_launch_w4a8_batch(const MatDesc* d, int n, int kind, const int8_t* qx, c
     if (rt < 1) return 0;
     const bool gather = rt == 1;
     if (gather) KW = (G + 3) / 4 < 8 ? (G + 3) / 4 : 8;
-    if (B <= (gather && G > 16 && G <= 32 ? 8 : 4)) return 0;
+    // (matrices of a joint launch are alone there, a launch each)
+    if (B <= (n > 1 ? (gather && G > 16 && G <= 32 ? 8 : 4) : w4a8_stay(N, rt, (T + rt - 1) / rt))) return 0;
     const int CPW = (G + KW - 1) / KW;
     KW = (G + CPW - 1) / CPW;
     auto soff_of = [&](bool x) {

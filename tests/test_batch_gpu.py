@@ -166,6 +166,16 @@ def test_w4a8_batch_columns_bit_exact(oracle_lib, M, N, B):
         assert (got[b * ms + M:(b + 1) * ms] == 7.0).all()
 
 
+# the last column count of one kernel and the first of the other, for the rules
+# by groups, by row tiles per block and by a badly filled last round of blocks
+@pytest.mark.parametrize("M,N,B", [(70, 256, 8), (70, 256, 9), (1003, 512, 16), (1003, 512, 17), (1003, 896, 16),
+                                   (1003, 896, 17), (100, 1152, 8), (100, 1152, 9), (4100, 4096, 10), (4100, 4096, 11),
+                                   (4100, 8192, 5), (4100, 8192, 6), (9000, 2560, 8), (9000, 2560, 9), (9216, 8192, 10),
+                                   (9216, 8192, 11), (20000, 2048, 9), (20000, 2048, 10), (70, 288, 5), (70, 288, 4)])
+def test_w4a8_batch_handover_bit_exact(oracle_lib, M, N, B):
+    test_w4a8_batch_columns_bit_exact(oracle_lib, M, N, B)
+
+
 # M, N, B, M_stride: part-filled row tiles and column tiles, one and two row
 # tiles per wavefront, rows that end inside a 128-column group or are shorter
 # than the wavefronts' split, both column-tile forms
@@ -431,7 +441,7 @@ def test_fused_int8_chains_bit_exact(table, Ms, N, B):
 
 # the fused fold handed on (tall), gathered, with codes from L2, and rows that
 # end inside a group; 2 matrices in a launch
-@pytest.mark.parametrize("Ms,N,B", [((8200,), 4096, 5), ((8200,), 4096, 17), ((5632, 5632), 2048, 32), ((2048,), 5632, 31),
+@pytest.mark.parametrize("Ms,N,B", [((8200,), 4096, 9), ((8200,), 4096, 17), ((5632, 5632), 2048, 32), ((2048,), 5632, 31),
                                     ((1000, 500), 6176, 20), ((500,), 2080, 9), ((40,), 64, 17), ((1003,), 2048, 16)])
 def test_fused_w4a8_columns_bit_exact(Ms, N, B):
     """The prompt's W4A8 products against the one-vector product, bit for bit."""
