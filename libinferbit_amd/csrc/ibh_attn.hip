@@ -619,7 +619,10 @@ __device__ unsigned long long ibh_as_tt[512][8];
 #define AS_TT(i) ((void)0)
 #endif
 
-template <int BITS, int GRP, int HD, bool ROPE = false>
+// SLOTS: blockIdx.z is a slot of a batched pass (consecutive positions, partials
+// of their own).  A form of its own here and in the merge: one position through
+// it took up to 0.3 us longer.
+template <int BITS, int GRP, int HD, bool ROPE = false, bool SLOTS = false>
 __global__ __launch_bounds__(kSplitThreads) void attn_split(float* __restrict__ out, float* __restrict__ part,
                                                            const float* __restrict__ q,
                                                            const uint8_t* __restrict__ kd,
@@ -638,10 +641,9 @@ __global__ __launch_bounds__(kSplitThreads) void attn_split(float* __restrict__ 
     constexpr int MB = 64;                                // chunks one merge pass loads per thread
     static_assert(TR >= 1 && CT % TR == 0, "P.V split");
     AS_TT(0);
-    // blockIdx.z: slot of a batched pass (consecutive positions, partials of
-    // their own); never with ROPE
+    static_assert(!(ROPE && SLOTS));
     if (dpos) T += *dpos;
-    if constexpr (!ROPE) {
+    if constexpr (SLOTS) {
         T += (int)blockIdx.z;
         q += (size_t)blockIdx.z * n_kv * GRP * HD;
         part += (size_t)blockIdx.z * n_kv * GRP * nstride * (HD + 2);
@@ -877,7 +879,7 @@ __global__ __launch_bounds__(kSplitThreads) void attn_split(float* __restrict__ 
 // d) holds chunks c = cq (mod 1024/DS), every load of the block issued at
 // once.  Slicing the dims spreads a head's partials over HD/DS blocks (the
 // weights e^(m_c - M) are recomputed by each).
-template <int HD, int DS = 32>
+template <int HD, bool SLOTS, int DS = 32>
 __global__ __launch_bounds__(1024) void attn_merge_wide(float* __restrict__ out, const float* __restrict__ part,
                                                         int T, const int* __restrict__ dpos, int ct, int nstride,
                                                         int rope) {
@@ -887,7 +889,8 @@ __global__ __launch_bounds__(1024) void attn_merge_wide(float* __restrict__ out,
     __shared__ float osum[NCQ][DS];
     __shared__ float tot;
     const int h = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const float* ph = part + ((size_t)blockIdx.z * gridDim.x + h) * nstride * (HD + 2);   // blockIdx.z: slot
+    const int row = SLOTS ? (int)(blockIdx.z * gridDim.x) + h : h;   // blockIdx.z: slot
+    const float* ph = part + (size_t)row * nstride * (HD + 2);
     const int cq = tid / DS, d = blockIdx.y * DS + tid % DS;
     // every slot of the head is loaded before the position is known (slots
     // past the last chunk hold stale values that are never used), so the
@@ -903,7 +906,7 @@ __global__ __launch_bounds__(1024) void attn_merge_wide(float* __restrict__ out,
         wlv = ph[(size_t)tid * (HD + 2) + 1];
     }
     if (dpos) T += *dpos;
-    T += (int)blockIdx.z;
+    if constexpr (SLOTS) T += (int)blockIdx.z;
     const int nch = rope ? (T - 1 + ct - 1) / ct + 1 : (T + ct - 1) / ct;   // rope: one more partial, position T-1
     if (tid < nch) {
         wm[tid] = wmv;
@@ -934,7 +937,7 @@ __global__ __launch_bounds__(1024) void attn_merge_wide(float* __restrict__ out,
         float r = 0.f;
 #pragma unroll
         for (int k = 0; k < NCQ; k++) r += osum[k][tid];
-        out[((size_t)blockIdx.z * gridDim.x + h) * HD + blockIdx.y * DS + tid] = r / tot;
+        out[(size_t)row * HD + blockIdx.y * DS + tid] = r / tot;
     }
 }
 
@@ -968,10 +971,13 @@ int launch_split(float* out, float* part, const float* q, const void* kdata, con
 #define IBH_AS(B_, G_, H_) do { \
         if (rope) attn_split<B_, G_, H_, true><<<dim3(n_kv, nchunk + 1), kSplitThreads, 0, st>>>( \
                       out, part, q, K, V, kscales, vscales, T, dpos, n_kv, scale, nstride, rp); \
-        else attn_split<B_, G_, H_, false><<<dim3(n_kv, nchunk, slots), kSplitThreads, 0, st>>>( \
+        else if (slots > 1) attn_split<B_, G_, H_, false, true><<<dim3(n_kv, nchunk, slots), kSplitThreads, 0, st>>>( \
+                 out, part, q, K, V, kscales, vscales, T, dpos, n_kv, scale, nstride, rp); \
+        else attn_split<B_, G_, H_, false><<<dim3(n_kv, nchunk), kSplitThreads, 0, st>>>( \
                  out, part, q, K, V, kscales, vscales, T, dpos, n_kv, scale, nstride, rp); \
         IBH_CHECK_LAUNCH("ibh_attn_decode (split)"); \
-        attn_merge_wide<H_><<<dim3(n_heads, H_ / 32, slots), 1024, 0, st>>>(out, part, T, dpos, ct, nstride, rope ? 1 : 0); } while (0)
+        if (slots > 1) attn_merge_wide<H_, true><<<dim3(n_heads, H_ / 32, slots), 1024, 0, st>>>(out, part, T, dpos, ct, nstride, 0); \
+        else attn_merge_wide<H_, false><<<dim3(n_heads, H_ / 32), 1024, 0, st>>>(out, part, T, dpos, ct, nstride, rope ? 1 : 0); } while (0)
 #define IBH_ASG(B_, H_) do { if (grp == 1) IBH_AS(B_, 1, H_); else if (grp == 2) IBH_AS(B_, 2, H_); \
                          else if (grp == 4) IBH_AS(B_, 4, H_); else IBH_AS(B_, 8, H_); } while (0)
 #define IBH_ASH(B_) do { if (head_dim == 64) IBH_ASG(B_, 64); else IBH_ASG(B_, 128); } while (0)

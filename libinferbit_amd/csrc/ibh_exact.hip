@@ -639,10 +639,12 @@ __global__ __launch_bounds__(64) void attn_scores_exact(float* __restrict__ att,
     __shared__ float qs[256];
     __shared__ float knew[ROPE ? 256 : 1];
     const int h = blockIdx.x;
-    // blockIdx.z: slot of a batched pass (the slots sit at consecutive positions)
-    const int T = *dpos + 1 + (int)blockIdx.z;
-    q += (size_t)blockIdx.z * n_heads * hd;
-    att += (size_t)blockIdx.z * n_heads * tstride;
+    // blockIdx.z: slot of a batched pass (consecutive positions; never with ROPE)
+    const int T = *dpos + 1 + (ROPE ? 0 : (int)blockIdx.z);
+    if constexpr (!ROPE) {
+        q += (size_t)blockIdx.z * n_heads * hd;
+        att += (size_t)blockIdx.z * n_heads * tstride;
+    }
     const int t = blockIdx.y * 64 + threadIdx.x;
     if ((int)blockIdx.y * 64 >= T) return;
     const int grp = n_heads / n_kv;
@@ -779,10 +781,12 @@ __global__ __launch_bounds__(64 * GRP) void attn_scores_grp(float* __restrict__ 
     __shared__ __align__(16) float knew[ROPE ? HD : 4];
     const int kh = blockIdx.x;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;   // wave g scores query head kh * GRP + g
-    // blockIdx.z: slot of a batched pass (the slots sit at consecutive positions)
-    const int T = *dpos + 1 + (int)blockIdx.z;
-    q += (size_t)blockIdx.z * n_kv * GRP * HD;
-    att += (size_t)blockIdx.z * n_kv * GRP * tstride;
+    // blockIdx.z: slot of a batched pass (consecutive positions; never with ROPE)
+    const int T = *dpos + 1 + (ROPE ? 0 : (int)blockIdx.z);
+    if constexpr (!ROPE) {
+        q += (size_t)blockIdx.z * n_kv * GRP * HD;
+        att += (size_t)blockIdx.z * n_kv * GRP * tstride;
+    }
     // position tiles in reverse launch order: the tile of the current
     // position (the block with the cache write) is dispatched first instead of
     // last, onto a CU not yet shared with two other tiles
